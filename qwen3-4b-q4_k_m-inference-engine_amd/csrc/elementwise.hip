@@ -7,19 +7,74 @@
 namespace qk {
 namespace {
 
+// 16-byte accesses (rows and tensors are only float-aligned: gfx950 takes
+// dword-aligned 16-byte global accesses); the last count % 4 elements go one
+// a lane.
 __global__ __launch_bounds__(256) void silu_multiply_kernel(const float* __restrict__ gate,
                                                             const float* __restrict__ up,
                                                             float* __restrict__ out,
                                                             int64_t count) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < count; i += stride) {
-    const float g = gate[i];
-    out[i] = (g / (1.0f + expf(-g))) * up[i];
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t quads = count / 4;
+  auto one = [](float g, float u) { return (g / (1.0f + expf(-g))) * u; };
+  for (int64_t i = first; i < quads; i += stride) {
+    const f32x4 g = *reinterpret_cast<const f32x4_a4*>(gate + 4 * i);
+    const f32x4 u = *reinterpret_cast<const f32x4_a4*>(up + 4 * i);
+    *reinterpret_cast<f32x4_a4*>(out + 4 * i) = f32x4{one(g.x, u.x), one(g.y, u.y), one(g.z, u.z), one(g.w, u.w)};
+  }
+  if (first < count - 4 * quads) {
+    const int64_t i = 4 * quads + first;
+    out[i] = one(gate[i], up[i]);
   }
 }
 
+// The sum of the workgroup's four waves' `sum`, in every thread.
+__device__ __forceinline__ float workgroup_sum(float sum, float (&partial)[4]) {
+  sum = row_lanes_sum<64>(sum);
+  if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  return (partial[0] + partial[1]) + (partial[2] + partial[3]);
+}
+
 // out = x * rsqrt(mean(x^2) + eps) * scale for one row per workgroup (the
-// mat-vec's RMSNorm fold does the same inside its prologue at M = 1).
+// mat-vec's RMSNorm fold does the same inside its prologue at M = 1). A few
+// rows are bound by latency alone, so a row of at most 1024 Q values stays in
+// registers: its Q 16-byte loads per thread and those of the scale are all
+// issued at entry, and the row is read once: 8 rows of 2560 in 4.8 us against
+// 7.3 with one value per lane and load, the row read twice (rocprof, in a
+// graph; a launch's own cost there is about 2).
+template <int Q>
+__global__ __launch_bounds__(256) void rms_norm_row_kernel(const float* __restrict__ x,
+                                                           const float* __restrict__ scale,
+                                                           float* __restrict__ out, int width,
+                                                           float eps) {
+  __shared__ float partial[4];
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * width;
+  const int tid = static_cast<int>(threadIdx.x);
+  const int quads = width / 4;
+  f32x4 v[Q], s[Q];
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {  // loads past the row re-read its last quad
+    const int at = 4 * min(tid + 256 * i, quads - 1);
+    v[i] = *reinterpret_cast<const f32x4_a4*>(x + row + at);
+    s[i] = *reinterpret_cast<const f32x4_a4*>(scale + at);
+  }
+  float sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    const float t = (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+    sum += tid + 256 * i < quads ? t : 0.0f;
+  }
+  const float inv = rsqrtf(workgroup_sum(sum, partial) / static_cast<float>(width) + eps);
+#pragma unroll
+  for (int i = 0; i < Q; ++i)
+    if (tid + 256 * i < quads)
+      *reinterpret_cast<f32x4_a4*>(out + row + 4 * (tid + 256 * i)) =
+          f32x4{(v[i].x * inv) * s[i].x, (v[i].y * inv) * s[i].y, (v[i].z * inv) * s[i].z, (v[i].w * inv) * s[i].w};
+}
+
+// Any other width: two passes over the row.
 __global__ __launch_bounds__(256) void rms_norm_kernel(const float* __restrict__ x,
                                                        const float* __restrict__ scale,
                                                        float* __restrict__ out, int width,
@@ -30,11 +85,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float* __restrict__
   const int tid = static_cast<int>(threadIdx.x);
   float sum = 0.0f;
   for (int i = tid; i < width; i += 256) sum += xr[i] * xr[i];
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-  if ((tid & 63) == 0) partial[tid >> 6] = sum;
-  __syncthreads();
-  const float total = (partial[0] + partial[1]) + (partial[2] + partial[3]);
-  const float inv = rsqrtf(total / static_cast<float>(width) + eps);
+  const float inv = rsqrtf(workgroup_sum(sum, partial) / static_cast<float>(width) + eps);
   for (int i = tid; i < width; i += 256) o[i] = (xr[i] * inv) * scale[i];
 }
 
@@ -42,32 +93,52 @@ __global__ __launch_bounds__(256) void residual_add_kernel(float* __restrict__ s
                                                            const float* __restrict__ branch,
                                                            int64_t count) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < count; i += stride)
-    state[i] += branch[i];
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t quads = count / 4;
+  for (int64_t i = first; i < quads; i += stride) {
+    f32x4_a4* s = reinterpret_cast<f32x4_a4*>(state + 4 * i);
+    *s = *s + *reinterpret_cast<const f32x4_a4*>(branch + 4 * i);
+  }
+  if (first < count - 4 * quads) state[4 * quads + first] += branch[4 * quads + first];
+}
+
+// Workgroups of an elementwise launch over `count` values, four a thread.
+uint32_t elementwise_grid(int64_t count) {
+  const int64_t blocks = (count + 1023) / 1024;
+  return static_cast<uint32_t>(blocks < 16384 ? blocks : 16384);
 }
 
 }  // namespace
 
 hipError_t launch_residual_add(float* state, const float* branch, int64_t count,
                                hipStream_t stream) {
-  const int64_t blocks = (count + 255) / 256;
-  const uint32_t grid = static_cast<uint32_t>(blocks < 16384 ? blocks : 16384);
-  residual_add_kernel<<<grid, 256, 0, stream>>>(state, branch, count);
+  residual_add_kernel<<<elementwise_grid(count), 256, 0, stream>>>(state, branch, count);
   return hipGetLastError();
 }
 
 hipError_t launch_rms_norm(const float* x, const float* scale, float* out, int64_t rows,
                            int64_t width, float eps, hipStream_t stream) {
-  rms_norm_kernel<<<static_cast<uint32_t>(rows), 256, 0, stream>>>(x, scale, out,
-                                                                   static_cast<int>(width), eps);
+  const dim3 grid(static_cast<uint32_t>(rows));
+  const int w = static_cast<int>(width);
+  // Whole quads up to 8192 values take the one-pass form (Q rounds of 1024).
+  if (w % 4 != 0 || w > 8192)
+    rms_norm_kernel<<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
+  else if (w <= 1024)
+    rms_norm_row_kernel<1><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
+  else if (w <= 2048)
+    rms_norm_row_kernel<2><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
+  else if (w <= 3072)
+    rms_norm_row_kernel<3><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
+  else if (w <= 4096)
+    rms_norm_row_kernel<4><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
+  else
+    rms_norm_row_kernel<8><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
   return hipGetLastError();
 }
 
 hipError_t launch_silu_multiply(const float* gate, const float* up, float* out, int64_t count,
                                 hipStream_t stream) {
-  const int64_t blocks = (count + 255) / 256;
-  const uint32_t grid = static_cast<uint32_t>(blocks < 16384 ? blocks : 16384);
-  silu_multiply_kernel<<<grid, 256, 0, stream>>>(gate, up, out, count);
+  silu_multiply_kernel<<<elementwise_grid(count), 256, 0, stream>>>(gate, up, out, count);
   return hipGetLastError();
 }
 

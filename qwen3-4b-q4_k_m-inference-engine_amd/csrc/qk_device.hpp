@@ -88,6 +88,43 @@ __device__ __forceinline__ void scale_min_k4(uint32_t g, uint32_t s0, uint32_t s
   m = static_cast<int>(ubfe(m_src, m_pos, low_width) | (ubfe(s1, pos + 6u, high_width) << 4));
 }
 
+// v + the same register of the lane selected by a DPP control (row-local).
+template <int CTRL>
+__device__ __forceinline__ float add_dpp(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
+                                                                   0xF, 0xF, false));
+}
+
+// v summed over lane bit 4 / lane bit 5 with the gfx950 lane-swap
+// instructions (VALU, no LDS round trip). The two results of a swap are
+// copied out as scalars before the bit casts: bit casting the subscripted
+// elements directly made the compiler use the first result twice.
+__device__ __forceinline__ float swap16_sum(float v) {
+  const auto t = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v),
+                                                  __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned a = t[0], b = t[1];
+  return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+__device__ __forceinline__ float swap32_sum(float v) {
+  const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v),
+                                                  __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned a = t[0], b = t[1];
+  return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+
+// Sum over the LPR lanes of each row (aligned lane groups); every lane of the
+// group receives the sum.
+template <int LPR>
+__device__ __forceinline__ float row_lanes_sum(float v) {
+  v = add_dpp<0xB1>(v);                             // lane bit 0 (quad_perm 1,0,3,2)
+  v = add_dpp<0x4E>(v);                             // lane bit 1 (quad_perm 2,3,0,1)
+  if constexpr (LPR >= 8) v = add_dpp<0x141>(v);    // lane bit 2 (row_half_mirror)
+  if constexpr (LPR >= 16) v = add_dpp<0x140>(v);   // lane bit 3 (row_mirror)
+  if constexpr (LPR >= 32) v = swap16_sum(v);       // lane bit 4
+  if constexpr (LPR >= 64) v = swap32_sum(v);       // lane bit 5
+  return v;
+}
+
 // Sum over the 8 lanes of each aligned lane octet (quad swaps, then the
 // half-row mirror); every lane of the octet receives the sum.
 __device__ __forceinline__ float octet_sum(float v) {
