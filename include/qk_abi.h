@@ -81,9 +81,9 @@ int qk_version(void);
  * M <= 8 (decode): one streaming mat-vec launch per 8 rows, Q8 quantisation
  * inside the kernel, integer dot products as the reference; nothing is
  * allocated. M > 8 (prefill): the activations' Q8 round trip, scaled per row
- * by a power of two, is stored as two fp16 planes hi + lo in a stream-ordered
- * scratch buffer (qk_matmul_workspace_size bytes, allocated and freed on
- * `stream` like the reference's per-call workspace) with the planes' 32-value
+ * by a power of two, is stored as two fp16 planes hi + lo in scratch of the
+ * call (qk_matmul_workspace_size bytes, from the library's cache of blocks,
+ * see qk_release_scratch) with the planes' 32-value
  * block sums; an MFMA GEMM multiplies them by the weights in fp32 accumulation:
  * Q4_K as the exact fp16 integers sc*q (hi*B + lo*B per step, d and dmin*m
  * applied once per superblock), Q6_K as sc*q = fp16(sc*q) + an exact
@@ -284,6 +284,14 @@ int qk_residual_add(float *state, const float *branch, int64_t count, qk_stream_
  * (include/Kernels.hpp:28-32) for engine kernels built outside this library. */
 int qk_check_launch(void);
 
+/* Entry points that need device scratch and are given none (M > 8) take it
+ * from up to 8 blocks per device of 16 or 64 MiB that stay allocated between
+ * calls (larger requests, requests while no block is idle, and calls under
+ * stream capture allocate and free stream-ordered). Waits for the current
+ * device and gives its idle blocks back; later calls allocate them anew. Not
+ * for use while a stream is being captured. */
+int qk_release_scratch(void);
+
 /* out = gate/(1+exp(-gate)) * up, elementwise. Replaces kernels::silu_multiply
  * (include/Kernels.hpp:72, src/cuda/silu_multiply.cu:19-23). */
 int qk_silu_multiply(const float *gate, const float *up, float *out, int64_t count,
@@ -324,8 +332,8 @@ int qk_event_elapsed_ms(float *ms, qk_event_t start, qk_event_t end);
  * call (the reference lists CUDA Graphs as future work, README.md:42). No
  * compute entry point records a memset. At M <= 8 none allocates, except
  * qk_ffn_gate_up_norm outside its M = 1 fold; at M > 8 qk_matmul,
- * qk_matmul_segments, qk_ffn_gate_up, qk_ffn_gate_up_norm and qk_ffn allocate
- * their scratch stream-ordered (captured as allocation nodes), while the _ws
+ * qk_matmul_segments, qk_ffn_gate_up, qk_ffn_gate_up_norm and qk_ffn take
+ * their scratch stream-ordered under capture (allocation nodes), while the _ws
  * entry points take a caller workspace and qk_matmul_noalloc uses the
  * library's scratch array: those allocate nothing.
  * ------------------------------------------------------------------------- */

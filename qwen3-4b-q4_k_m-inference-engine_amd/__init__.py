@@ -89,6 +89,7 @@ _SIGNATURES = {
     "qk_rms_norm": [_c_void_p, _c_void_p, _c_void_p, _i64, _i64, _float, _c_void_p],
     "qk_residual_add": [_c_void_p, _c_void_p, _i64, _c_void_p],
     "qk_check_launch": [],
+    "qk_release_scratch": [],
     "qk_malloc": [ctypes.POINTER(_c_void_p), _size],
     "qk_free": [_c_void_p],
     "qk_malloc_async": [ctypes.POINTER(_c_void_p), _size, _c_void_p],
@@ -489,6 +490,11 @@ def rms_norm(x, scale, out, rows: int, width: int, eps: float, stream=None) -> N
 def residual_add(state, branch, count: int, stream=None) -> None:
     """qk_residual_add: state += branch."""
     check(load().qk_residual_add(_ptr(state), _ptr(branch), count, _stream_ptr(stream)))
+
+
+def release_scratch() -> None:
+    """qk_release_scratch: the library's idle scratch blocks given back."""
+    check(load().qk_release_scratch())
 
 
 def synth_superblocks(w, qtype: int, N: int, K: int, seed: int, dmax: float,

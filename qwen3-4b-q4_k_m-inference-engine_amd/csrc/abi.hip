@@ -14,6 +14,7 @@
 
 #include "qk_abi.h"
 #include "qk_launch.hpp"
+#include "scratch.hpp"
 
 namespace {
 
@@ -132,7 +133,7 @@ int run_single(const float* x, const qk_q8_block* q8, const void* w, int type, i
 
 // Prefill path (M > 8 rows): activation prep once, then one MFMA GEMM per
 // weight matrix. Without a caller workspace the fp16 activation scratch is
-// allocated stream-ordered for the call, as the reference allocates its Q8
+// taken for the call (scratch.hpp), where the reference allocates its Q8
 // workspace per call (src/cuda/matmul.cu:143-145).
 int run_gemm(const float* x, int64_t M, int64_t K, const qk_segment* segments, int count,
              void* workspace, size_t workspace_bytes, hipStream_t stream) {
@@ -147,12 +148,13 @@ int run_gemm(const float* x, int64_t M, int64_t K, const qk_segment* segments, i
   for (int j = 0; j < count; ++j)
     need = std::max(need, qk::gemm_workspace_bytes(M, K, segments[j].type, segments[j].N));
   void* scratch = workspace;
+  qk::Scratch own(stream);
   if (scratch) {
     if (workspace_bytes < need) return fail(QK_ERR_INVALID_ARGUMENT, "matmul workspace too small");
     if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0)
       return fail(QK_ERR_INVALID_ARGUMENT, "matmul workspace must be 16-byte aligned");
   } else {
-    const hipError_t error = hipMallocAsync(&scratch, need, stream);
+    const hipError_t error = own.get(need, scratch);
     if (error != hipSuccess) return hip_fail(error, "matmul workspace allocation failed");
   }
   // short prompt against narrow matrices: the GEMM forms its planes from x
@@ -179,7 +181,6 @@ int run_gemm(const float* x, int64_t M, int64_t K, const qk_segment* segments, i
     error = qk::launch_gemm_core(x_short, scratch, segments[j].w, segments[j].type, K, segments[j].N,
                                  segments[j].y, M, stream);
   }
-  if (!workspace) (void)hipFreeAsync(scratch, stream);
   return error == hipSuccess ? QK_OK : hip_fail(error, "matmul launch failed");
 }
 
@@ -281,7 +282,7 @@ namespace {
 // Prefill FFN (M > 8): gate and up through the GEMM (one launch for both
 // where no split K is needed) into scratch, then SiLU(gate) * up into h. The
 // scratch (gate and up outputs, then the GEMM workspace) is the caller's
-// workspace when given, else allocated stream-ordered for the call.
+// workspace when given, else taken for the call (scratch.hpp).
 size_t ffn_gemm_bytes(int type, int64_t K, int64_t N, int64_t M) {
   const size_t gu = (2 * static_cast<size_t>(M) * static_cast<size_t>(N) * sizeof(float) + 255) & ~size_t{255};
   return gu + qk::gemm_workspace_bytes(M, K, type, N);
@@ -291,12 +292,13 @@ int run_ffn_gemm(const float* x, const void* gate, const void* up, int type, int
                  float* h, int64_t M, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   const size_t need = ffn_gemm_bytes(type, K, N, M);
   void* scratch = workspace;
+  qk::Scratch own(stream);
   if (scratch) {
     if (workspace_bytes < need) return fail(QK_ERR_INVALID_ARGUMENT, "ffn workspace too small");
     if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0)
       return fail(QK_ERR_INVALID_ARGUMENT, "ffn workspace must be 16-byte aligned");
   } else {
-    const hipError_t error = hipMallocAsync(&scratch, need, stream);
+    const hipError_t error = own.get(need, scratch);
     if (error != hipSuccess) return hip_fail(error, "ffn scratch allocation failed");
   }
   float* gu = static_cast<float*>(scratch);
@@ -308,7 +310,6 @@ int run_ffn_gemm(const float* x, const void* gate, const void* up, int type, int
     const hipError_t error = qk::launch_silu_multiply(gu, gu + M * N, h, M * N, stream);
     if (error != hipSuccess) status = hip_fail(error, "silu_multiply launch failed");
   }
-  if (!workspace) (void)hipFreeAsync(scratch, stream);
   return status;
 }
 
@@ -440,16 +441,16 @@ int qk_ffn_gate_up_norm(const float* x, const float* norm, float eps, const void
     if (error != hipSuccess) return hip_fail(error, "matmul launch failed");
     if (launched) return QK_OK;
   }
-  // Otherwise the norm runs on its own into stream-ordered scratch, then the
+  // Otherwise the norm runs on its own into the call's scratch, then the
   // fused gate/up product.
-  float* normalized = nullptr;
-  hipError_t error = hipMallocAsync(reinterpret_cast<void**>(&normalized),
-                                    static_cast<size_t>(M * K) * sizeof(float), s);
+  void* scratch = nullptr;
+  qk::Scratch own(s);
+  hipError_t error = own.get(static_cast<size_t>(M * K) * sizeof(float), scratch);
+  float* normalized = static_cast<float*>(scratch);
   if (error != hipSuccess) return hip_fail(error, "RMSNorm scratch allocation failed");
   error = qk::launch_rms_norm(x, norm, normalized, M, K, eps, s);
   int result = error == hipSuccess ? QK_OK : hip_fail(error, "RMSNorm launch failed");
   if (result == QK_OK) result = qk_ffn_gate_up(normalized, gate, up, type, K, N, h, M, stream);
-  (void)hipFreeAsync(normalized, s);
   return result;
 }
 
@@ -644,6 +645,11 @@ int qk_residual_add(float* state, const float* branch, int64_t count, qk_stream_
   if (!state || !branch) return fail(QK_ERR_INVALID_ARGUMENT, "pointers must be non-null");
   const hipError_t error = qk::launch_residual_add(state, branch, count, as_stream(stream));
   return error == hipSuccess ? QK_OK : hip_fail(error, "residual_add launch failed");
+}
+
+int qk_release_scratch(void) {
+  const hipError_t error = qk::release_scratch();
+  return error == hipSuccess ? QK_OK : hip_fail(error, "scratch release failed");
 }
 
 int qk_check_launch(void) {

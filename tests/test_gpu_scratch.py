@@ -1,0 +1,105 @@
+"""The scratch of calls that bring none: qk_matmul at M > 8 from more streams
+than there are blocks, from threads that share a stream, on recreated streams,
+across block sizes, under capture and after a release, each result equal bit
+for bit to qk_matmul_ws on a workspace of its own."""
+from __future__ import annotations
+
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+Q4, Q6 = 12, 14
+
+
+class Case:
+    def __init__(self, qk, oracle, qtype, K, N, M, seed):
+        self.qk, self.args = qk, (qtype, K, N, M)
+        self.w = qk.DeviceBuffer.from_array(oracle.synth_superblocks(qtype, N, K, seed, 0.01, 0.01))
+        self.x = qk.DeviceBuffer.from_array(oracle.synth_normal(M * K, seed + 1))
+        self.y = qk.DeviceBuffer(4 * M * N)
+        need = qk.matmul_workspace_size(qtype, K, N, M)
+        ws = qk.DeviceBuffer(need)
+        self.run(None, ws, need)
+        qk.synchronize()
+        self.want = self.y.download(np.uint32)
+        self.y.fill(0)
+
+    def run(self, stream, ws=None, need=0):
+        qtype, K, N, M = self.args
+        if ws is None:
+            self.qk.matmul(self.x, self.w, qtype, K, N, self.y, M, stream)
+        else:
+            self.qk.matmul_ws(self.x, self.w, qtype, K, N, self.y, M, ws, need, stream)
+
+    def check(self):
+        assert np.array_equal(self.y.download(np.uint32), self.want)
+        self.y.fill(0)
+
+
+# scratch below, at and past the 16 and 64 MiB classes: 0.6, 15.2, 17, 40 and 80 MiB
+SHAPES = [(Q4, 2560, 256, 33), (Q6, 9728, 64, 400), (Q4, 4096, 96, 1040), (Q4, 9728, 64, 1040), (Q6, 9728, 32, 2060)]
+
+
+def test_streams_and_sizes(gpu, oracle):
+    cases = [Case(gpu, oracle, *SHAPES[i % len(SHAPES)], 20261201 + i) for i in range(11)]
+    streams = [gpu.Stream() for _ in cases]
+    for _ in range(3):
+        for c, s in zip(cases, streams):
+            c.run(s.ptr)
+        gpu.synchronize()
+        for c in cases:
+            c.check()
+        for s in streams:
+            s.destroy()
+        streams = [gpu.Stream() for _ in cases]
+    gpu.release_scratch()
+    for c in cases:  # one stream, every size in turn
+        c.run(streams[0].ptr)
+    gpu.synchronize()
+    for c in cases:
+        c.check()
+    for s in streams:
+        s.destroy()
+
+
+def test_threads_sharing_a_stream(gpu, oracle):
+    cases = [Case(gpu, oracle, *SHAPES[i % 3], 20261301 + i) for i in range(6)]
+    stream = gpu.Stream()
+    errors = []
+
+    def work(c):
+        try:
+            for _ in range(20):
+                c.run(stream.ptr)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(c,)) for c in cases]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    gpu.synchronize()
+    assert not errors
+    for c in cases:
+        c.check()
+    stream.destroy()
+
+
+def test_capture_between_cached_calls(gpu, oracle):
+    a, b = (Case(gpu, oracle, Q4, 2560, 256, 33 + i, 20261401 + i) for i in range(2))
+    stream = gpu.Stream()
+    a.run(stream.ptr)
+    graph = gpu.Graph.capture(stream, lambda: a.run(stream.ptr))
+    for _ in range(3):
+        b.run(stream.ptr)
+        graph.launch(stream.ptr)
+        b.run(stream.ptr)
+        gpu.synchronize()
+        a.check()
+        b.check()
+    graph.destroy()
+    stream.destroy()
