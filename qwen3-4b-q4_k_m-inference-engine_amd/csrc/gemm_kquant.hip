@@ -889,7 +889,7 @@ struct KQPlan {
 // ffn_down 41.3 -> 36.2.
 constexpr int64_t kPlanCUs = 256;
 
-KQPlan plan(int type, int64_t M, int64_t N, int64_t K) {
+KQPlan rule_plan(int type, int64_t M, int64_t N, int64_t K) {
   const int64_t tiles64 = ((M + 63) / 64) * ((N + 127) / 128);
   const int64_t tiles32 = ((M + 31) / 32) * ((N + 127) / 128);
   // (M <= 32: one row of tiles either way, and a 64-row tile would compute
@@ -908,6 +908,59 @@ KQPlan plan(int type, int64_t M, int64_t N, int64_t K) {
   // 65535 rows; the check states it)
   const bool fits_reduce = M <= 65535;
   return {wide, fits_reduce ? static_cast<int>(std::min(by_grid, by_depth)) : 1};
+}
+
+// Estimated time (ns) of a plan: the busiest CU's work units one after
+// another (a CU with several resident takes as long as with one at a time:
+// 2.2-2.5 us per superblock of a 64-row Q4_K tile whether 1, 2 or 3 are
+// resident, a lone unit up to a third more), then the reduce of the splits (a
+// launch, and the partial products once through memory).
+double plan_cost(int type, bool wide, int64_t tiles, int64_t splits, int64_t M, int64_t N, int64_t S) {
+  const bool q6 = type == QK_TYPE_Q6_K;
+  const double superblock_ns = q6 ? (wide ? 3400.0 : 2400.0) : wide ? 2350.0 : 1500.0;
+  const int64_t units = (tiles * splits + kPlanCUs - 1) / kPlanCUs;  // of the busiest CU
+  const double gemm = superblock_ns * static_cast<double>(units) * static_cast<double>((S + splits - 1) / splits);
+  const double reduce = 3500.0 + 1e-3 * static_cast<double>(splits) * static_cast<double>(M) * static_cast<double>(N);
+  return gemm * (units == 1 ? 1.3 : 1.0) + (splits > 1 ? reduce : 0.0);
+}
+
+// The rules above hold for K < 4096 at M > 64 and for M <= 32. For deep K, and
+// for the few tiles of M = 33..64, they leave up to half of the time on CUs
+// that wait for the busiest one; there the plan is the tile height and split
+// of least estimated time. Measured against the rules (us, prep and reduce
+// included; 22 shapes timed under every plan, the chosen one 1.13 times as fast
+// as the rules' on average and never more than 1% behind it): 2560 x 9728 Q6_K at M = 48 / 100 / 200 /
+// 350 / 800 37.4 / 63.3 / 78.8 / 112.6 / 256 -> 33.6 / 41.4 / 62.7 / 88.6 /
+// 219, Q4_K at M = 100 / 512 38.9 / 97.9 -> 31.7 / 78.7, 1024 x 2560 Q6_K at
+// M = 48 21.0 -> 14.6. (At smaller K and larger M finer splits gain less, and
+// a row's sums are the same there at every M.)
+constexpr int64_t kPlanSplits = 6;
+
+KQPlan plan(int type, int64_t M, int64_t N, int64_t K) {
+  const KQPlan rule = rule_plan(type, M, N, K);
+  const int64_t S = K / 256;
+  if (M <= 32 || M > 65535 || (M > 64 && S < 16)) return rule;
+  const int64_t n_tiles = (N + 127) / 128;
+  const int64_t tiles32 = ((M + 31) / 32) * n_tiles, tiles64 = ((M + 63) / 64) * n_tiles;
+  // Splits of at least 4 superblocks (2 at M <= 64) that keep the workspace
+  // within the scratch of qk_matmul_noalloc where the rule's plan is within it.
+  const int64_t most = std::clamp<int64_t>(S / (M <= 64 ? 2 : 4), 1, kPlanSplits);
+  const int64_t planes = M * K * 4 + M * S * 32 + M * 4 + 512;
+  const bool within = planes + (rule.splits > 1 ? rule.splits * M * N * 4 : 0) <= static_cast<int64_t>(QK_NOALLOC_SCRATCH_BYTES);
+  KQPlan best{false, 1};
+  double least = plan_cost(type, false, tiles32, 1, M, N, S);
+  for (const bool wide : {false, true})
+    for (int64_t splits = 1; splits <= most; ++splits) {
+      if (splits > rule.splits && within &&
+          planes + splits * M * N * 4 > static_cast<int64_t>(QK_NOALLOC_SCRATCH_BYTES))
+        break;
+      const double cost = plan_cost(type, wide, wide ? tiles64 : tiles32, splits, M, N, S);
+      if (cost < least) {
+        least = cost;
+        best = {wide, static_cast<int>(splits)};
+      }
+    }
+  return best;
 }
 
 }  // namespace

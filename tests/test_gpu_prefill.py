@@ -471,3 +471,30 @@ def test_ffn_gate_up_matches_separate_kernels(gpu, oracle, M, K, N):
         with np.errstate(over="ignore"):
             ref = g / (1.0 + np.exp(-g)) * u
         check(oracle, got.reshape(M, N), ref, f"ffn gate/up M={M}")
+
+
+@pytest.mark.parametrize("qtype,K,N,M", [
+    (Q4, 2560, 1024, 33), (Q6, 2560, 130, 64),      # M = 33..64: as few as two superblocks a split
+    (Q4, 512, 300, 48), (Q6, 256, 65, 40),          # two superblocks and one: no split to make
+    (Q6, 9728, 2560, 100), (Q4, 9728, 640, 513),    # deep K: 64-row tiles, six splits of uneven length
+    (Q4, 4096, 2560, 65), (Q6, 4352, 1030, 129),    # K = 4096 and just past it
+])
+def test_prefill_planned_splits_against_oracle(gpu, oracle, qtype, K, N, M):
+    """Shapes whose tile height and split come from the estimated time (deep K,
+    and M = 33..64), against the float64 product; the workspace they ask for
+    is enough and ends where it says (the bytes past it stay)."""
+    w = make_weight(gpu, qtype, N, K, SEED + 90 + M)
+    x = oracle.synth_normal(M * K, SEED + 91 + K)
+    xd = gpu.DeviceBuffer.from_array(x)
+    need = gpu.matmul_workspace_size(qtype, K, N, M)
+    ws = gpu.DeviceBuffer.from_array(np.full(need + 256, 0xFF, np.uint8))
+    y = gpu.DeviceBuffer(4 * M * N)
+    gpu.matmul_ws(xd, w, qtype, K, N, y, M, ws, need)
+    gpu.synchronize()
+    print(f"[case] planned type={qtype} M={M} N={N} K={K} launch {gpu.last_launch()}", flush=True)
+    assert np.all(ws.download(np.uint8)[need:] == 0xFF)
+    rows = sorted({0, 31, 32, M // 2, M - 1})
+    got = y.download(np.float32).reshape(M, N)[rows]
+    xr = np.concatenate([x.reshape(M, K)[r] for r in rows])
+    ref = float64_reference(oracle, xr, w.download(np.uint8), qtype, K, N, len(rows))
+    check(oracle, got, ref, f"planned {qtype} {M}x{N}x{K}")
