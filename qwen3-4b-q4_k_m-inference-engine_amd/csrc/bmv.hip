@@ -92,14 +92,7 @@ __device__ __forceinline__ void bmv_body(const BmvParams& p, const BmvShare& sh,
   cursor_seek(start, sh, u_lo < u_hi ? u_lo : 0);
   start.left = ntiles;
 
-  BmvLane L;
-  L.n = lane & 15;
-  L.kq = lane >> 4;
-  L.zero = static_cast<uint32_t>(8 * stride);
-  L.a4_valid = (L.n < 8) == (L.kq < 2);
-  L.a4_base = static_cast<uint32_t>((L.n & 7) * stride + 16 * (L.kq & 1));
-  L.a6_valid = (L.n >> 2) == L.kq;
-  L.a6_base = static_cast<uint32_t>((L.n & 3) * stride + 16 * L.kq);
+  const BmvLane L = bmv_lane(lane, stride);
 
   // the first P tiles
   BmvTile<TYPE> buf[P];

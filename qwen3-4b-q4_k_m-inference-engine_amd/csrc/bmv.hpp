@@ -16,8 +16,9 @@
 //         64 qs bytes); A rows 0..7 = activation rows 0..7 against j1, rows
 //         8..15 = the same rows against j2, zero elsewhere.
 //   Q6_K: k = 4 sub-blocks of 16 (one nibble of 64 ql bytes with their qh
-//         bit pairs); A rows 4b..4b+3 = 4 activation rows against sub-block
-//         b; a second MFMA on the same B takes activation rows 4..7.
+//         bit pairs); M <= 4: A rows 4b..4b+3 = the activation rows against
+//         sub-block b; M > 4: two MFMAs on the same B, in product p A rows
+//         4b..4b+3 = activation rows 4*(b&1)..+3 against sub-block 2*(b>>1)+p.
 // Lane l holds A[l%16][16(l/16)..+16], B[16(l/16)..+16][l%16] and receives
 // C[4(l/16)+i][l%16], i < 4 (probed on gfx950), so lane (n, kq) = (l%16, l/16)
 // loads the 16 weight bytes of row n for k-quarter kq straight from memory,
@@ -153,10 +154,26 @@ struct BmvLane {
   int n, kq;
   uint32_t a4_base;   // Q4_K A: this lane's activation row and k-quarter, or the zero line
   bool a4_valid;
-  uint32_t a6_base;   // Q6_K A (activation rows 0..3; rows 4..7 add 4*stride)
+  uint32_t a6_base;   // Q6_K A at M <= 4
   bool a6_valid;
+  uint32_t a6p_base;  // Q6_K A at M > 4: product p reads it in the lanes of odd (p) / even k-quarters
+  bool a6p_valid[2];
   uint32_t zero;
 };
+
+__device__ __forceinline__ BmvLane bmv_lane(int lane, int stride) {
+  BmvLane L;
+  L.n = lane & 15;
+  L.kq = lane >> 4;
+  L.zero = static_cast<uint32_t>(8 * stride);
+  L.a4_valid = (L.n < 8) == (L.kq < 2);
+  L.a4_base = static_cast<uint32_t>((L.n & 7) * stride + 16 * (L.kq & 1));
+  L.a6_valid = (L.n >> 2) == L.kq;
+  L.a6_base = static_cast<uint32_t>((L.n & 3) * stride + 16 * L.kq);
+  L.a6p_base = static_cast<uint32_t>((L.n & 7) * stride + 16 * L.kq);
+  for (int p = 0; p < 2; ++p) L.a6p_valid[p] = (L.n >> 3) == (L.kq >> 1) && (L.kq & 1) == p;
+  return L;
+}
 
 // Q4_K tile at superblock column s: acc[i] += row n's dot for activation row
 // 4*(kq&1)+i over the sub-blocks of set kq>>1 (the other set sits in lane l^32).
@@ -211,54 +228,124 @@ __device__ __forceinline__ void bmv_tile(const Q4Tile& t, int s, const BmvLane& 
   for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(-dmin, minv[i], __builtin_fmaf(d, mainv[i], acc[i]));
 }
 
-// Q6_K tile at superblock column s: acc[mh][i] += row n's dot for activation
-// row 4*mh+i over the sub-blocks 8h+4nib+kq (the other kq in lanes l^16, l^32).
-template <int MH>
-__device__ __forceinline__ void bmv_tile(const Q6Tile& t, int s, const BmvLane& L, int stride,
-                                         const lds_u8* codes, const lds_f32* xs, const lds_f32* xf,
-                                         f32x4 (&acc)[2]) {
+// 16 codes of a Q6_K tile's half h and nibble nib (ql nibble | qh pair << 4,
+// 0..63): src/cuda/matmul.cu:71-79. sh0 / sh1 move the qh bit pair of group
+// 2 nib + (k-quarter >> 1) to bits 4-5 of each byte.
+__device__ __forceinline__ u32x4 bmv_codes6(const Q6Tile& t, int h, int nib, uint32_t sh) {
+  const u32x4 ql = h ? t.lb : t.la;
+  const u32x4 qh = h ? t.hb : t.ha;
+  u32x4 b;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t lo = nib ? (ql[e] >> 4) & 0x0F0F0F0Fu : ql[e] & 0x0F0F0F0Fu;
+    b[e] = bit_insert(0x30303030u, __builtin_amdgcn_alignbit(qh[e], qh[e], sh), lo);
+  }
+  return b;
+}
+
+// Q6_K tile at superblock column s, M <= 4: acc[i] += row n's dot for
+// activation row i over the sub-blocks 8h+4nib+kq (the other kq in lanes l^16,
+// l^32). The -32 offset of the codes enters as the MFMA's accumulator input
+// -32 * sum(activation codes), so the integer dot is exact.
+__device__ __forceinline__ void bmv_tile6(const Q6Tile& t, int s, const BmvLane& L, const lds_u8* codes,
+                                          const lds_f32* xs, const lds_f32* xf, f32x4& acc) {
   const int khi = L.kq >> 1;
-  // qh bit pair of group g = 2nib + khi moved to bits 4-5 of each byte
   const uint32_t sh0 = 28u + 2u * static_cast<uint32_t>(khi), sh1 = 2u * static_cast<uint32_t>(khi);
-  f32x4 accsb[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+  f32x4 accsb = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
 #pragma unroll
     for (int nib = 0; nib < 2; ++nib) {
-      // 16 codes (ql nibble | qh pair << 4, 0..63; the -32 offset enters
-      // as the MFMA's accumulator input -32 * sum(activation codes), so the
-      // integer dot is exact): src/cuda/matmul.cu:71-79
-      const u32x4 ql = h ? t.lb : t.la;
-      const u32x4 qh = h ? t.hb : t.ha;
-      const uint32_t sh = nib ? sh1 : sh0;
-      u32x4 b;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t lo = nib ? (ql[e] >> 4) & 0x0F0F0F0Fu : ql[e] & 0x0F0F0F0Fu;
-        const uint32_t hs = __builtin_amdgcn_alignbit(qh[e], qh[e], sh);
-        b[e] = bit_insert(0x30303030u, hs, lo);
-      }
+      const u32x4 b = bmv_codes6(t, h, nib, nib ? sh1 : sh0);
       const int sb16 = 8 * h + 4 * nib + L.kq;  // this lane's sub-block
       const float scf = static_cast<float>(static_cast<int8_t>((t.sc[2 * h + nib] >> (8 * L.kq)) & 0xFFu));
       const int blk = 4 * h + 2 * nib + khi;  // its Q8 block
+      const uint32_t aoff = L.a6_valid ? L.a6_base + 256 * s + 128 * h + 64 * nib : L.zero;
+      const i32x4 n4 = lds_read_i32x4(reinterpret_cast<const lds_u8*>(xf), 4u * ((16 * s + sb16) * 8));
+      const i32x4 ci = mfma_i8(lds_read_i32x4(codes, aoff), b, n4);
+      const f32x4 x4 = lds_read_f32x4(xs + (8 * s + blk) * 8);
 #pragma unroll
-      for (int mh = 0; mh < MH; ++mh) {
-        const uint32_t aoff = L.a6_valid ? L.a6_base + 4 * mh * stride + 256 * s + 128 * h + 64 * nib : L.zero;
-        const i32x4 n4 = lds_read_i32x4(reinterpret_cast<const lds_u8*>(xf), 4u * ((16 * s + sb16) * 8 + 4 * mh));
-        const i32x4 ci = mfma_i8(lds_read_i32x4(codes, aoff), b, n4);
-        const f32x4 x4 = lds_read_f32x4(xs + (8 * s + blk) * 8 + 4 * mh);
+      for (int i = 0; i < 4; ++i) accsb[i] = __builtin_fmaf(scf, x4[i] * static_cast<float>(ci[i]), accsb[i]);
+    }
+  }
+  const float d = half_bits_to_float(t.d);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          accsb[mh][i] = __builtin_fmaf(scf, x4[i] * static_cast<float>(ci[i]), accsb[mh][i]);
+  for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(d, accsb[i], acc[i]);
+}
+
+// Q6_K tile, M = 5..8: acc[i] += row n's dot for activation row 4*(kq&1)+i
+// over the Q8 blocks 4h+2nib+(kq>>1) (the others in lane l^32). A rows 4g..
+// 4g+3 hold activation rows 4*(g&1).. against k-quarter 2*(g>>1)+p in product
+// p, so a lane's two products are the two sub-blocks of ONE Q8 block and the
+// same four activation rows: sc0*dot0 + sc1*dot1 is formed in integers (|dot|
+// <= 16*127*32 < 2^17 and |sc| <= 128: exact in 32 bits) and takes one
+// conversion and one block scale, where a product of its own per half of the
+// activation rows took two of each (lm_head at M = 5 / 8: 79.2 / 80.2 -> 75.4 / 76.4 us).
+__device__ __forceinline__ void bmv_tile6_pair(const Q6Tile& t, int s, const BmvLane& L, const lds_u8* codes,
+                                               const lds_f32* xs, const lds_f32* xf, f32x4& acc) {
+  const int khi = L.kq >> 1, klo = L.kq & 1;
+  const uint32_t sh0 = 28u + 2u * static_cast<uint32_t>(khi), sh1 = 2u * static_cast<uint32_t>(khi);
+  f32x4 accsb = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int nib = 0; nib < 2; ++nib) {
+      const u32x4 b = bmv_codes6(t, h, nib, nib ? sh1 : sh0);
+      const int blk = 4 * h + 2 * nib + khi;  // this lane's Q8 block
+      i32x4 dot[2];
+      int sc[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const uint32_t aoff = L.a6p_valid[p] ? L.a6p_base + 256 * s + 128 * h + 64 * nib : L.zero;
+        const i32x4 n4 =
+            lds_read_i32x4(reinterpret_cast<const lds_u8*>(xf), 4u * ((16 * s + 2 * blk + p) * 8 + 4 * klo));
+        dot[p] = mfma_i8(lds_read_i32x4(codes, aoff), b, n4);
+        sc[p] = __builtin_amdgcn_sbfe(static_cast<int>(t.sc[2 * h + nib]), 16 * khi + 8 * p, 8);
+      }
+      const f32x4 x4 = lds_read_f32x4(xs + (8 * s + blk) * 8 + 4 * klo);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int sum = __mul24(dot[0][i], sc[0]) + __mul24(dot[1][i], sc[1]);
+        accsb[i] = __builtin_fmaf(x4[i], static_cast<float>(sum), accsb[i]);
       }
     }
   }
   const float d = half_bits_to_float(t.d);
 #pragma unroll
-  for (int mh = 0; mh < MH; ++mh)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[mh][i] = __builtin_fmaf(d, accsb[mh][i], acc[mh][i]);
+  for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(d, accsb[i], acc[i]);
 }
+
+// The tile of either type: MH = 1 for M <= 4, 2 for M = 5..8 (Q4_K: the same).
+template <int MH>
+__device__ __forceinline__ void bmv_tile_any(const Q4Tile& t, int s, const BmvLane& L, int stride, const lds_u8* codes,
+                                             const lds_f32* xs, const lds_f32* xss, const lds_f32*, f32x4& acc) {
+  bmv_tile(t, s, L, stride, codes, xs, xss, acc);
+}
+template <int MH>
+__device__ __forceinline__ void bmv_tile_any(const Q6Tile& t, int s, const BmvLane& L, int, const lds_u8* codes,
+                                             const lds_f32* xs, const lds_f32*, const lds_f32* xf, f32x4& acc) {
+  if constexpr (MH == 1)
+    bmv_tile6(t, s, L, codes, xs, xf, acc);
+  else
+    bmv_tile6_pair(t, s, L, codes, xs, xf, acc);
+}
+
+// A unit's sums over its lanes: every lane of the result holds activation rows
+// 4*(kq&1).. (Q4_K, and Q6_K at M > 4: the other sub-block set is in lane
+// l^32) or rows 0..3 (Q6_K at M <= 4: one sub-block of four in each kq).
+template <int TYPE, int MH>
+__device__ __forceinline__ f32x4 bmv_lane_sums(const f32x4& acc) {
+  f32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[i] = swap32_sum(acc[i]);
+    if constexpr (TYPE == QK_TYPE_Q6_K && MH == 1) v[i] = swap16_sum(v[i]);
+  }
+  return v;
+}
+// Lanes whose kq is below this hold distinct sums.
+template <int TYPE, int MH>
+constexpr int kBmvSumLanes = TYPE == QK_TYPE_Q6_K && MH == 1 ? 1 : 2;
 
 // Position of a wave in its stream of tiles: unit (part, group g, run rr),
 // superblock s of the run [s, s_end), tiles left including this one.
@@ -310,28 +397,13 @@ __device__ __forceinline__ const uint8_t* bmv_sb(const BmvShare& sh, const BmvCu
 }
 
 // Unit sums into LDS: sums[((part*groups_max + g)*16 + n)*ranges + rr][m].
+template <int TYPE, int MH>
 __device__ __forceinline__ void bmv_flush(const f32x4& acc, const BmvCursor& c, const BmvLane& L,
                                           int groups_max, int ranges, lds_f32* sums) {
-  f32x4 v;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) v[i] = swap32_sum(acc[i]);  // both sub-block sets
-  if (L.kq < 2)
+  const f32x4 v = bmv_lane_sums<TYPE, MH>(acc);
+  if (L.kq < kBmvSumLanes<TYPE, MH>)
     *reinterpret_cast<lds_f32x4*>(sums + (((c.part * groups_max + c.g) * 16 + L.n) * ranges + c.rr) * 8 +
                                   4 * L.kq) = v;
-}
-template <int MH>
-__device__ __forceinline__ void bmv_flush(const f32x4 (&acc)[2], const BmvCursor& c, const BmvLane& L,
-                                          int groups_max, int ranges, lds_f32* sums) {
-  f32x4 v[2];
-#pragma unroll
-  for (int mh = 0; mh < MH; ++mh)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[mh][i] = swap16_sum(swap32_sum(acc[mh][i]));  // all four kq
-  if (L.kq == 0) {
-    lds_f32* p = sums + (((c.part * groups_max + c.g) * 16 + L.n) * ranges + c.rr) * 8;
-#pragma unroll
-    for (int mh = 0; mh < MH; ++mh) *reinterpret_cast<lds_f32x4*>(p + 4 * mh) = v[mh];
-  }
 }
 
 // One type's share: the tile stream of this wave, then (after the caller's
@@ -342,32 +414,16 @@ __device__ __forceinline__ void bmv_stream(const BmvShare& sh, BmvCursor lc, con
                                            const lds_f32* xss, const lds_f32* xf, lds_f32* sums,
                                            BmvTile<TYPE> (&buf)[P], BmvCursor cc) {
   constexpr int B = TYPE == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KBytes;
-  using Acc = typename std::conditional<TYPE == QK_TYPE_Q4_K, f32x4, f32x4[2]>::type;
-  Acc acc;
-  auto clear = [&]() {
-    if constexpr (TYPE == QK_TYPE_Q4_K) {
-      acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    } else {
-      acc[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      acc[1] = acc[0];
-    }
-  };
-  clear();
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
   const int ntiles = cc.left;
   for (int base = 0; base < ntiles; base += P) {
 #pragma unroll
     for (int j = 0; j < P; ++j) {
       if (base + j < ntiles) {
-        if constexpr (TYPE == QK_TYPE_Q4_K)
-          bmv_tile(buf[j], cc.s, L, stride, codes, xs, xss, acc);
-        else
-          bmv_tile<MH>(buf[j], cc.s, L, stride, codes, xs, xf, acc);
+        bmv_tile_any<MH>(buf[j], cc.s, L, stride, codes, xs, xss, xf, acc);
         if (cc.s + 1 == cc.s_end) {  // last tile of the unit
-          if constexpr (TYPE == QK_TYPE_Q4_K)
-            bmv_flush(acc, cc, L, groups_max, sh.ranges, sums);
-          else
-            bmv_flush<MH>(acc, cc, L, groups_max, sh.ranges, sums);
-          clear();
+          bmv_flush<TYPE, MH>(acc, cc, L, groups_max, sh.ranges, sums);
+          acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
         cursor_next(cc, sh);
       }

@@ -43,27 +43,26 @@ struct BmvPassParams {
   int32_t ppg, pad;  // passes per group (ceil(S / C))
 };
 
-// Rows of one pass: group g (rows 16g .. 16g + 15, clamped to N - 1: rows
-// past the matrix re-read its last row and are never stored), columns
-// [c0, c0 + C) (clamped to S: a short last pass re-reads the last column,
-// never computed).
-template <int TYPE, int J>
-__device__ __forceinline__ void bp_issue(u32x4 (&buf)[J], const BmvPassParams& p, __amdgpu_buffer_rsrc_t rsrc,
-                                         int g, int c0, const int (&run)[J], const int (&q)[J]) {
-  constexpr int B = TYPE == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KBytes;
-  // Cache policy: default. A run of C superblocks starts and ends inside
-  // 128-byte lines that the row's neighbouring passes (the same wave's next
-  // ones) also read; with the nontemporal hint those lines left the L2 in
-  // between and were fetched again: FETCH_SIZE 1.26x the matrix at M = 8,
-  // 1.03x without the hint (lm_head 97-105 -> 94-98 us).
-  constexpr int kNt = 0;
-  const int64_t row_bytes = static_cast<int64_t>(p.S) * B;
+// The chunks of one pass: base[j] = this lane's run j's row x row bytes, q16[j]
+// = its chunk's 16-byte offset in the run, at = the first byte of the pass's
+// first run. Rows past the matrix and a short last pass's missing columns read
+// what follows, or zeros past the matrix's end (the descriptor's range), and
+// are never stored or never computed. Everything that depends on the lane is
+// formed once per launch: three VALU a chunk (lm_head at M = 3 / 8: 65.8 / 76.4
+// -> 64.1 / 74.5 us against 64-bit row arithmetic in every pass).
+// Cache policy: default. A run of C superblocks starts and ends inside
+// 128-byte lines that the row's neighbouring passes (the same wave's next
+// ones) also read; with the nontemporal hint those lines left the L2 in
+// between and were fetched again: FETCH_SIZE 1.26x the matrix at M = 8,
+// 1.03x without the hint (lm_head 97-105 -> 94-98 us).
+template <int J>
+__device__ __forceinline__ void bp_issue(u32x4 (&buf)[J], __amdgpu_buffer_rsrc_t rsrc, uint32_t at,
+                                         const uint32_t (&base)[J], const uint32_t (&q16)[J]) {
+  constexpr int kDefault = 0;
 #pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int64_t row = min(16 * g + run[j], p.N - 1);
-    const int64_t first = row * row_bytes + static_cast<int64_t>(min(c0, p.S - 1)) * B;
-    buf[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>((first & ~int64_t{3}) + 16 * q[j]), 0, kNt);
-  }
+  for (int j = 0; j < J; ++j)
+    buf[j] = __builtin_amdgcn_raw_buffer_load_b128(
+        rsrc, static_cast<int>(((base[j] + at) & ~3u) + q16[j]), 0, kDefault);
 }
 
 template <int TYPE, int J>
@@ -97,13 +96,15 @@ __global__ __launch_bounds__(64 * kBpWaves) void bmv_pass_kernel(const BmvPassPa
   const int npass = ngroups * ppg;
   // each lane's chunks of a pass: chunk c = lane + 64 j (clamped to the last)
   // of run c / cpr, chunk c % cpr of the run
+  const uint32_t row_bytes = static_cast<uint32_t>(S) * B;
   const int nchunks = 16 * cpr;
-  int run[J], q[J];
+  uint32_t base[J], q16[J];
 #pragma unroll
   for (int j = 0; j < J; ++j) {
-    const int c = min(lane + 64 * j, nchunks - 1);
-    run[j] = c / cpr;
-    q[j] = c - run[j] * cpr;
+    const uint32_t c = static_cast<uint32_t>(min(lane + 64 * j, nchunks - 1));
+    const uint32_t run = c / static_cast<uint32_t>(cpr);
+    base[j] = run * row_bytes;
+    q16[j] = 16u * (c - run * static_cast<uint32_t>(cpr));
   }
   // loads through a descriptor whose range ends at the dword boundary at or
   // above the matrix end: dwords past it read as zero
@@ -115,11 +116,14 @@ __global__ __launch_bounds__(64 * kBpWaves) void bmv_pass_kernel(const BmvPassPa
     g = wid + W * gi;
     c0 = (i - gi * ppg) * C;
   };
+  auto pass_byte = [&](int g, int c0) {  // (below 2^31: the launcher's bound on the matrix)
+    return static_cast<uint32_t>(16 * g) * row_bytes + static_cast<uint32_t>(c0) * B;
+  };
   u32x4 buf[J];
   {
     int g, c0;
     pass_at(0, g, c0);
-    bp_issue<TYPE, J>(buf, p, rsrc, min(g, groups - 1), c0, run, q);
+    bp_issue<J>(buf, rsrc, pass_byte(min(g, groups - 1), c0), base, q16);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -141,30 +145,12 @@ __global__ __launch_bounds__(64 * kBpWaves) void bmv_pass_kernel(const BmvPassPa
   if (tid == 0) *reinterpret_cast<lds_u32x4*>(codes + 8 * stride) = u32x4{0u, 0u, 0u, 0u};
   __syncthreads();
 
-  BmvLane L;
-  L.n = lane & 15;
-  L.kq = lane >> 4;
-  L.zero = static_cast<uint32_t>(8 * stride);
-  L.a4_valid = (L.n < 8) == (L.kq < 2);
-  L.a4_base = static_cast<uint32_t>((L.n & 7) * stride + 16 * (L.kq & 1));
-  L.a6_valid = (L.n >> 2) == L.kq;
-  L.a6_base = static_cast<uint32_t>((L.n & 3) * stride + 16 * L.kq);
-  const int64_t row_bytes = static_cast<int64_t>(S) * B;
+  const BmvLane L = bmv_lane(lane, stride);
   const lds_u8* my_run = slot + 16 * cpr * L.n;  // lane's row's run
 
   auto body = [&](auto mh) {
     constexpr int MH = decltype(mh)::value;
-    using Acc = typename std::conditional<TYPE == QK_TYPE_Q4_K, f32x4, f32x4[2]>::type;
-    Acc acc;
-    auto clear = [&]() {
-      if constexpr (TYPE == QK_TYPE_Q4_K) {
-        acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      } else {
-        acc[0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        acc[1] = acc[0];
-      }
-    };
-    clear();
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int i = 0; i < npass; ++i) {
       int g, c0;
       pass_at(i, g, c0);
@@ -172,62 +158,36 @@ __global__ __launch_bounds__(64 * kBpWaves) void bmv_pass_kernel(const BmvPassPa
       // came first in this wave's program order)
 #pragma unroll
       for (int j = 0; j < J; ++j)
-        *reinterpret_cast<lds_u32x4*>(slot + 16 * (run[j] * cpr + q[j])) = buf[j];
+        *reinterpret_cast<lds_u32x4*>(slot + 16 * min(lane + 64 * j, nchunks - 1)) = buf[j];
       asm volatile("" ::: "memory");
       {  // the next pass (the last one again past the end), unconditionally
         int g2, c2;
         pass_at(min(i + 1, npass - 1), g2, c2);
-        bp_issue<TYPE, J>(buf, p, rsrc, g2, c2, run, q);
+        bp_issue<J>(buf, rsrc, pass_byte(g2, c2), base, q16);
       }
-      // this lane's row of the group and where its run starts in the slot
-      const int row = min(16 * g + L.n, N - 1);
-      const uint32_t o = static_cast<uint32_t>((row * row_bytes + static_cast<int64_t>(c0) * B) & 3);
+      // where this lane's row's run starts in the slot
+      const uint32_t o = (static_cast<uint32_t>(L.n) * row_bytes + pass_byte(g, c0)) & 3u;
 #pragma unroll 1
       for (int cc = 0; cc < C; ++cc) {
         const int s = c0 + cc;
         if (s < S) {
-          if constexpr (TYPE == QK_TYPE_Q4_K) {
-            Q4Tile t;
-            ws_tile(t, my_run + o + cc * B, L.kq);
-            bmv_tile(t, s, L, stride, codes, xs, xss, acc);
-          } else {
-            Q6Tile t;
-            ws_tile(t, my_run + o + cc * B, L.kq);
-            bmv_tile<MH>(t, s, L, stride, codes, xs, xf, acc);
-          }
+          BmvTile<TYPE> t;
+          ws_tile(t, my_run + o + cc * B, L.kq);
+          bmv_tile_any<MH>(t, s, L, stride, codes, xs, xss, xf, acc);
         }
       }
       asm volatile("" ::: "memory");  // the next pass's slot writes follow these reads
       if (c0 + C >= S) {  // the group's last pass: row totals of the lanes, store
         const int r = 16 * g + L.n;
-        if constexpr (TYPE == QK_TYPE_Q4_K) {
-          f32x4 v;
+        const f32x4 v = bmv_lane_sums<TYPE, MH>(acc);
+        if (L.kq < kBmvSumLanes<TYPE, MH> && r < N) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = swap32_sum(acc[e]);  // both sub-block sets
-          if (L.kq < 2 && r < N) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int m = 4 * L.kq + e;
-              if (m < M) p.y[static_cast<int64_t>(m) * N + r] = v[e];
-            }
-          }
-        } else {
-          f32x4 v[2];
-#pragma unroll
-          for (int h = 0; h < MH; ++h)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[h][e] = swap16_sum(swap32_sum(acc[h][e]));  // all four kq
-          if (L.kq == 0 && r < N) {
-#pragma unroll
-            for (int h = 0; h < MH; ++h)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const int m = 4 * h + e;
-                if (m < M) p.y[static_cast<int64_t>(m) * N + r] = v[h][e];
-              }
+          for (int e = 0; e < 4; ++e) {
+            const int m = 4 * L.kq + e;
+            if (m < M) p.y[static_cast<int64_t>(m) * N + r] = v[e];
           }
         }
-        clear();
+        acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       }
     }
   };

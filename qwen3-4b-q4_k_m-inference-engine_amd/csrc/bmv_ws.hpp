@@ -218,14 +218,7 @@ __device__ __forceinline__ void bmv_ws_body(const BmvWsParams& p, const uint8_t*
   }
   __syncthreads();
 
-  BmvLane L;
-  L.n = lane & 15;
-  L.kq = lane >> 4;
-  L.zero = static_cast<uint32_t>(8 * stride);
-  L.a4_valid = (L.n < 8) == (L.kq < 2);
-  L.a4_base = static_cast<uint32_t>((L.n & 7) * stride + 16 * (L.kq & 1));
-  L.a6_valid = (L.n >> 2) == L.kq;
-  L.a6_base = static_cast<uint32_t>((L.n & 3) * stride + 16 * L.kq);
+  const BmvLane L = bmv_lane(lane, stride);
   // the lane's row (rows past the share redo its last one; their sums are
   // never added) and where its wave put it
   const int ic = min(L.n, nrows - 1);
@@ -236,28 +229,20 @@ __device__ __forceinline__ void bmv_ws_body(const BmvWsParams& p, const uint8_t*
   const lds_u8* rowp = regions + (part * kWp + ic / kRpw) * reg_bytes + o + (ic % kRpw) * row_bytes;
   const int s_lo = S * wv / kWp, s_hi = S * (wv + 1) / kWp;
   const BmvCursor c{part, 0, wv, 0, 0, 0};
-  if constexpr (TYPE == QK_TYPE_Q4_K) {
+  auto run = [&](auto mh) {
+    constexpr int MH = decltype(mh)::value;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int s = s_lo; s < s_hi; ++s) {
-      Q4Tile t;
+      BmvTile<TYPE> t;
       ws_tile(t, rowp + s * B, L.kq);
-      bmv_tile(t, s, L, stride, codes, xs, xss, acc);
+      bmv_tile_any<MH>(t, s, L, stride, codes, xs, xss, xf, acc);
     }
-    bmv_flush(acc, c, L, 1, kWp, sums);
-  } else {
-    auto run = [&](auto mh) {
-      constexpr int MH = decltype(mh)::value;
-      f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
-      for (int s = s_lo; s < s_hi; ++s) {
-        Q6Tile t;
-        ws_tile(t, rowp + s * B, L.kq);
-        bmv_tile<MH>(t, s, L, stride, codes, xs, xf, acc);
-      }
-      bmv_flush<MH>(acc, c, L, 1, kWp, sums);
-    };
-    if (M > 4) run(std::integral_constant<int, 2>{});
-    else run(std::integral_constant<int, 1>{});
-  }
+    bmv_flush<TYPE, MH>(acc, c, L, 1, kWp, sums);
+  };
+  if (TYPE == QK_TYPE_Q4_K || M <= 4)
+    run(std::integral_constant<int, 1>{});
+  else
+    run(std::integral_constant<int, 2>{});
   __syncthreads();
 
   // row totals: the waves' column sums added in wave order; one thread per

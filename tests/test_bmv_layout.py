@@ -517,3 +517,56 @@ def test_bmv_q8h_blocks_close_once(N, M, count):
     for r in range(0, N, max(1, N // 97)):
         g = _owner(r, per, rem)
         assert g * per + min(g, rem) <= r < g * per + min(g, rem) + per + (1 if g < rem else 0)
+
+
+@pytest.mark.parametrize("K", [256, 2560])
+def test_q6k_pair_tile_model(K):
+    """Q6_K at M = 5..8 (bmv_tile6_pair): product p's A rows 4g..4g+3 hold
+    activation rows 4(g & 1).. against k-quarter 2(g >> 1) + p, so that lane
+    (n, kq) gets both sub-blocks of Q8 block 4h + 2nib + (kq >> 1) for activation
+    rows 4(kq & 1)..; every read stays in its LDS array, the integer sums stay
+    below 2^24 at the extreme codes and scales, and the lanes' sums are the
+    product's."""
+    stride, Z, S = K + 16, 8 * (K + 16) + 16, K // 256
+    rng = np.random.default_rng(K)
+    x = rng.integers(-127, 128, (8, K))
+    q, sc = rng.integers(0, 64, (16, K)), rng.integers(-128, 128, (16, K // 16))
+    x[:, :32], q[:, :32], sc[:, :2] = -127, 0, -128  # the extreme: 16 * 127 * 32 * 128, twice
+    xs = rng.standard_normal((K // 32, 8))
+    lds = np.zeros((8, stride), np.int64)
+    lds[:, :K] = x
+    lds = np.concatenate([lds.ravel(), np.zeros(16, np.int64)])
+    neg = -32 * x.reshape(8, -1, 16).sum(2).T  # [K / 16][8]
+    acc = np.zeros((64, 4))
+    klo, khi = LKQ & 1, LKQ >> 1
+    for s in range(S):
+        for h in range(2):
+            for nib in range(2):
+                k0 = 256 * s + 128 * h + 64 * nib
+                blk = 4 * h + 2 * nib + khi
+                total = np.zeros((64, 4), np.int64)
+                for p in range(2):
+                    valid = ((LN >> 3) == khi) & (klo == p)
+                    aoff = np.where(valid, (LN & 7) * stride + 16 * LKQ + k0, 8 * stride)
+                    assert np.all(aoff % 16 == 0) and np.all(aoff + 16 <= 8 * stride + 16)
+                    A, Bm = np.zeros((16, 64), np.int64), np.zeros((64, 16), np.int64)
+                    for l in range(64):
+                        A[LN[l], 16 * LKQ[l]:16 * LKQ[l] + 16] = lds[aoff[l]:aoff[l] + 16]
+                        Bm[16 * LKQ[l]:16 * LKQ[l] + 16, LN[l]] = q[LN[l], k0 + 16 * LKQ[l]:k0 + 16 * LKQ[l] + 16]
+                    D = A @ Bm
+                    off = Z + 2 * K + 4 * ((16 * s + 2 * blk + p) * 8 + 4 * klo)
+                    assert np.all(off >= Z + 2 * K) and np.all(off + 16 <= Z + 4 * K)
+                    sb = 16 * s + 2 * blk + p
+                    for l in range(64):
+                        dot = D[4 * LKQ[l]:4 * LKQ[l] + 4, LN[l]] + neg[sb[l], 4 * klo[l]:4 * klo[l] + 4]
+                        assert np.all(np.abs(dot) < 1 << 23)
+                        total[l] += dot * sc[LN[l], sb[l]]
+                assert np.abs(total).max() <= 1 << 24
+                off = Z + 4 * ((8 * s + blk) * 8 + 4 * klo)
+                assert np.all(off + 16 <= Z + K)
+                for l in range(64):
+                    acc[l] += xs[8 * s + blk[l], 4 * klo[l]:4 * klo[l] + 4] * total[l]
+    v = acc + acc[LANE ^ 32]
+    want = np.einsum("mk,nk->nm", x * np.repeat(xs.T, 32, 1), (q - 32) * np.repeat(sc, 16, 1))
+    for l in range(32):
+        assert np.allclose(v[l], want[LN[l], 4 * LKQ[l]:4 * LKQ[l] + 4], rtol=1e-12)
