@@ -942,15 +942,16 @@ KQPlan plan(int type, int64_t M, int64_t N, int64_t K) {
   if (M <= 32 || M > 65535 || (M > 64 && S < 16)) return rule;
   const int64_t n_tiles = (N + 127) / 128;
   const int64_t tiles32 = ((M + 31) / 32) * n_tiles, tiles64 = ((M + 63) / 64) * n_tiles;
-  // Splits of at least 4 superblocks (2 at M <= 64) that keep the workspace
-  // within the scratch of qk_matmul_noalloc where the rule's plan is within it.
-  const int64_t most = std::clamp<int64_t>(S / (M <= 64 ? 2 : 4), 1, kPlanSplits);
+  // Splits of at least 4 superblocks (2 at M <= 64), no fewer than the rule's
+  // (longer fp32 sums), that keep the workspace within the scratch of
+  // qk_matmul_noalloc where the rule's plan is within it.
+  const int64_t most = std::max<int64_t>(rule.splits, std::clamp<int64_t>(S / (M <= 64 ? 2 : 4), 1, kPlanSplits));
   const int64_t planes = M * K * 4 + M * S * 32 + M * 4 + 512;
   const bool within = planes + (rule.splits > 1 ? rule.splits * M * N * 4 : 0) <= static_cast<int64_t>(QK_NOALLOC_SCRATCH_BYTES);
-  KQPlan best{false, 1};
-  double least = plan_cost(type, false, tiles32, 1, M, N, S);
+  KQPlan best = rule;
+  double least = plan_cost(type, rule.wide, rule.wide ? tiles64 : tiles32, rule.splits, M, N, S);
   for (const bool wide : {false, true})
-    for (int64_t splits = 1; splits <= most; ++splits) {
+    for (int64_t splits = rule.splits; splits <= most; ++splits) {
       if (splits > rule.splits && within &&
           planes + splits * M * N * 4 > static_cast<int64_t>(QK_NOALLOC_SCRATCH_BYTES))
         break;
