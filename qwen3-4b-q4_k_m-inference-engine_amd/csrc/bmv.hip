@@ -1,10 +1,10 @@
 // Batched mat-vec kernel entry (bmv.hpp) and its host launcher: M = 2..8
-// activation rows in fp32, one workgroup per CU, CUs dealt to the segments
-// in proportion to their bytes.
+// activation rows in fp32 or Q8 blocks, one matrix or gate and up, one
+// workgroup per CU.
 #include <algorithm>
 #include <climits>
 
-#include "bmv.hpp"
+#include "bmv_ws.hpp"
 
 namespace qk {
 
@@ -59,25 +59,45 @@ __device__ __forceinline__ void bmv_close_blocks(const BmvParams& p, const BmvSh
                    quantize_quarter(v));
 }
 
-// One type's path of a workgroup: prefetch, quantise, stream, totals.
-template <int TYPE, int MODE, int P>
+// A workgroup's path: prefetch, activations into LDS, stream, totals.
+template <int TYPE, int MODE, bool Q8IN>
 __device__ __forceinline__ void bmv_body(const BmvParams& p, const BmvShare& sh, int rows_seg,
                                          float* yout, int groups_max, unsigned char* lds_raw) {
   constexpr int B = TYPE == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KBytes;
+  constexpr bool kSlots = TYPE == QK_TYPE_Q6_K && MODE == 0;
+  constexpr int P = TYPE == QK_TYPE_Q4_K ? kBmvP4 : kSlots ? kBmvSlotP : kBmvP6;
   constexpr int kParts = MODE == 1 ? 2 : 1;
-  constexpr int kBmvXStaged = TYPE == QK_TYPE_Q4_K ? kBmvXStaged4 : kBmvXStaged6;
+  constexpr int kThreads = 64 * kBmvWaves;
   const int K = p.K, M = p.M, stride = p.stride;
   const int tid = static_cast<int>(threadIdx.x);
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  // activation tasks (8 values each): the first kBmvXStaged per lane load
+  // activations: the first tasks (8 fp32 values) or Q8 blocks per lane load
   // ahead of the weights
   const int groups8 = K / 8, tasks = M * groups8;
-  f32x4 xa[kBmvXStaged], xb[kBmvXStaged];
+  const int bpr = K / 32, nblocks = M * bpr;
+  f32x4 xa[Q8IN ? 1 : kBmvXStaged], xb[Q8IN ? 1 : kBmvXStaged];
+  u32x4 qa[Q8IN ? kBmvQ8Staged : 1], qb[Q8IN ? kBmvQ8Staged : 1], qr[Q8IN ? kBmvQ8Staged : 1];
+  auto load_blocks = [&](int first) {
+    const u32x4* src = reinterpret_cast<const u32x4*>(p.q8);
 #pragma unroll
-  for (int i = 0; i < kBmvXStaged; ++i)
-    load_x_group(p.x, M, K, min(tid + 64 * kBmvWaves * i, tasks - 1), xa[i], xb[i]);
+    for (int i = 0; i < kBmvQ8Staged; ++i) {
+      const int b = min(first + kThreads * i, nblocks - 1);
+      qa[i] = src[3 * b];
+      qb[i] = src[3 * b + 1];
+      qr[i] = src[3 * b + 2];
+    }
+  };
+  auto load_tasks = [&](int first) {
+#pragma unroll
+    for (int i = 0; i < kBmvXStaged; ++i)
+      load_x_group(p.x, M, K, min(first + kThreads * i, tasks - 1), xa[i], xb[i]);
+  };
+  if constexpr (Q8IN)
+    load_blocks(tid);
+  else
+    load_tasks(tid);
   __builtin_amdgcn_sched_barrier(0);
 
   // this wave's units [u_lo, u_hi) and its tile count
@@ -95,11 +115,37 @@ __device__ __forceinline__ void bmv_body(const BmvParams& p, const BmvShare& sh,
   const BmvLane L = bmv_lane(lane, stride);
 
   // the first P tiles
-  BmvTile<TYPE> buf[P];
+  BmvTile<TYPE> buf[kSlots ? 1 : P];
+  u32x4 chunk[kSlots ? P : 1][kBmvSlotLoads];
   BmvCursor lc = start;
+  // slots: this lane's chunks c = lane + 64 j (clamped to the share's last) of
+  // a tile, chunk c % 14 of row c / 14; loads through a descriptor that ends
+  // at the dword boundary at or above the matrix end (dwords past it are zero)
+  uint32_t base[kBmvSlotLoads], q16[kBmvSlotLoads];
+  const int nchunks = kBmvSlotChunks * sh.nrows;
+  const uint32_t end4 = (static_cast<uint32_t>(rows_seg) * static_cast<uint32_t>(sh.row_bytes) + 3u) & ~3u;
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(sh.w[0]), 0, static_cast<int>(end4), 0x00020000);
+  auto issue = [&](u32x4 (&to)[kBmvSlotLoads], int s) {
+#pragma unroll
+    for (int j = 0; j < kBmvSlotLoads; ++j)
+      to[j] = __builtin_amdgcn_raw_buffer_load_b128(
+          rsrc, static_cast<int>(((base[j] + static_cast<uint32_t>(s * B)) & ~3u) + q16[j]), 0, 0);
+  };
+  if constexpr (kSlots) {
+#pragma unroll
+    for (int j = 0; j < kBmvSlotLoads; ++j) {
+      const int c = min(lane + 64 * j, nchunks - 1), row = c / kBmvSlotChunks;
+      base[j] = static_cast<uint32_t>(sh.r0 + row) * static_cast<uint32_t>(sh.row_bytes);
+      q16[j] = 16u * static_cast<uint32_t>(c - kBmvSlotChunks * row);
+    }
+  }
 #pragma unroll
   for (int j = 0; j < P; ++j) {
-    bmv_load(buf[j], bmv_sb<B>(sh, lc, L.n), L.kq);
+    if constexpr (kSlots)
+      issue(chunk[j], lc.s);
+    else
+      bmv_load(buf[j], bmv_sb<B>(sh, lc, L.n), L.kq);
     cursor_next(lc, sh);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -109,52 +155,72 @@ __device__ __forceinline__ void bmv_body(const BmvParams& p, const BmvShare& sh,
   lds_f32* xss = xs + K / 4;
   lds_f32* xf = xs + K / 2;
   lds_f32* sums = xs + K;
-  // Chunk c = tasks tid + 64*kBmvWaves*(kBmvXStaged*c + i), i < kBmvXStaged;
-  // chunk 0 is staged. Wider rows (8 x 4096, 8 x 9728) run the later chunks
-  // two buffers deep: chunk c+1 loads while chunk c is quantised. The loads
-  // are unconditional (clamped into x; a chunk past the end re-reads the last
-  // task) so the waits count them exactly.
-  constexpr int kChunk = 64 * kBmvWaves * kBmvXStaged;
-  auto quantize_chunk = [&](const f32x4 (&a)[kBmvXStaged], const f32x4 (&b)[kBmvXStaged], int c) {
+  // the staged round, then (wide rows) one round after another
+  if constexpr (Q8IN) {
+    for (int b0 = tid; b0 < nblocks; b0 += kThreads * kBmvQ8Staged) {
+      if (b0 != tid) load_blocks(b0);
 #pragma unroll
-    for (int i = 0; i < kBmvXStaged; ++i) {
-      const int t = tid + kChunk * c + 64 * kBmvWaves * i;
-      if (t < tasks) bmv_quantize_task(a[i], b[i], t, groups8, stride, codes, xs, xss, xf);
-    }
-  };
-  auto load_chunk = [&](f32x4 (&a)[kBmvXStaged], f32x4 (&b)[kBmvXStaged], int c) {
-#pragma unroll
-    for (int i = 0; i < kBmvXStaged; ++i)
-      load_x_group(p.x, M, K, min(tid + kChunk * c + 64 * kBmvWaves * i, tasks - 1), a[i], b[i]);
-  };
-  const int chunks = (tasks + kChunk - 1) / kChunk;
-  if (chunks > 1) {
-    f32x4 ya[kBmvXStaged], yb[kBmvXStaged];
-    for (int c = 0; c < chunks; c += 2) {
-      load_chunk(ya, yb, c + 1);
-      quantize_chunk(xa, xb, c);
-      load_chunk(xa, xb, c + 2);
-      if (c + 1 < chunks) quantize_chunk(ya, yb, c + 1);
+      for (int i = 0; i < kBmvQ8Staged; ++i) {
+        const int b = b0 + kThreads * i;
+        if (b < nblocks) bmv_store_block(qa[i], qb[i], qr[i], b, bpr, stride, codes, xs, xss, xf);
+      }
     }
   } else {
-    quantize_chunk(xa, xb, 0);
+    for (int t0 = tid; t0 < tasks; t0 += kThreads * kBmvXStaged) {
+      if (t0 != tid) load_tasks(t0);
+#pragma unroll
+      for (int i = 0; i < kBmvXStaged; ++i) {
+        const int t = t0 + kThreads * i;
+        if (t < tasks) bmv_quantize_task(xa[i], xb[i], t, groups8, stride, codes, xs, xss, xf);
+      }
+    }
   }
   if (tid == 0) *reinterpret_cast<lds_u32x4*>(codes + 8 * stride) = u32x4{0u, 0u, 0u, 0u};
   __syncthreads();
 
-  if constexpr (TYPE == QK_TYPE_Q4_K) {
-    bmv_stream<TYPE, P, 1>(sh, lc, L, stride, groups_max, codes, xs, xss, xf, sums, buf, start);
-  } else {
-    if (M > 4)
-      bmv_stream<TYPE, P, 2>(sh, lc, L, stride, groups_max, codes, xs, xss, xf, sums, buf, start);
-    else
-      bmv_stream<TYPE, P, 1>(sh, lc, L, stride, groups_max, codes, xs, xss, xf, sums, buf, start);
-  }
+  auto stream = [&](auto mh) {
+    constexpr int MH = decltype(mh)::value;
+    if constexpr (kSlots) {
+      lds_u8* slot = (lds_u8*)(sums) + 16 * sh.ranges * 32 + wave * bmv_slot_bytes(p.rows_max);
+      const int n = min(L.n, sh.nrows - 1);  // rows past the share redo its last one and are not stored
+      const lds_u8* row = slot + bmv_slot_bytes(n);
+      BmvCursor cc = start;
+      f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+      const int ntiles = cc.left;
+      for (int t0 = 0; t0 < ntiles; t0 += P) {
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+          if (t0 + j < ntiles) {
+#pragma unroll
+            for (int i = 0; i < kBmvSlotLoads; ++i)
+              *reinterpret_cast<lds_u32x4*>(slot + 16 * min(lane + 64 * i, nchunks - 1)) = chunk[j][i];
+            asm volatile("" ::: "memory");  // (a wave's LDS accesses keep their order)
+            const uint32_t first = static_cast<uint32_t>(sh.r0 + n) * static_cast<uint32_t>(sh.row_bytes);
+            ws_tile6<MH>(row + ((first + static_cast<uint32_t>(cc.s * B)) & 3u), cc.s, L, codes, xs, xf, acc);
+            asm volatile("" ::: "memory");  // the next tile's slot writes follow these reads
+            if (cc.s + 1 == cc.s_end) {
+              bmv_flush<TYPE, MH>(acc, cc, L, groups_max, sh.ranges, sums);
+              acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            cursor_next(cc, sh);
+          }
+          issue(chunk[j], lc.s);  // P tiles ahead (past the end: the last tile again)
+          cursor_next(lc, sh);
+        }
+      }
+    } else {
+      bmv_stream<TYPE, P, MH>(sh, lc, L, stride, groups_max, codes, xs, xss, xf, sums, buf, start);
+    }
+  };
+  if (TYPE == QK_TYPE_Q4_K || M <= 4)
+    stream(std::integral_constant<int, 1>{});
+  else
+    stream(std::integral_constant<int, 2>{});
   __syncthreads();
 
   // row totals: runs added in order; one thread per (activation row, row)
   const int nrows = sh.nrows, R = sh.ranges;
-  for (int idx = tid; idx < nrows * M; idx += 64 * kBmvWaves) {
+  for (int idx = tid; idx < nrows * M; idx += kThreads) {
     const int m = idx / nrows, row = idx - m * nrows;
     const lds_f32* pa = sums + ((row >> 4) * 16 + (row & 15)) * R * 8 + m;
     float a = 0.0f;
@@ -178,33 +244,19 @@ __device__ __forceinline__ void bmv_body(const BmvParams& p, const BmvShare& sh,
   }
 }
 
-// TYPE: QK_TYPE_Q4_K or QK_TYPE_Q6_K for launches of one type, 0 for a mixed
-// launch (each workgroup takes its segment's type).
-template <int TYPE, int MODE>
+template <int TYPE, int MODE, bool Q8IN>
 __global__ __launch_bounds__(64 * kBmvWaves) void bmv_kernel(const BmvParams p) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
 #pragma unroll
-  for (int j = 0; j < kMaxSegments; ++j)
+  for (int j = 0; j < 2; ++j)
     asm volatile("" ::"s"(p.seg[j].w), "s"(p.seg[j].y), "s"(p.seg[j].rows), "s"(p.seg[j].type),
                  "s"(p.seg[j].wg_begin), "s"(p.seg[j].per), "s"(p.seg[j].rem), "s"(p.seg[j].pad));
-  asm volatile("" ::"s"(p.x), "s"(p.h), "s"(p.hq), "s"(p.arrive), "s"(p.M), "s"(p.K), "s"(p.S), "s"(p.nseg),
-               "s"(p.stride), "s"(p.ranges), "s"(p.groups_max), "s"(p.pad));
+  asm volatile("" ::"s"(p.x), "s"(p.q8), "s"(p.h), "s"(p.hq), "s"(p.arrive), "s"(p.M), "s"(p.K), "s"(p.S),
+               "s"(p.stride), "s"(p.ranges), "s"(p.groups_max), "s"(p.rows_max));
   __builtin_amdgcn_sched_barrier(0);
-  const int wg = static_cast<int>(blockIdx.x), nseg = p.nseg;
-  const int j = (nseg > 1 && wg >= p.seg[1].wg_begin) + (nseg > 2 && wg >= p.seg[2].wg_begin) +
-                (nseg > 3 && wg >= p.seg[3].wg_begin);
-  auto pick = [j](auto f0, auto f1, auto f2, auto f3) {
-    return j == 0 ? f0 : j == 1 ? f1 : j == 2 ? f2 : f3;
-  };
-  const int type = pick(p.seg[0].type, p.seg[1].type, p.seg[2].type, p.seg[3].type);
-  const int rows = pick(p.seg[0].rows, p.seg[1].rows, p.seg[2].rows, p.seg[3].rows);
-  const int g = wg - pick(p.seg[0].wg_begin, p.seg[1].wg_begin, p.seg[2].wg_begin, p.seg[3].wg_begin);
-  const int per = pick(p.seg[0].per, p.seg[1].per, p.seg[2].per, p.seg[3].per);
-  const int rem = pick(p.seg[0].rem, p.seg[1].rem, p.seg[2].rem, p.seg[3].rem);
-  float* yout = pick(p.seg[0].y, p.seg[1].y, p.seg[2].y, p.seg[3].y);
-
+  const int g = static_cast<int>(blockIdx.x), per = p.seg[0].per, rem = p.seg[0].rem;
   BmvShare sh;
-  sh.w[0] = pick(p.seg[0].w, p.seg[1].w, p.seg[2].w, p.seg[3].w);
+  sh.w[0] = p.seg[0].w;
   sh.w[1] = MODE == 1 ? p.seg[1].w : sh.w[0];
   sh.r0 = g * per + min(g, rem);
   sh.nrows = per + (g < rem ? 1 : 0);
@@ -215,34 +267,19 @@ __global__ __launch_bounds__(64 * kBmvWaves) void bmv_kernel(const BmvParams p) 
   sh.ranges = p.ranges;
   sh.run_q = p.S / p.ranges;
   sh.run_r = p.S - sh.run_q * p.ranges;
-  if constexpr (TYPE == 0) {
-    if (type == QK_TYPE_Q4_K) {
-      sh.row_bytes = p.S * kQ4KBytes;
-      bmv_body<QK_TYPE_Q4_K, MODE, kBmvP4>(p, sh, rows, yout, p.groups_max, lds_raw);
-    } else {
-      sh.row_bytes = p.S * kQ6KBytes;
-      bmv_body<QK_TYPE_Q6_K, MODE, kBmvP6Mixed>(p, sh, rows, yout, p.groups_max, lds_raw);
-    }
-  } else {
-    sh.row_bytes = p.S * (TYPE == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KBytes);
-    bmv_body<TYPE, MODE, TYPE == QK_TYPE_Q4_K ? kBmvP4 : kBmvP6>(p, sh, rows, yout, p.groups_max, lds_raw);
-  }
+  sh.row_bytes = p.S * (TYPE == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KBytes);
+  bmv_body<TYPE, MODE, Q8IN>(p, sh, p.seg[0].rows, p.seg[0].y, p.groups_max, lds_raw);
 }
 
 using BmvKernel = void (*)(BmvParams);
 
-BmvKernel bmv_kernel_for(int type, int mode) {
-  if (mode == 1) {
-    if (type == QK_TYPE_Q4_K) return &bmv_kernel<QK_TYPE_Q4_K, 1>;
-    if (type == QK_TYPE_Q6_K) return &bmv_kernel<QK_TYPE_Q6_K, 1>;
-    return nullptr;
-  }
-  if (type == QK_TYPE_Q4_K) return &bmv_kernel<QK_TYPE_Q4_K, 0>;
-  if (type == QK_TYPE_Q6_K) return &bmv_kernel<QK_TYPE_Q6_K, 0>;
-  return &bmv_kernel<0, 0>;
+BmvKernel bmv_kernel_for(int type, int mode, bool q8) {
+  if (type == QK_TYPE_Q4_K)
+    return mode == 1 ? &bmv_kernel<QK_TYPE_Q4_K, 1, false>
+                     : q8 ? &bmv_kernel<QK_TYPE_Q4_K, 0, true> : &bmv_kernel<QK_TYPE_Q4_K, 0, false>;
+  return mode == 1 ? &bmv_kernel<QK_TYPE_Q6_K, 1, false>
+                   : q8 ? &bmv_kernel<QK_TYPE_Q6_K, 0, true> : &bmv_kernel<QK_TYPE_Q6_K, 0, false>;
 }
-
-int superblock_bytes(int type) { return type == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KBytes; }
 
 }  // namespace
 
@@ -257,50 +294,31 @@ int64_t bmv_wave_tiles(int64_t rows, int parts, int S, int ranges) {
   return per_wave * ((S + ranges - 1) / ranges);
 }
 
-// The workgroup counts and run split of a launch (shared with the CPU index
+// The workgroup count and run split of a launch (shared with the CPU index
 // model of the tests through the same rules). Returns false when the shape
 // does not fit this kernel's LDS plan.
-bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int (&count)[kMaxSegments],
-              int& ranges, int& groups_max, int& lds) {
-  const int nseg = mode == 1 ? 1 : p.nseg;
+bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int& count, int& ranges, int& groups_max,
+              int& lds) {
   const int parts = mode == 1 ? 2 : 1;
-  if (nseg > cus) return false;
-  double bytes[kMaxSegments] = {0.0}, total = 0.0;
-  for (int j = 0; j < nseg; ++j) {
-    bytes[j] = static_cast<double>(p.seg[j].rows) * p.S * superblock_bytes(p.seg[j].type) * parts;
-    total += bytes[j];
-  }
-  int sum = 0;
-  for (int j = 0; j < nseg; ++j) {
-    count[j] = std::clamp(static_cast<int>(cus * bytes[j] / total + 0.5), 1, p.seg[j].rows);
-    sum += count[j];
-  }
-  while (sum > cus) {  // trim the segment with the most workgroups
-    int big = 0;
-    for (int j = 1; j < nseg; ++j)
-      if (count[j] > count[big]) big = j;
-    --count[big];
-    --sum;
-  }
+  const int rows = p.seg[0].rows;
+  count = std::clamp(cus, 1, rows);
   const int stride = p.K + 16;
-  groups_max = 0;
-  for (int j = 0; j < nseg; ++j) {
-    const int rows_max = (p.seg[j].rows + count[j] - 1) / count[j];
-    groups_max = std::max(groups_max, (rows_max + 15) / 16);
-  }
+  const int rows_max = (rows + count - 1) / count;
+  groups_max = (rows_max + 15) / 16;
+  const bool slots = mode == 0 && p.seg[0].type == QK_TYPE_Q6_K;
+  if (slots && (rows_max > kBmvSlotRows || static_cast<int64_t>(rows) * p.S * kQ6KBytes + 16 > INT32_MAX)) return false;
+  const int slot_bytes = slots ? kBmvWaves * bmv_slot_bytes(rows_max) : 0;
   // runs per group: the fewest tiles on the busiest wave of any workgroup,
   // then the fewest units (each unit ends with a lane reduction)
   ranges = 0;
   int64_t best = INT64_MAX;
   for (int r = 1; r <= p.S; ++r) {
-    if (bmv_lds_bytes(p.K, stride, parts, groups_max, r) > max_lds) break;
+    if (bmv_lds_bytes(p.K, stride, parts, groups_max, r) + slot_bytes > max_lds) break;
     int64_t tiles = 0, units = 0;
-    for (int j = 0; j < nseg; ++j) {
-      const int per = p.seg[j].rows / count[j];
-      for (int n : {per, per + 1}) {
-        tiles = std::max(tiles, bmv_wave_tiles(n, parts, p.S, r));
-        units = std::max<int64_t>(units, (parts * ((n + 15) / 16) * r + kBmvWaves - 1) / kBmvWaves);
-      }
+    const int per = rows / count;
+    for (int n : {per, per + 1}) {
+      tiles = std::max(tiles, bmv_wave_tiles(n, parts, p.S, r));
+      units = std::max<int64_t>(units, (parts * ((n + 15) / 16) * r + kBmvWaves - 1) / kBmvWaves);
     }
     const int64_t cost = 8 * tiles + units;
     if (cost < best) {
@@ -309,59 +327,55 @@ bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int (&count
     }
   }
   if (ranges == 0) return false;
-  lds = bmv_lds_bytes(p.K, stride, parts, groups_max, ranges);
+  lds = bmv_lds_bytes(p.K, stride, parts, groups_max, ranges) + slot_bytes;
   return true;
 }
 
 hipError_t launch_bmv(const MatvecParams& p, int mode, hipStream_t stream, bool& launched) {
   launched = false;
-  // The gate/up launch (mode 1) only, for now: measured on MI355X at M = 8
-  // against the streaming and batched whole-share kernels, gate/up 14.7 us
-  // against 19.1; the one-matrix and q/k/v launches are not yet faster here.
-  if (p.x == nullptr || p.M < 2 || p.M > 8 || mode != 1) return hipSuccess;
+  // Gate/up (mode 1), and at M >= 3 one matrix (mode 0) of at most 16 rows a
+  // workgroup (Q6_K: 13) that the whole-share kernel does not take (its weights
+  // and activations exceed LDS: ffn_down, K = 9728). Measured on MI355X, us, the
+  // streaming kernel before: ffn_down in fp32 Q4_K at M = 3 / 8 13.2 / 22.2 ->
+  // 9.5 / 14.6, Q6_K 13.1 / 22.4 -> 12.2 / 17.9; at M = 2 it is the faster one
+  // (9.2 against 9.5, 10.3 against 11.4).
+  if (p.M < (mode == 1 ? 2 : 3) || p.M > 8 || (mode != 0 && mode != 1)) return hipSuccess;
+  if (mode == 1 ? p.x == nullptr || p.nseg != 2 : p.nseg != 1) return hipSuccess;
   if (p.K > (INT32_MAX - 64) / 8) return hipSuccess;
   int cus = 0, max_lds = 0;
   hipError_t e = device_limits(cus, max_lds);
   if (e != hipSuccess) return e;
-  int count[kMaxSegments] = {0}, ranges = 0, groups_max = 0, lds = 0;
+  int count = 0, ranges = 0, groups_max = 0, lds = 0;
   if (!bmv_plan(p, mode, cus, max_lds, count, ranges, groups_max, lds)) return hipSuccess;
+  if (mode == 0 && groups_max > 1) return hipSuccess;
   if (p.hq != nullptr) {  // Q8(h) in the launch: a quad per (block, activation row) of a share
-    const int64_t rows_max = (p.seg[0].rows + count[0] - 1) / count[0];
+    const int64_t rows_max = (p.seg[0].rows + count - 1) / count;
     const int64_t blocks = (rows_max + 30) / 32 + 1;  // blocks a run of rows_max rows can touch
     if (p.seg[0].rows % 32 != 0 || blocks > kBmvMaxCloseBlocks || 4 * blocks * p.M > 64 * kBmvWaves ||
         p.arrive == nullptr)
       return hipSuccess;
   }
 
-  const int nseg = mode == 1 ? 1 : p.nseg;
   BmvParams bp{};
   bp.x = p.x;
+  bp.q8 = p.x == nullptr ? p.q8 : nullptr;
   bp.h = p.h;
   bp.hq = p.hq;
   bp.arrive = p.hq != nullptr ? p.arrive : nullptr;
   bp.M = p.M;
   bp.K = p.K;
   bp.S = p.S;
-  bp.nseg = nseg;
   bp.stride = p.K + 16;
   bp.ranges = ranges;
   bp.groups_max = groups_max;
-  bool q4 = false, q6 = false;
-  int begin = 0;
-  for (int j = 0; j < nseg; ++j) {
-    bp.seg[j] = {p.seg[j].w, p.seg[j].y, p.seg[j].rows, p.seg[j].type, begin,
-                 p.seg[j].rows / count[j], p.seg[j].rows % count[j], 0};
-    (p.seg[j].type == QK_TYPE_Q4_K ? q4 : q6) = true;
-    begin += count[j];
-  }
-  if (mode == 1) bp.seg[1] = {p.seg[1].w, nullptr, p.seg[1].rows, p.seg[1].type, 0, 0, 0, 0};
-  const int type = q4 && q6 ? 0 : q4 ? QK_TYPE_Q4_K : QK_TYPE_Q6_K;
-  const BmvKernel fn = bmv_kernel_for(type, mode);
-  if (!fn) return hipSuccess;
+  bp.rows_max = (p.seg[0].rows + count - 1) / count;
+  for (int j = 0; j < (mode == 1 ? 2 : 1); ++j)
+    bp.seg[j] = {p.seg[j].w, p.seg[j].y, p.seg[j].rows, p.seg[j].type, 0, p.seg[0].rows / count, p.seg[0].rows % count, 0};
+  const BmvKernel fn = bmv_kernel_for(p.seg[0].type, mode, p.x == nullptr);
   e = allow_lds(reinterpret_cast<const void*>(fn), lds);
   if (e != hipSuccess) return e;
-  note("bmv_kernel", begin, type, mode, ranges, groups_max, p.hq != nullptr);
-  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(begin)), dim3(64 * kBmvWaves),
+  note("bmv_kernel", count, p.seg[0].type, mode, ranges, groups_max, p.hq != nullptr);
+  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(count)), dim3(64 * kBmvWaves),
                      static_cast<size_t>(lds), stream, bp);
   launched = true;
   return hipGetLastError();

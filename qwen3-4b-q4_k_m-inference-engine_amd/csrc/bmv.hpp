@@ -1,6 +1,6 @@
 // Batched mat-vec on the int8 matrix cores: M = 2..8 activation rows (the
 // decode batch of several sequences), fp32 activations quantised in the
-// kernel. Replaces quantize + project<Q4_K/Q6_K> with gridDim.y = rows
+// kernel or Q8 blocks copied in. Replaces quantize + project<Q4_K/Q6_K> with gridDim.y = rows
 // (src/cuda/matmul.cu:8-22, 86-125, 151-158), which re-reads every weight row
 // once per activation row.
 //
@@ -27,8 +27,8 @@
 // fp32 (Q4_K: d*sc*xs*dot - dmin*m*xs*sum(codes); Q6_K: d*sc*xs*(dot - 32
 // sum(codes)), src/cuda/matmul.cu:24-84).
 //
-// A workgroup (one per CU) owns a contiguous range of rows of one segment;
-// its rows are cut into groups of 16 and each group's superblock columns
+// A workgroup (one per CU) owns a contiguous range of rows (mode 1: of gate
+// and of up); its rows are cut into groups of 16 and each group's superblock columns
 // into `ranges` runs. Work units (part, group, run) are dealt to the waves in
 // contiguous blocks; a wave streams its units' tiles (16 rows x one
 // superblock) through a ring of P register buffers, P tiles ahead, so
@@ -43,32 +43,40 @@
 
 namespace qk {
 
-// 8 waves of up to 256 registers each: deep per-wave tile rings without
-// spills (a scratch reload counts in the same vmcnt as the weight loads, so
-// one spill in the loop would serialise the stream)
-constexpr int kBmvWaves = 8;    // waves per workgroup (one workgroup per CU)
-// activation tasks per lane whose loads are issued before the weights (held
-// in registers with the first tiles during the quantisation)
-constexpr int kBmvXStaged4 = 5;
-constexpr int kBmvXStaged6 = 5;
-constexpr int kBmvP4 = 6;       // Q4_K tiles in flight per wave
-constexpr int kBmvP6 = 4;       // Q6_K tiles in flight per wave
-constexpr int kBmvP6Mixed = 3;  // Q6_K tiles in flight in a launch with both types
+// 16 waves with shallow rings: a wave has 1 to 4 tiles, so deep rings mostly
+// load tiles again past its end, and four waves a SIMD hide the LDS reads and
+// the MFMAs of each other's tiles. Measured, gate/up (Q4_K) at M = 3 / 8: 8
+// waves with rings of 6 13.6 / 14.7 us, 16 waves with rings of 4 12.4 / 13.0, of
+// 2 11.0 / 11.8 (of 1: equal); Q6_K 26.1 / 27.3 -> 22.0 / 23.2.
+constexpr int kBmvWaves = 16;   // waves per workgroup (one workgroup per CU)
+// activation tasks (Q8 blocks) per lane whose loads are issued before the
+// weights
+constexpr int kBmvXStaged = 2;
+constexpr int kBmvQ8Staged = 2;
+constexpr int kBmvP4 = 2;       // Q4_K tiles in flight per wave
+constexpr int kBmvP6 = 1;       // Q6_K tiles in flight per wave (mode 1)
+// Q6_K in mode 0: a tile's rows go through a slot of the wave in LDS
+constexpr int kBmvSlotChunks = 14;  // 16-byte chunks that cover a superblock from the dword boundary below it
+constexpr int kBmvSlotLoads = 3;    // chunks per lane and tile
+constexpr int kBmvSlotRows = 64 * kBmvSlotLoads / kBmvSlotChunks;  // rows of a workgroup at most: 13
+constexpr int kBmvSlotP = 1;        // tiles in flight per wave
 // Q8 blocks of h one workgroup may complete (M activation rows each, a quad
 // per block row): the launcher checks blocks * M * 4 <= threads.
 constexpr int kBmvMaxCloseBlocks = 16;
 
 struct BmvParams {
-  const float* x;       // [M x K]
+  const float* x;       // [M x K], or null:
+  const qk_q8_block* q8;  // [M x K/32] (mode 0)
   float* h;             // mode 1 output [M x N]
   qk_q8_block* hq;      // mode 1, optional: Q8 of h [M][N/32], formed in the launch
   uint32_t* arrive;     // with hq: per-block arrival counters [N/32], zero between launches
-  int32_t M, K, S, nseg;
+  int32_t M, K, S;
   int32_t stride;      // LDS bytes per activation row of codes (K + 16)
   int32_t ranges;      // superblock runs per row group
   int32_t groups_max;  // row groups of the largest workgroup share
+  int32_t rows_max;    // its rows
   int32_t pad;
-  StreamSegment seg[kMaxSegments];
+  StreamSegment seg[2];  // the matrix; mode 1: gate and up
 };
 
 // LDS image (byte offsets; K a multiple of 256):
@@ -79,12 +87,14 @@ struct BmvParams {
 //   xf    [K/16][8] int32 -32*(sum of 16 codes)    at Z + 2K (the Q6_K offset,
 //                                                  the MFMA's accumulator input)
 //   sums  [parts][groups_max][16][ranges][8] fp32  at Z + 4K
+//   slots [waves][rows][14 chunks]                 after the sums (Q6_K, mode 0)
 // Rows m >= M of every array are left unwritten: they feed only results for
 // activation rows that are never stored.
 __host__ __device__ constexpr int bmv_lds_z(int stride) { return 8 * stride + 16; }
 __host__ __device__ constexpr int bmv_lds_bytes(int K, int stride, int parts, int groups, int ranges) {
   return bmv_lds_z(stride) + 4 * K + parts * groups * 16 * ranges * 32;
 }
+__host__ __device__ constexpr int bmv_slot_bytes(int rows) { return 16 * kBmvSlotChunks * rows; }
 
 typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 
@@ -108,6 +118,27 @@ __device__ __forceinline__ void bmv_quantize_task(f32x4 a, f32x4 b, int t, int g
     xi[(2 * blk) * 8 + m] = -32 * q.pair;
     xi[(2 * blk + 1) * 8 + m] = -32 * q.other;
   }
+}
+
+// Block b of caller-provided Q8 blocks [M][K/32] (its three 16-byte words:
+// codes 0..15, codes 16..31, then scale / scale*sum / -32*sum(0..15) /
+// -32*sum(16..31)) into the LDS image bmv_quantize_task writes: the same
+// codes, the same scale, the same fp32 product scale*sum and the same
+// integer offsets. The record is bit cast as a whole vector: a bit cast of
+// one subscripted element (rec.y) was compiled as the vector's first element.
+__device__ __forceinline__ void bmv_store_block(u32x4 c0, u32x4 c1, u32x4 rec, int b, int bpr, int stride,
+                                                lds_u8* codes, lds_f32* xs, lds_f32* xss, lds_f32* xf) {
+  const int m = b / bpr, blk = b - m * bpr;
+  lds_u8* row = codes + m * stride + 32 * blk;
+  *reinterpret_cast<lds_u32x4*>(row) = c0;
+  *reinterpret_cast<lds_u32x4*>(row + 16) = c1;
+  const f32x4 rf = __builtin_bit_cast(f32x4, rec);
+  const float scale = rf.x;
+  xs[blk * 8 + m] = scale;
+  xss[blk * 8 + m] = rf.y;
+  lds_i32* xi = reinterpret_cast<lds_i32*>(xf);
+  xi[(2 * blk) * 8 + m] = static_cast<int32_t>(rec.z);
+  xi[(2 * blk + 1) * 8 + m] = static_cast<int32_t>(rec.w);
 }
 
 // A lane's register image of one tile (16 rows x one superblock).
@@ -228,12 +259,11 @@ __device__ __forceinline__ void bmv_tile(const Q4Tile& t, int s, const BmvLane& 
   for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(-dmin, minv[i], __builtin_fmaf(d, mainv[i], acc[i]));
 }
 
-// 16 codes of a Q6_K tile's half h and nibble nib (ql nibble | qh pair << 4,
-// 0..63): src/cuda/matmul.cu:71-79. sh0 / sh1 move the qh bit pair of group
-// 2 nib + (k-quarter >> 1) to bits 4-5 of each byte.
-__device__ __forceinline__ u32x4 bmv_codes6(const Q6Tile& t, int h, int nib, uint32_t sh) {
-  const u32x4 ql = h ? t.lb : t.la;
-  const u32x4 qh = h ? t.hb : t.ha;
+// 16 codes of nibble nib of a Q6_K half's bytes (ql nibble | qh pair << 4,
+// 0..63): src/cuda/matmul.cu:71-79. The qh bit pair of group 2 nib + khi moves
+// to bits 4-5 of each byte.
+__device__ __forceinline__ u32x4 bmv_codes6(u32x4 ql, u32x4 qh, int nib, int khi) {
+  const uint32_t sh = (nib ? 0u : 28u) + 2u * static_cast<uint32_t>(khi);
   u32x4 b;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -243,76 +273,58 @@ __device__ __forceinline__ u32x4 bmv_codes6(const Q6Tile& t, int h, int nib, uin
   return b;
 }
 
-// Q6_K tile at superblock column s, M <= 4: acc[i] += row n's dot for
-// activation row i over the sub-blocks 8h+4nib+kq (the other kq in lanes l^16,
-// l^32). The -32 offset of the codes enters as the MFMA's accumulator input
-// -32 * sum(activation codes), so the integer dot is exact.
-__device__ __forceinline__ void bmv_tile6(const Q6Tile& t, int s, const BmvLane& L, const lds_u8* codes,
-                                          const lds_f32* xs, const lds_f32* xf, f32x4& acc) {
-  const int khi = L.kq >> 1;
-  const uint32_t sh0 = 28u + 2u * static_cast<uint32_t>(khi), sh1 = 2u * static_cast<uint32_t>(khi);
-  f32x4 accsb = {0.0f, 0.0f, 0.0f, 0.0f};
+// Half h of a Q6_K tile at superblock column s (sc[nib]: scales 8h+4nib..+3).
+// The -32 offset of the codes enters as the MFMA's accumulator input
+// -32 * sum(activation codes), so the integer dots are exact.
+//  MH = 1 (M <= 4): acc[i] += row n's dot for activation row i over the
+//    sub-blocks 8h+4nib+kq (the other kq in lanes l^16, l^32).
+//  MH = 2 (M = 5..8): acc[i] += the dot for activation row 4*(kq&1)+i over the
+//    Q8 blocks 4h+2nib+(kq>>1) (the others in lane l^32). A rows 4g..4g+3 hold
+//    activation rows 4*(g&1).. against k-quarter 2*(g>>1)+p in product p, so a
+//    lane's two products are the two sub-blocks of ONE Q8 block and the same
+//    four activation rows: sc0*dot0 + sc1*dot1 is formed in integers (|dot| <=
+//    16*127*32 < 2^17 and |sc| <= 128: exact in 32 bits) and takes one
+//    conversion and one block scale, where a product of its own per half of
+//    the activation rows took two of each (lm_head at M = 5 / 8: 79.2 / 80.2
+//    -> 75.4 / 76.4 us).
+template <int MH>
+__device__ __forceinline__ void bmv_half6(u32x4 ql, u32x4 qh, uint32_t sc0, uint32_t sc1, int h, int s,
+                                          const BmvLane& L, const lds_u8* codes, const lds_f32* xs,
+                                          const lds_f32* xf, f32x4& acc) {
+  const int khi = L.kq >> 1, klo = L.kq & 1;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-#pragma unroll
-    for (int nib = 0; nib < 2; ++nib) {
-      const u32x4 b = bmv_codes6(t, h, nib, nib ? sh1 : sh0);
+  for (int nib = 0; nib < 2; ++nib) {
+    const u32x4 b = bmv_codes6(ql, qh, nib, khi);
+    const uint32_t scw = nib ? sc1 : sc0;
+    const int blk = 4 * h + 2 * nib + khi;  // this lane's Q8 block
+    const lds_u8* neg = reinterpret_cast<const lds_u8*>(xf);
+    if constexpr (MH == 1) {
       const int sb16 = 8 * h + 4 * nib + L.kq;  // this lane's sub-block
-      const float scf = static_cast<float>(static_cast<int8_t>((t.sc[2 * h + nib] >> (8 * L.kq)) & 0xFFu));
-      const int blk = 4 * h + 2 * nib + khi;  // its Q8 block
+      const float scf = static_cast<float>(static_cast<int8_t>((scw >> (8 * L.kq)) & 0xFFu));
       const uint32_t aoff = L.a6_valid ? L.a6_base + 256 * s + 128 * h + 64 * nib : L.zero;
-      const i32x4 n4 = lds_read_i32x4(reinterpret_cast<const lds_u8*>(xf), 4u * ((16 * s + sb16) * 8));
+      const i32x4 n4 = lds_read_i32x4(neg, 4u * ((16 * s + sb16) * 8));
       const i32x4 ci = mfma_i8(lds_read_i32x4(codes, aoff), b, n4);
       const f32x4 x4 = lds_read_f32x4(xs + (8 * s + blk) * 8);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) accsb[i] = __builtin_fmaf(scf, x4[i] * static_cast<float>(ci[i]), accsb[i]);
-    }
-  }
-  const float d = half_bits_to_float(t.d);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(d, accsb[i], acc[i]);
-}
-
-// Q6_K tile, M = 5..8: acc[i] += row n's dot for activation row 4*(kq&1)+i
-// over the Q8 blocks 4h+2nib+(kq>>1) (the others in lane l^32). A rows 4g..
-// 4g+3 hold activation rows 4*(g&1).. against k-quarter 2*(g>>1)+p in product
-// p, so a lane's two products are the two sub-blocks of ONE Q8 block and the
-// same four activation rows: sc0*dot0 + sc1*dot1 is formed in integers (|dot|
-// <= 16*127*32 < 2^17 and |sc| <= 128: exact in 32 bits) and takes one
-// conversion and one block scale, where a product of its own per half of the
-// activation rows took two of each (lm_head at M = 5 / 8: 79.2 / 80.2 -> 75.4 / 76.4 us).
-__device__ __forceinline__ void bmv_tile6_pair(const Q6Tile& t, int s, const BmvLane& L, const lds_u8* codes,
-                                               const lds_f32* xs, const lds_f32* xf, f32x4& acc) {
-  const int khi = L.kq >> 1, klo = L.kq & 1;
-  const uint32_t sh0 = 28u + 2u * static_cast<uint32_t>(khi), sh1 = 2u * static_cast<uint32_t>(khi);
-  f32x4 accsb = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-#pragma unroll
-    for (int nib = 0; nib < 2; ++nib) {
-      const u32x4 b = bmv_codes6(t, h, nib, nib ? sh1 : sh0);
-      const int blk = 4 * h + 2 * nib + khi;  // this lane's Q8 block
+      for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(scf, x4[i] * static_cast<float>(ci[i]), acc[i]);
+    } else {
       i32x4 dot[2];
       int sc[2];
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         const uint32_t aoff = L.a6p_valid[p] ? L.a6p_base + 256 * s + 128 * h + 64 * nib : L.zero;
-        const i32x4 n4 =
-            lds_read_i32x4(reinterpret_cast<const lds_u8*>(xf), 4u * ((16 * s + 2 * blk + p) * 8 + 4 * klo));
+        const i32x4 n4 = lds_read_i32x4(neg, 4u * ((16 * s + 2 * blk + p) * 8 + 4 * klo));
         dot[p] = mfma_i8(lds_read_i32x4(codes, aoff), b, n4);
-        sc[p] = __builtin_amdgcn_sbfe(static_cast<int>(t.sc[2 * h + nib]), 16 * khi + 8 * p, 8);
+        sc[p] = __builtin_amdgcn_sbfe(static_cast<int>(scw), 16 * khi + 8 * p, 8);
       }
       const f32x4 x4 = lds_read_f32x4(xs + (8 * s + blk) * 8 + 4 * klo);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int sum = __mul24(dot[0][i], sc[0]) + __mul24(dot[1][i], sc[1]);
-        accsb[i] = __builtin_fmaf(x4[i], static_cast<float>(sum), accsb[i]);
+        acc[i] = __builtin_fmaf(x4[i], static_cast<float>(sum), acc[i]);
       }
     }
   }
-  const float d = half_bits_to_float(t.d);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(d, accsb[i], acc[i]);
 }
 
 // The tile of either type: MH = 1 for M <= 4, 2 for M = 5..8 (Q4_K: the same).
@@ -324,10 +336,12 @@ __device__ __forceinline__ void bmv_tile_any(const Q4Tile& t, int s, const BmvLa
 template <int MH>
 __device__ __forceinline__ void bmv_tile_any(const Q6Tile& t, int s, const BmvLane& L, int, const lds_u8* codes,
                                              const lds_f32* xs, const lds_f32*, const lds_f32* xf, f32x4& acc) {
-  if constexpr (MH == 1)
-    bmv_tile6(t, s, L, codes, xs, xf, acc);
-  else
-    bmv_tile6_pair(t, s, L, codes, xs, xf, acc);
+  f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+  bmv_half6<MH>(t.la, t.ha, t.sc.x, t.sc.y, 0, s, L, codes, xs, xf, sum);
+  bmv_half6<MH>(t.lb, t.hb, t.sc.z, t.sc.w, 1, s, L, codes, xs, xf, sum);
+  const float d = half_bits_to_float(t.d);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(d, sum[i], acc[i]);
 }
 
 // A unit's sums over its lanes: every lane of the result holds activation rows

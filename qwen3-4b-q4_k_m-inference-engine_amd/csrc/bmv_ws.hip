@@ -56,7 +56,7 @@ bool bmv_ws_plan(const MatvecParams& p, int mode, int cus, int max_lds, BmvWsPla
     --plan.count[big];
     --sum;
   }
-  const int rpw = 16 / (kBmvWaves / parts);
+  const int rpw = 16 / (kWsWaves / parts);
   int rows_max = 0;
   plan.reg = 0;
   for (int j = 0; j < nseg; ++j) {
@@ -66,8 +66,8 @@ bool bmv_ws_plan(const MatvecParams& p, int mode, int cus, int max_lds, BmvWsPla
     plan.reg = std::max(plan.reg, bmv_ws_reg_bytes(rpw, static_cast<int>(row_bytes)));
   }
   if (rows_max > 16) return false;
-  const int64_t staged = p.x != nullptr ? static_cast<int64_t>(p.M) * (p.K / 8) - 64 * kBmvWaves * kWsXStaged
-                                        : static_cast<int64_t>(p.M) * (p.K / 32) - 64 * kBmvWaves * kWsQ8Staged;
+  const int64_t staged = p.x != nullptr ? static_cast<int64_t>(p.M) * (p.K / 8) - 64 * kWsWaves * kWsXStaged
+                                        : static_cast<int64_t>(p.M) * (p.K / 32) - 64 * kWsWaves * kWsQ8Staged;
   if (staged > 0) return false;
   plan.lds = bmv_ws_lds_bytes(p.K, parts, plan.reg);
   return plan.lds <= max_lds;
@@ -112,7 +112,7 @@ hipError_t launch_bmv_ws(const MatvecParams& p, int mode, hipStream_t stream, bo
   e = allow_lds(reinterpret_cast<const void*>(fn), plan.lds);
   if (e != hipSuccess) return e;
   note("bmv_ws_kernel", begin, type, mode, q8in, plan.reg);
-  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(begin)), dim3(64 * kBmvWaves),
+  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(begin)), dim3(64 * kWsWaves),
                      static_cast<size_t>(plan.lds), stream, bp);
   launched = true;
   return hipGetLastError();

@@ -33,6 +33,8 @@
 
 namespace qk {
 
+constexpr int kWsWaves = 8;  // waves per workgroup (one workgroup per CU)
+
 constexpr int kWsJ = 6;         // 16-byte loads per lane
 constexpr int kWsXStaged = 8;   // fp32 activation tasks per lane, all staged ahead of the weights
 constexpr int kWsQ8Staged = 4;  // Q8-input blocks per lane, all staged
@@ -106,25 +108,26 @@ __device__ __forceinline__ void ws_tile(Q6Tile& t, const lds_u8* sb, int kq) {
   t.d = __builtin_amdgcn_alignbit(b[53], b[52], sh) & 0xFFFFu;  // d at byte 208
 }
 
-// Block b of caller-provided Q8 blocks [M][K/32] (its three 16-byte words:
-// codes 0..15, codes 16..31, then scale / scale*sum / -32*sum(0..15) /
-// -32*sum(16..31)) into the LDS image bmv_quantize_task writes: the same
-// codes, the same scale, the same fp32 product scale*sum and the same
-// integer offsets. The record is bit cast as a whole vector: a bit cast of
-// one subscripted element (rec.y) was compiled as the vector's first element.
-__device__ __forceinline__ void bmv_store_block(u32x4 c0, u32x4 c1, u32x4 rec, int b, int bpr, int stride,
-                                                lds_u8* codes, lds_f32* xs, lds_f32* xss, lds_f32* xf) {
-  const int m = b / bpr, blk = b - m * bpr;
-  lds_u8* row = codes + m * stride + 32 * blk;
-  *reinterpret_cast<lds_u32x4*>(row) = c0;
-  *reinterpret_cast<lds_u32x4*>(row + 16) = c1;
-  const f32x4 rf = __builtin_bit_cast(f32x4, rec);
-  const float scale = rf.x;
-  xs[blk * 8 + m] = scale;
-  xss[blk * 8 + m] = rf.y;
-  lds_i32* xi = reinterpret_cast<lds_i32*>(xf);
-  xi[(2 * blk) * 8 + m] = static_cast<int32_t>(rec.z);
-  xi[(2 * blk + 1) * 8 + m] = static_cast<int32_t>(rec.w);
+// The Q6_K tile of a superblock in LDS, one half's fields at a time (fewer
+// registers than the whole image).
+template <int MH>
+__device__ __forceinline__ void ws_tile6(const lds_u8* sb, int s, const BmvLane& L, const lds_u8* codes,
+                                         const lds_f32* xs, const lds_f32* xf, f32x4& acc) {
+  const uint32_t mis = lds_offset(sb) & 3u, sh = 8u * mis;
+  const lds_u32_t* b = reinterpret_cast<const lds_u32_t*>(sb - mis);
+  f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const u32x4 ql = lds16_realign(b, 16 * h + 4 * L.kq, sh);
+    const u32x4 qh = lds16_realign(b, 32 + 8 * h + 4 * (L.kq & 1), sh);
+    const uint32_t d0 = b[48 + 2 * h], d1 = b[49 + 2 * h], d2 = b[50 + 2 * h];
+    bmv_half6<MH>(ql, qh, __builtin_amdgcn_alignbit(d1, d0, sh), __builtin_amdgcn_alignbit(d2, d1, sh), h, s, L, codes,
+                  xs, xf, sum);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const float d = half_bits_to_float(__builtin_amdgcn_alignbit(b[53], b[52], sh) & 0xFFFFu);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(d, sum[i], acc[i]);
 }
 
 // One type's path of a workgroup: rows [r0, r0 + nrows) (nrows <= 16) of a
@@ -135,7 +138,7 @@ __device__ __forceinline__ void bmv_ws_body(const BmvWsParams& p, const uint8_t*
                                             unsigned char* lds_raw) {
   constexpr int B = TYPE == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KBytes;
   constexpr int kParts = MODE == 1 ? 2 : 1;
-  constexpr int kWp = kBmvWaves / kParts;  // waves per part
+  constexpr int kWp = kWsWaves / kParts;  // waves per part
   constexpr int kRpw = 16 / kWp;           // rows per wave
   const int K = p.K, M = p.M, S = p.S, stride = p.stride;
   const int tid = static_cast<int>(threadIdx.x);
@@ -154,7 +157,7 @@ __device__ __forceinline__ void bmv_ws_body(const BmvWsParams& p, const uint8_t*
     const u32x4* src = reinterpret_cast<const u32x4*>(p.q8);
 #pragma unroll
     for (int i = 0; i < kWsQ8Staged; ++i) {
-      const int b = min(tid + 64 * kBmvWaves * i, nblocks - 1);
+      const int b = min(tid + 64 * kWsWaves * i, nblocks - 1);
       qa[i] = src[3 * b];
       qb[i] = src[3 * b + 1];
       qr[i] = src[3 * b + 2];
@@ -162,7 +165,7 @@ __device__ __forceinline__ void bmv_ws_body(const BmvWsParams& p, const uint8_t*
   } else {
 #pragma unroll
     for (int i = 0; i < kWsXStaged; ++i)
-      load_x_group(p.x, M, K, min(tid + 64 * kBmvWaves * i, tasks - 1), xa[i], xb[i]);
+      load_x_group(p.x, M, K, min(tid + 64 * kWsWaves * i, tasks - 1), xa[i], xb[i]);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -187,13 +190,13 @@ __device__ __forceinline__ void bmv_ws_body(const BmvWsParams& p, const uint8_t*
   if constexpr (Q8IN) {
 #pragma unroll
     for (int i = 0; i < kWsQ8Staged; ++i) {
-      const int b = tid + 64 * kBmvWaves * i;
+      const int b = tid + 64 * kWsWaves * i;
       if (b < nblocks) bmv_store_block(qa[i], qb[i], qr[i], b, bpr, stride, codes, xs, xss, xf);
     }
   } else {
 #pragma unroll
     for (int i = 0; i < kWsXStaged; ++i) {
-      const int t = tid + 64 * kBmvWaves * i;
+      const int t = tid + 64 * kWsWaves * i;
       if (t < tasks) bmv_quantize_task(xa[i], xb[i], t, groups8, stride, codes, xs, xss, xf);
     }
   }
@@ -247,7 +250,7 @@ __device__ __forceinline__ void bmv_ws_body(const BmvWsParams& p, const uint8_t*
 
   // row totals: the waves' column sums added in wave order; one thread per
   // (activation row, row)
-  for (int idx = tid; idx < nrows * M; idx += 64 * kBmvWaves) {
+  for (int idx = tid; idx < nrows * M; idx += 64 * kWsWaves) {
     const int m = idx / nrows, row = idx - m * nrows;
     const lds_f32* pa = sums + row * kWp * 8 + m;
     float a = 0.0f;
@@ -268,7 +271,7 @@ __device__ __forceinline__ void bmv_ws_body(const BmvWsParams& p, const uint8_t*
 // TYPE: QK_TYPE_Q4_K or QK_TYPE_Q6_K, or 0 for a launch of both types (each
 // workgroup takes its segment's type).
 template <int TYPE, int MODE, bool Q8IN>
-__global__ __launch_bounds__(64 * kBmvWaves) void bmv_ws_kernel(const BmvWsParams p) {
+__global__ __launch_bounds__(64 * kWsWaves) void bmv_ws_kernel(const BmvWsParams p) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
 #pragma unroll
   for (int j = 0; j < kMaxSegments; ++j)

@@ -570,3 +570,51 @@ def test_q6k_pair_tile_model(K):
     want = np.einsum("mk,nk->nm", x * np.repeat(xs.T, 32, 1), (q - 32) * np.repeat(sc, 16, 1))
     for l in range(32):
         assert np.allclose(v[l], want[LN[l], 4 * LKQ[l]:4 * LKQ[l] + 4], rtol=1e-12)
+
+
+# The launch form of bmv.hpp: 16 waves, rings of 2 (Q4_K) and 1 (Q6_K) tiles;
+# one matrix (mode 0) in up to 16 rows a workgroup, Q6_K through LDS slots.
+@pytest.mark.parametrize("rows,types,K,mode,M", [
+    ([9728, 9728], [12, 12], 2560, 1, 8), ([9728, 9728], [14, 14], 2560, 1, 3), ([300, 300], [12, 12], 512, 1, 2),
+    ([2560], [12], 9728, 0, 8), ([4096], [12], 11008, 0, 3), ([17], [12], 256, 0, 5),
+])
+def test_bmv_sixteen_waves(monkeypatch, rows, types, K, mode, M):
+    import sys
+
+    module = sys.modules[__name__]
+    monkeypatch.setattr(module, "WAVES", 16)
+    monkeypatch.setattr(module, "P", {12: 2, 14: 1})
+    check_indices(rows, types, K, mode, M, [0] * len(rows))
+
+
+@pytest.mark.parametrize("N,S", [(2560, 38), (3328, 10), (2561, 7), (3, 1), (40, 41)])
+def test_bmv_q6k_slots(N, S):
+    """Q6_K in mode 0: the tile's chunks (dword-aligned 16-byte loads, at most
+    three a lane) put every superblock of the share's rows into the wave's slot
+    whole, where ws_tile6 reads its 54 dwords; no load passes the matrix's last
+    dword except into the descriptor's zeros, no write passes the slot."""
+    CH, LOADS = 14, 3
+    count = min(CUS, N)
+    rows_max = -(-N // count)
+    assert rows_max <= 64 * LOADS // CH
+    rb, total = S * 210, N * S * 210
+    end4 = (total + 3) & ~3
+    per, rem = N // count, N % count
+    mat = np.zeros(end4 + 64, np.uint8)
+    mat[:total] = np.arange(total, dtype=np.int64) * 2654435761 % 251 + 1
+    for g in {0, rem, count - 1}:
+        r0, nrows = g * per + min(g, rem), per + (1 if g < rem else 0)
+        n = CH * nrows
+        c = np.minimum(np.arange(64 * LOADS), n - 1)
+        assert n <= 64 * LOADS and 16 * n <= 16 * CH * rows_max
+        for s in range(S):
+            off = (((r0 + c // CH) * rb + s * 210) & ~3) + 16 * (c % CH)
+            slot = np.zeros(16 * n, np.uint8)
+            for o, k in zip(off, c):
+                assert o % 4 == 0
+                slot[16 * k:16 * k + 16] = np.where(o + np.arange(16) < end4, mat[np.minimum(o + np.arange(16), end4)], 0)
+            for row in range(nrows):
+                first = (r0 + row) * rb + s * 210
+                o = 16 * CH * row + (first & 3)
+                assert (first & 3) in (0, 2) and 4 * 54 <= 16 * CH
+                assert np.array_equal(slot[o:o + 210], mat[first:first + 210])
