@@ -181,7 +181,7 @@ __device__ __forceinline__ void bmv_body(const BmvParams& p, const BmvShare& sh,
   auto stream = [&](auto mh) {
     constexpr int MH = decltype(mh)::value;
     if constexpr (kSlots) {
-      lds_u8* slot = (lds_u8*)(sums) + 16 * sh.ranges * 32 + wave * bmv_slot_bytes(p.rows_max);
+      lds_u8* slot = (lds_u8*)(sums) + groups_max * 16 * sh.ranges * 32 + wave * bmv_slot_bytes(p.rows_max);
       const int n = min(L.n, sh.nrows - 1);  // rows past the share redo its last one and are not stored
       const lds_u8* row = slot + bmv_slot_bytes(n);
       BmvCursor cc = start;
@@ -244,19 +244,34 @@ __device__ __forceinline__ void bmv_body(const BmvParams& p, const BmvShare& sh,
   }
 }
 
+// TYPE: the type of the matrix (mode 1: of gate and up), or 0 for a launch of
+// several matrices, where each workgroup takes its matrix's. (The other
+// launches read their two segments' arguments only: with all four read in
+// the prologue the FFN block at M = 8 took 0.8 us longer.)
 template <int TYPE, int MODE, bool Q8IN>
 __global__ __launch_bounds__(64 * kBmvWaves) void bmv_kernel(const BmvParams p) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < (TYPE == 0 ? kMaxSegments : MODE + 1); ++j)
     asm volatile("" ::"s"(p.seg[j].w), "s"(p.seg[j].y), "s"(p.seg[j].rows), "s"(p.seg[j].type),
                  "s"(p.seg[j].wg_begin), "s"(p.seg[j].per), "s"(p.seg[j].rem), "s"(p.seg[j].pad));
   asm volatile("" ::"s"(p.x), "s"(p.q8), "s"(p.h), "s"(p.hq), "s"(p.arrive), "s"(p.M), "s"(p.K), "s"(p.S),
-               "s"(p.stride), "s"(p.ranges), "s"(p.groups_max), "s"(p.rows_max));
+               "s"(p.stride), "s"(p.ranges), "s"(p.groups_max), "s"(p.rows_max), "s"(p.nseg));
   __builtin_amdgcn_sched_barrier(0);
-  const int g = static_cast<int>(blockIdx.x), per = p.seg[0].per, rem = p.seg[0].rem;
+  const int wg = static_cast<int>(blockIdx.x), nseg = TYPE == 0 ? p.nseg : 1;
+  const int j = (nseg > 1 && wg >= p.seg[1].wg_begin) + (nseg > 2 && wg >= p.seg[2].wg_begin) +
+                (nseg > 3 && wg >= p.seg[3].wg_begin);
+  auto pick = [j](auto f0, auto f1, auto f2, auto f3) {
+    if constexpr (TYPE != 0) return f0;
+    return j == 0 ? f0 : j == 1 ? f1 : j == 2 ? f2 : f3;
+  };
+  const int g = wg - pick(p.seg[0].wg_begin, p.seg[1].wg_begin, p.seg[2].wg_begin, p.seg[3].wg_begin);
+  const int per = pick(p.seg[0].per, p.seg[1].per, p.seg[2].per, p.seg[3].per);
+  const int rem = pick(p.seg[0].rem, p.seg[1].rem, p.seg[2].rem, p.seg[3].rem);
+  const int rows = pick(p.seg[0].rows, p.seg[1].rows, p.seg[2].rows, p.seg[3].rows);
+  float* const yout = pick(p.seg[0].y, p.seg[1].y, p.seg[2].y, p.seg[3].y);
   BmvShare sh;
-  sh.w[0] = p.seg[0].w;
+  sh.w[0] = pick(p.seg[0].w, p.seg[1].w, p.seg[2].w, p.seg[3].w);
   sh.w[1] = MODE == 1 ? p.seg[1].w : sh.w[0];
   sh.r0 = g * per + min(g, rem);
   sh.nrows = per + (g < rem ? 1 : 0);
@@ -267,18 +282,25 @@ __global__ __launch_bounds__(64 * kBmvWaves) void bmv_kernel(const BmvParams p) 
   sh.ranges = p.ranges;
   sh.run_q = p.S / p.ranges;
   sh.run_r = p.S - sh.run_q * p.ranges;
-  sh.row_bytes = p.S * (TYPE == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KBytes);
-  bmv_body<TYPE, MODE, Q8IN>(p, sh, p.seg[0].rows, p.seg[0].y, p.groups_max, lds_raw);
+  if (TYPE == QK_TYPE_Q4_K ||
+      (TYPE == 0 && pick(p.seg[0].type, p.seg[1].type, p.seg[2].type, p.seg[3].type) == QK_TYPE_Q4_K)) {
+    if constexpr (TYPE != QK_TYPE_Q6_K) {
+      sh.row_bytes = p.S * kQ4KBytes;
+      bmv_body<QK_TYPE_Q4_K, MODE, Q8IN>(p, sh, rows, yout, p.groups_max, lds_raw);
+    }
+  } else if constexpr (TYPE != QK_TYPE_Q4_K) {
+    sh.row_bytes = p.S * kQ6KBytes;
+    bmv_body<QK_TYPE_Q6_K, MODE, Q8IN>(p, sh, rows, yout, p.groups_max, lds_raw);
+  }
 }
 
 using BmvKernel = void (*)(BmvParams);
 
 BmvKernel bmv_kernel_for(int type, int mode, bool q8) {
-  if (type == QK_TYPE_Q4_K)
-    return mode == 1 ? &bmv_kernel<QK_TYPE_Q4_K, 1, false>
-                     : q8 ? &bmv_kernel<QK_TYPE_Q4_K, 0, true> : &bmv_kernel<QK_TYPE_Q4_K, 0, false>;
-  return mode == 1 ? &bmv_kernel<QK_TYPE_Q6_K, 1, false>
-                   : q8 ? &bmv_kernel<QK_TYPE_Q6_K, 0, true> : &bmv_kernel<QK_TYPE_Q6_K, 0, false>;
+  if (type == 0) return q8 || mode == 1 ? nullptr : &bmv_kernel<0, 0, false>;
+  if (mode == 1) return type == QK_TYPE_Q4_K ? &bmv_kernel<QK_TYPE_Q4_K, 1, false> : &bmv_kernel<QK_TYPE_Q6_K, 1, false>;
+  if (type == QK_TYPE_Q4_K) return q8 ? &bmv_kernel<QK_TYPE_Q4_K, 0, true> : &bmv_kernel<QK_TYPE_Q4_K, 0, false>;
+  return q8 ? &bmv_kernel<QK_TYPE_Q6_K, 0, true> : &bmv_kernel<QK_TYPE_Q6_K, 0, false>;
 }
 
 }  // namespace
@@ -294,20 +316,53 @@ int64_t bmv_wave_tiles(int64_t rows, int parts, int S, int ranges) {
   return per_wave * ((S + ranges - 1) / ranges);
 }
 
-// The workgroup count and run split of a launch (shared with the CPU index
-// model of the tests through the same rules). Returns false when the shape
-// does not fit this kernel's LDS plan.
-bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int& count, int& ranges, int& groups_max,
-              int& lds) {
-  const int parts = mode == 1 ? 2 : 1;
-  const int rows = p.seg[0].rows;
-  count = std::clamp(cus, 1, rows);
-  const int stride = p.K + 16;
-  const int rows_max = (rows + count - 1) / count;
+// The workgroups of each matrix and the run split of a launch (the CPU index
+// model of the tests restates these rules). One matrix, or gate and up, over
+// every CU; several matrices: at most kBmvMaxGroups row groups of 16 a
+// workgroup (Q6_K: one of at most kBmvSlotRows rows, through the slots), the
+// fewest that fit the CUs, what is left in proportion to the bytes. Returns
+// false when the shape does not fit.
+bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int (&count)[kMaxSegments], int& ranges,
+              int& groups_max, int& rows_max, int& lds) {
+  const int parts = mode == 1 ? 2 : 1, nseg = mode == 1 ? 1 : p.nseg;
+  bool slots = false;
+  if (nseg == 1) {
+    count[0] = std::clamp(cus, 1, p.seg[0].rows);
+    slots = mode == 0 && p.seg[0].type == QK_TYPE_Q6_K;
+  } else {
+    int sum = cus + 1;
+    for (int groups = 1; groups <= kBmvMaxGroups && sum > cus; ++groups) {
+      sum = 0;
+      for (int j = 0; j < nseg; ++j) {
+        const int rows = p.seg[j].type == QK_TYPE_Q6_K ? kBmvSlotRows : 16 * groups;
+        count[j] = p.seg[j].rows / rows + (p.seg[j].rows % rows != 0);
+        sum += count[j];
+      }
+    }
+    if (sum > cus) return false;
+    double bytes[kMaxSegments] = {0.0}, total = 0.0;
+    for (int j = 0; j < nseg; ++j) {
+      slots = slots || p.seg[j].type == QK_TYPE_Q6_K;
+      bytes[j] = static_cast<double>(p.seg[j].rows) * (p.seg[j].type == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KBytes);
+      total += bytes[j];
+    }
+    const int left = cus - sum;
+    for (int j = 0; j < nseg; ++j)
+      count[j] = std::min(p.seg[j].rows, count[j] + static_cast<int>(left * bytes[j] / total));
+  }
+  rows_max = 0;
+  int slot_rows = 0;
+  for (int j = 0; j < nseg; ++j) {
+    const int rows = p.seg[j].rows / count[j] + (p.seg[j].rows % count[j] != 0);
+    rows_max = std::max(rows_max, rows);
+    if (mode == 0 && p.seg[j].type == QK_TYPE_Q6_K) {
+      slot_rows = std::max(slot_rows, rows);
+      if (rows > kBmvSlotRows || static_cast<int64_t>(p.seg[j].rows) * p.S * kQ6KBytes + 16 > INT32_MAX) return false;
+    }
+  }
   groups_max = (rows_max + 15) / 16;
-  const bool slots = mode == 0 && p.seg[0].type == QK_TYPE_Q6_K;
-  if (slots && (rows_max > kBmvSlotRows || static_cast<int64_t>(rows) * p.S * kQ6KBytes + 16 > INT32_MAX)) return false;
-  const int slot_bytes = slots ? kBmvWaves * bmv_slot_bytes(rows_max) : 0;
+  if (slots) rows_max = slot_rows;  // (what the slots are sized by)
+  const int stride = p.K + 16, slot_bytes = slots ? kBmvWaves * bmv_slot_bytes(slot_rows) : 0;
   // runs per group: the fewest tiles on the busiest wave of any workgroup,
   // then the fewest units (each unit ends with a lane reduction)
   ranges = 0;
@@ -315,10 +370,12 @@ bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int& count,
   for (int r = 1; r <= p.S; ++r) {
     if (bmv_lds_bytes(p.K, stride, parts, groups_max, r) + slot_bytes > max_lds) break;
     int64_t tiles = 0, units = 0;
-    const int per = rows / count;
-    for (int n : {per, per + 1}) {
-      tiles = std::max(tiles, bmv_wave_tiles(n, parts, p.S, r));
-      units = std::max<int64_t>(units, (parts * ((n + 15) / 16) * r + kBmvWaves - 1) / kBmvWaves);
+    for (int j = 0; j < nseg; ++j) {
+      const int per = p.seg[j].rows / count[j];
+      for (int n : {per, per + 1}) {
+        tiles = std::max(tiles, bmv_wave_tiles(n, parts, p.S, r));
+        units = std::max<int64_t>(units, (parts * ((n + 15) / 16) * r + kBmvWaves - 1) / kBmvWaves);
+      }
     }
     const int64_t cost = 8 * tiles + units;
     if (cost < best) {
@@ -339,17 +396,23 @@ hipError_t launch_bmv(const MatvecParams& p, int mode, hipStream_t stream, bool&
   // streaming kernel before: ffn_down in fp32 Q4_K at M = 3 / 8 13.2 / 22.2 ->
   // 9.5 / 14.6, Q6_K 13.1 / 22.4 -> 12.2 / 17.9; at M = 2 it is the faster one
   // (9.2 against 9.5, 10.3 against 11.4).
-  if (p.M < (mode == 1 ? 2 : 3) || p.M > 8 || (mode != 0 && mode != 1)) return hipSuccess;
-  if (mode == 1 ? p.x == nullptr || p.nseg != 2 : p.nseg != 1) return hipSuccess;
+  // Several matrices (q/k/v): all-Q4_K at M = 3 / 5 / 8 8.3 / 11.5 / 11.8 -> 6.7 /
+  // 7.1 / 8.0, with a Q6_K v 7.4 / 10.9 / 11.3 -> 7.3 / 7.9 / 8.7 (at M = 2 the
+  // streaming kernel's 6.4 us are the faster ones there).
+  bool all_q4 = true;
+  for (int j = 0; j < p.nseg; ++j) all_q4 = all_q4 && p.seg[j].type == QK_TYPE_Q4_K;
+  const int least = mode == 1 || (p.nseg > 1 && all_q4) ? 2 : 3;
+  if (p.M < least || p.M > 8 || (mode != 0 && mode != 1)) return hipSuccess;
+  if (mode == 1 ? p.x == nullptr || p.nseg != 2 : p.nseg > 1 && p.x == nullptr) return hipSuccess;
   if (p.K > (INT32_MAX - 64) / 8) return hipSuccess;
   int cus = 0, max_lds = 0;
   hipError_t e = device_limits(cus, max_lds);
   if (e != hipSuccess) return e;
-  int count = 0, ranges = 0, groups_max = 0, lds = 0;
-  if (!bmv_plan(p, mode, cus, max_lds, count, ranges, groups_max, lds)) return hipSuccess;
-  if (mode == 0 && groups_max > 1) return hipSuccess;
+  int count[kMaxSegments] = {0}, ranges = 0, groups_max = 0, rows_max = 0, lds = 0;
+  if (!bmv_plan(p, mode, cus, max_lds, count, ranges, groups_max, rows_max, lds)) return hipSuccess;
+  if (mode == 0 && p.nseg == 1 && groups_max > 1) return hipSuccess;
   if (p.hq != nullptr) {  // Q8(h) in the launch: a quad per (block, activation row) of a share
-    const int64_t rows_max = (p.seg[0].rows + count - 1) / count;
+    const int64_t rows_max = (p.seg[0].rows + count[0] - 1) / count[0];
     const int64_t blocks = (rows_max + 30) / 32 + 1;  // blocks a run of rows_max rows can touch
     if (p.seg[0].rows % 32 != 0 || blocks > kBmvMaxCloseBlocks || 4 * blocks * p.M > 64 * kBmvWaves ||
         p.arrive == nullptr)
@@ -368,14 +431,21 @@ hipError_t launch_bmv(const MatvecParams& p, int mode, hipStream_t stream, bool&
   bp.stride = p.K + 16;
   bp.ranges = ranges;
   bp.groups_max = groups_max;
-  bp.rows_max = (p.seg[0].rows + count - 1) / count;
-  for (int j = 0; j < (mode == 1 ? 2 : 1); ++j)
-    bp.seg[j] = {p.seg[j].w, p.seg[j].y, p.seg[j].rows, p.seg[j].type, 0, p.seg[0].rows / count, p.seg[0].rows % count, 0};
-  const BmvKernel fn = bmv_kernel_for(p.seg[0].type, mode, p.x == nullptr);
+  bp.rows_max = rows_max;
+  bp.nseg = p.nseg;
+  int begin = 0;
+  for (int j = 0; j < p.nseg; ++j) {
+    const int c = mode == 1 ? count[0] : count[j];
+    bp.seg[j] = {p.seg[j].w, p.seg[j].y, p.seg[j].rows, p.seg[j].type, begin, p.seg[j].rows / c, p.seg[j].rows % c, 0};
+    if (mode == 0 || j == 0) begin += c;
+  }
+  const int type = mode == 0 && p.nseg > 1 ? 0 : p.seg[0].type;
+  const BmvKernel fn = bmv_kernel_for(type, mode, p.x == nullptr);
+  if (!fn) return hipSuccess;
   e = allow_lds(reinterpret_cast<const void*>(fn), lds);
   if (e != hipSuccess) return e;
-  note("bmv_kernel", count, p.seg[0].type, mode, ranges, groups_max, p.hq != nullptr);
-  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(count)), dim3(64 * kBmvWaves),
+  note("bmv_kernel", begin, type, mode, ranges, groups_max, p.hq != nullptr);
+  hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(begin)), dim3(64 * kBmvWaves),
                      static_cast<size_t>(lds), stream, bp);
   launched = true;
   return hipGetLastError();

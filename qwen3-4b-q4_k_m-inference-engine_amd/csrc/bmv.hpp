@@ -27,8 +27,8 @@
 // fp32 (Q4_K: d*sc*xs*dot - dmin*m*xs*sum(codes); Q6_K: d*sc*xs*(dot - 32
 // sum(codes)), src/cuda/matmul.cu:24-84).
 //
-// A workgroup (one per CU) owns a contiguous range of rows (mode 1: of gate
-// and of up); its rows are cut into groups of 16 and each group's superblock columns
+// A workgroup (one per CU) owns a contiguous range of rows of one matrix (mode
+// 1: of gate and of up); its rows are cut into groups of 16 and each group's superblock columns
 // into `ranges` runs. Work units (part, group, run) are dealt to the waves in
 // contiguous blocks; a wave streams its units' tiles (16 rows x one
 // superblock) through a ring of P register buffers, P tiles ahead, so
@@ -60,6 +60,7 @@ constexpr int kBmvSlotChunks = 14;  // 16-byte chunks that cover a superblock fr
 constexpr int kBmvSlotLoads = 3;    // chunks per lane and tile
 constexpr int kBmvSlotRows = 64 * kBmvSlotLoads / kBmvSlotChunks;  // rows of a workgroup at most: 13
 constexpr int kBmvSlotP = 1;        // tiles in flight per wave
+constexpr int kBmvMaxGroups = 2;    // row groups a workgroup in a launch of several matrices (q/k/v)
 // Q8 blocks of h one workgroup may complete (M activation rows each, a quad
 // per block row): the launcher checks blocks * M * 4 <= threads.
 constexpr int kBmvMaxCloseBlocks = 16;
@@ -74,9 +75,10 @@ struct BmvParams {
   int32_t stride;      // LDS bytes per activation row of codes (K + 16)
   int32_t ranges;      // superblock runs per row group
   int32_t groups_max;  // row groups of the largest workgroup share
-  int32_t rows_max;    // its rows
+  int32_t rows_max;    // rows of the largest share that goes through slots
   int32_t pad;
-  StreamSegment seg[2];  // the matrix; mode 1: gate and up
+  int32_t nseg, pad2;
+  StreamSegment seg[kMaxSegments];  // mode 0: the matrices; mode 1: gate and up
 };
 
 // LDS image (byte offsets; K a multiple of 256):

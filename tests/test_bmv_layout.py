@@ -618,3 +618,34 @@ def test_bmv_q6k_slots(N, S):
                 o = 16 * CH * row + (first & 3)
                 assert (first & 3) in (0, 2) and 4 * 54 <= 16 * CH
                 assert np.array_equal(slot[o:o + 210], mat[first:first + 210])
+
+
+def multi_plan(rows, types, cus=CUS):
+    """bmv_plan's workgroups per matrix of a launch of several."""
+    total = cus + 1
+    for groups in (1, 2):
+        need = [-(-r // (13 if t == 14 else 16 * groups)) for r, t in zip(rows, types)]
+        total = sum(need)
+        if total <= cus:
+            break
+    if total > cus:
+        return None
+    byt = [r * BYTES[t] for r, t in zip(rows, types)]
+    return [min(r, c + int((cus - total) * b / sum(byt))) for r, c, b in zip(rows, need, byt)]
+
+
+@pytest.mark.parametrize("rows,types", [
+    ([4096, 1024, 1024], [12, 12, 14]), ([4096, 1024, 1024], [12, 12, 12]), ([2048, 1024, 1024], [12, 12, 14]),
+    ([1700, 33, 1560, 17], [14, 12, 14, 12]), ([8160, 32], [12, 12]), ([1, 1, 1], [14, 12, 14]),
+])
+def test_bmv_several_matrices_plan(rows, types):
+    """Every matrix's rows are cut among its workgroups without a gap, no
+    workgroup has more rows than its form takes, the grid fits the CUs."""
+    count = multi_plan(rows, types)
+    assert count is not None and sum(count) <= CUS
+    for r, t, c in zip(rows, types, count):
+        shares = [r // c + (1 if g < r % c else 0) for g in range(c)]
+        assert sum(shares) == r and min(shares) >= 1
+        assert max(shares) <= (13 if t == 14 else 32)
+    assert multi_plan([1700, 33, 1700, 17], [14, 12, 14, 12]) is None
+    assert multi_plan([8160, 33], [12, 12]) is None

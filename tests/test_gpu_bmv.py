@@ -44,3 +44,34 @@ def test_one_wide_matrix(gpu, oracle, qtype, K, N, M, takes):
         gpu.synchronize()
         assert gpu.last_launch().startswith("bmv_kernel")
         assert np.array_equal(y.download(np.float32)[:M * N].reshape(M, N), got)
+
+
+@pytest.mark.parametrize("K,shapes,M,takes", [
+    (2560, [(Q4, 4096), (Q4, 1024), (Q6, 1024)], 3, True),   # q, k and v of both types
+    (2560, [(Q4, 4096), (Q4, 1024), (Q6, 1024)], 8, True),
+    (2560, [(Q4, 4096), (Q4, 1024), (Q4, 1024)], 2, True),   # all Q4_K: from M = 2
+    (2560, [(Q4, 4096), (Q4, 1024), (Q4, 1024)], 7, True),
+    (2560, [(Q4, 4096), (Q4, 1024), (Q6, 1024)], 2, False),
+    (2560, [(Q6, 1700), (Q4, 33), (Q6, 1560), (Q4, 17)], 5, True),   # 13 rows of Q6_K a workgroup
+    (2560, [(Q6, 1700), (Q4, 33), (Q6, 1700), (Q4, 17)], 5, False),  # past the CUs
+    (1024, [(Q4, 8160), (Q4, 32)], 4, True),                 # 256 workgroups of 32 rows
+    (1024, [(Q4, 8160), (Q4, 33)], 4, False),
+])
+def test_several_matrices(gpu, oracle, K, shapes, M, takes):
+    """One launch of 2..4 matrices on fp32 activations against the oracle's
+    products, at the row counts where its plan ends (256 CUs)."""
+    hosts = [oracle.synth_superblocks(q, N, K, SEED + 7 * i + N, 0.01, 0.01) for i, (q, N) in enumerate(shapes)]
+    ws = [gpu.DeviceBuffer.from_array(h) for h in hosts]
+    x = oracle.synth_normal(M * K, SEED + 60 + M)
+    xd = gpu.DeviceBuffer.from_array(x)
+    ys = [gpu.DeviceBuffer.from_array(np.full(M * N + 1, 123.0, np.float32)) for _, N in shapes]
+    gpu.matmul_segments(xd, M, K, [(w, q, N, y) for w, (q, N), y in zip(ws, shapes, ys)])
+    gpu.synchronize()
+    launch = gpu.last_launch()
+    print(f"[case] K={K} {shapes} M={M} launch {launch}", flush=True)
+    assert launch.startswith("bmv_kernel") == takes
+    for h, (q, N), y in zip(hosts, shapes, ys):
+        out = y.download(np.float32)
+        assert out[-1] == 123.0
+        ref = oracle.reference_product(x, h, q, K, N).reshape(M, N)
+        assert oracle.row_norm_error(out[:-1].reshape(M, N), ref) <= 1e-5
