@@ -117,29 +117,48 @@ __device__ __forceinline__ Q8Quarter quantize_quarter(const float (&v)[8]) {
   amax = fmaxf(amax, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
                          0, __builtin_bit_cast(int, amax), 0x4E, 0xF, 0xF, false)));
   const bool usual = amax >= 0x1p-64f && amax <= 0x1p64f;
-  int code[8];
-  float scale;
-  if (usual) {
-    const float r = refined_rcp(amax);
+  const float r = refined_rcp(amax);
+  float scale = markstein_div(amax, 127.0f, 1.0f / 127.0f);
+  // x * (127 r) is within 2^-15 of the reference's RN(RN(x / amax) * 127) (two
+  // roundings each of at most 127 * 2^-24 either side), so where it is more
+  // than 2^-14 away from a half its nearest integer is the code. Added to
+  // 1.5 * 2^23 that integer is the result's low byte: about five VALU a value,
+  // and the exact form below only in the lanes of a group with a near tie
+  // (about one wave in 16 on smooth data), a NaN or an unusual amax.
+  constexpr float kMagic = 12582912.0f;
+  const float r127 = 127.0f * r;
+  uint32_t bits[8];
+  float worst = 0.0f, total = 0.0f;  // (total: the codes' sum, or NaN)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) code[i] = q8_code(v[i], amax, r);
-    scale = markstein_div(amax, 127.0f, 1.0f / 127.0f);
-  } else if (amax == 0.0f) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) code[i] = 0;
-    scale = 0.0f;
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) code[i] = static_cast<int>(roundf((v[i] / amax) * 127.0f));
-    scale = amax / 127.0f;
+  for (int i = 0; i < 8; ++i) {
+    const float y = __builtin_fmaf(v[i], r127, kMagic), code = y - kMagic;
+    worst = fmaxf(worst, fabsf(__builtin_fmaf(v[i], r127, -code)));
+    total += code;
+    bits[i] = __builtin_bit_cast(uint32_t, y);
   }
-  uint32_t lo = 0, hi = 0;
-  int sum = 0;
+  auto pack = [](uint32_t a, uint32_t b, uint32_t c, uint32_t d) {  // their low bytes
+    return __builtin_amdgcn_perm(__builtin_amdgcn_perm(d, c, 0x0C0C0400u), __builtin_amdgcn_perm(b, a, 0x0C0C0400u),
+                                 0x05040100u);
+  };
+  uint32_t lo = pack(bits[0], bits[1], bits[2], bits[3]), hi = pack(bits[4], bits[5], bits[6], bits[7]);
+  int sum = static_cast<int>(total);
+  if (!(usual && worst < 0.5f - 0x1p-14f && total == total)) {
+    int code[8];
+    if (usual) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    lo |= (static_cast<uint32_t>(code[i]) & 0xFFu) << (8 * i);
-    hi |= (static_cast<uint32_t>(code[i + 4]) & 0xFFu) << (8 * i);
-    sum += code[i] + code[i + 4];
+      for (int i = 0; i < 8; ++i) code[i] = q8_code(v[i], amax, r);
+    } else if (amax == 0.0f) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) code[i] = 0;
+      scale = 0.0f;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) code[i] = static_cast<int>(roundf((v[i] / amax) * 127.0f));
+      scale = amax / 127.0f;
+    }
+    lo = pack(code[0], code[1], code[2], code[3]);
+    hi = pack(code[4], code[5], code[6], code[7]);
+    sum = dot4(lo, 0x01010101u, dot4(hi, 0x01010101u, 0));
   }
   // lanes 0,1 of the quad hold codes 0..15, lanes 2,3 codes 16..31
   const int pair = sum + __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, false);
