@@ -97,16 +97,14 @@ hipError_t launch_bmv_ws(const MatvecParams& p, int mode, hipStream_t stream, bo
   bp.stride = p.K + 16;
   bp.reg = plan.reg;
   bp.act = bmv_ws_act_bytes(p.K);
-  bool q4 = false, q6 = false;
   int begin = 0;
   for (int j = 0; j < nseg; ++j) {
     bp.seg[j] = {p.seg[j].w, p.seg[j].y, p.seg[j].rows, p.seg[j].type, begin,
                  p.seg[j].rows / plan.count[j], p.seg[j].rows % plan.count[j], 0};
-    (p.seg[j].type == QK_TYPE_Q4_K ? q4 : q6) = true;
     begin += plan.count[j];
   }
   if (mode == 1) bp.seg[1] = {p.seg[1].w, nullptr, p.seg[1].rows, p.seg[1].type, 0, 0, 0, 0};
-  const int type = q4 && q6 ? 0 : q4 ? QK_TYPE_Q4_K : QK_TYPE_Q6_K;
+  const int type = nseg > 1 ? 0 : p.seg[0].type;
   const BmvWsKernel fn = bmv_ws_kernel_for(type, mode, q8in);
   if (!fn) return hipSuccess;
   e = allow_lds(reinterpret_cast<const void*>(fn), plan.lds);
