@@ -58,8 +58,13 @@ constexpr int kPrepGroups = 8;  // groups of 8 activations held per thread: K <=
 
 // One workgroup per activation row: the row's max |x| (for the power-of-two
 // scale), then the Q8 round trip of every 32-value block. Rows up to 16384
-// values stay in registers between the two steps; wider rows are read twice.
-// K % 32 == 0, so the 4 lanes of a quad are always in or out together.
+// values stay in registers between the two steps (G groups of 8 per thread,
+// the least that holds the row: a launch over few rows is all latency, and
+// rounds that no thread takes part in still cost their branches: 1024 x 2560 at
+// M = 200 19.0 -> 18.5 us with its GEMM, 9728 x 2560 at M = 23 19.4 -> 18.4, the
+// quantiser's nearest-integer form included); wider rows (G = 0) are read twice. K % 32 == 0, so the 4 lanes of a quad are always in or
+// out together.
+template <int G>
 __global__ __launch_bounds__(256) void prep_rows_kernel(const float* __restrict__ x,
                                                         _Float16* __restrict__ hi,
                                                         _Float16* __restrict__ lo,
@@ -70,18 +75,17 @@ __global__ __launch_bounds__(256) void prep_rows_kernel(const float* __restrict_
   const float* xr = x + row * K;
   const int tid = static_cast<int>(threadIdx.x);
   const int groups = K / 8;
-  const bool resident = groups <= 256 * kPrepGroups;
-  f32x4 va[kPrepGroups], vb[kPrepGroups];
+  f32x4 va[G > 0 ? G : 1], vb[G > 0 ? G : 1];
   float amax = 0.0f;
-  if (resident) {
+  if constexpr (G > 0) {
 #pragma unroll
-    for (int i = 0; i < kPrepGroups; ++i) {
-      const int g = tid + 256 * i;
-      va[i] = vb[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (g < groups) {
-        va[i] = *reinterpret_cast<const f32x4_a4*>(xr + 8 * g);
-        vb[i] = *reinterpret_cast<const f32x4_a4*>(xr + 8 * g + 4);
-      }
+    for (int i = 0; i < G; ++i) {  // loads past the row re-read its last group
+      const int g = min(tid + 256 * i, groups - 1);
+      va[i] = *reinterpret_cast<const f32x4_a4*>(xr + 8 * g);
+      vb[i] = *reinterpret_cast<const f32x4_a4*>(xr + 8 * g + 4);
+    }
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
       const f32x4 m4 = f32x4{fmaxf(fabsf(va[i].x), fabsf(vb[i].x)), fmaxf(fabsf(va[i].y), fabsf(vb[i].y)),
                              fmaxf(fabsf(va[i].z), fabsf(vb[i].z)), fmaxf(fabsf(va[i].w), fabsf(vb[i].w))};
       amax = fmaxf(amax, fmaxf(fmaxf(m4.x, m4.y), fmaxf(m4.z, m4.w)));
@@ -92,7 +96,7 @@ __global__ __launch_bounds__(256) void prep_rows_kernel(const float* __restrict_
       amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
     }
   }
-  for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+  amax = wave_max(amax);
   if ((tid & 63) == 0) partial[tid >> 6] = amax;
   __syncthreads();
   amax = fmaxf(fmaxf(partial[0], partial[1]), fmaxf(partial[2], partial[3]));
@@ -100,9 +104,9 @@ __global__ __launch_bounds__(256) void prep_rows_kernel(const float* __restrict_
   const float up = ldexpf(1.0f, s);
   if (tid == 0) row_scale[row] = ldexpf(1.0f, -s);
 
-  if (resident) {
+  if constexpr (G > 0) {
 #pragma unroll
-    for (int i = 0; i < kPrepGroups; ++i) {
+    for (int i = 0; i < G; ++i) {
       const int g = tid + 256 * i;
       if (g < groups)
         prep_group(va[i], vb[i], up, hi, lo, row * K + 8 * g, xs, xsum_index(row, g >> 2, K / 256),
@@ -153,8 +157,14 @@ hipError_t launch_gemm_prep(const float* x, int64_t M, int64_t K, void* workspac
                             hipStream_t stream, bool skip) {
   if (skip) return hipSuccess;  // every GEMM of the call forms its planes itself
   const WorkspaceLayout ws = layout(workspace, M, K);
-  prep_rows_kernel<<<static_cast<uint32_t>(M), 256, 0, stream>>>(x, ws.hi, ws.lo, ws.row_scale,
-                                                                  ws.xs, static_cast<int>(K));
+  const int64_t rounds = (K / 8 + 255) / 256;
+  const auto kernel = rounds <= 1   ? &prep_rows_kernel<1>
+                      : rounds <= 2 ? &prep_rows_kernel<2>
+                      : rounds <= 5 ? &prep_rows_kernel<5>
+                      : rounds <= kPrepGroups ? &prep_rows_kernel<kPrepGroups>
+                                              : &prep_rows_kernel<0>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(M)), dim3(256), 0, stream, x, ws.hi, ws.lo, ws.row_scale, ws.xs,
+                     static_cast<int>(K));
   return hipGetLastError();
 }
 

@@ -35,21 +35,33 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t&
 
 // One lane's 8 values of a 32-value block with maximum |x| = bmax: the codes
 // and scale as the reference computes them in float (for bmax in [2^-64,
-// 2^64] through the exact reciprocal and Markstein quotient of the mat-vec
-// quantiser, equal to IEEE division), v = (code * scale) * up split into fp16
-// pairs h / l, and the sum of the 8 v in order.
+// 2^64] the nearest integer of x * (127 / bmax) where that is not near a half,
+// else through the exact reciprocal and Markstein quotient, both equal to IEEE
+// division: see the mat-vec quantiser), v = (code * scale) * up split into
+// fp16 pairs h / l, and the sum of the 8 v in order.
 __device__ __forceinline__ void q8_scaled_planes(const float (&v)[8], float bmax, float up, uint32_t (&h)[4],
                                                  uint32_t (&l)[4], float& sum) {
-  float code[8], scale;
-  if (bmax >= 0x1p-64f && bmax <= 0x1p64f) {
-    const float r = refined_rcp(bmax);
+  float code[8];
+  float scale = markstein_div(bmax, 127.0f, 1.0f / 127.0f);
+  const float r = refined_rcp(bmax), r127 = 127.0f * r;
+  constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
+  float worst = 0.0f, total = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) code[i] = static_cast<float>(q8_code(v[i], bmax, r));
-    scale = markstein_div(bmax, 127.0f, 1.0f / 127.0f);
-  } else {
+  for (int i = 0; i < 8; ++i) {
+    code[i] = __builtin_fmaf(v[i], r127, kMagic) - kMagic;
+    worst = fmaxf(worst, fabsf(__builtin_fmaf(v[i], r127, -code[i])));
+    total += code[i];
+  }
+  const bool usual = bmax >= 0x1p-64f && bmax <= 0x1p64f;
+  if (!(usual && worst < 0.5f - 0x1p-14f && total == total)) {  // a near tie, a NaN, an unusual bmax
+    if (usual) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) code[i] = bmax == 0.0f ? 0.0f : roundf((v[i] / bmax) * 127.0f);
-    scale = bmax / 127.0f;
+      for (int i = 0; i < 8; ++i) code[i] = static_cast<float>(q8_code(v[i], bmax, r));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) code[i] = bmax == 0.0f ? 0.0f : roundf((v[i] / bmax) * 127.0f);
+      scale = bmax / 127.0f;
+    }
   }
   sum = 0.0f;
 #pragma unroll

@@ -125,6 +125,24 @@ __device__ __forceinline__ float row_lanes_sum(float v) {
   return v;
 }
 
+// Maximum over the wave (of values >= 0), in every lane: the same exchanges.
+template <int CTRL>
+__device__ __forceinline__ float max_dpp(float v) {
+  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF,
+                                                                       false)));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  v = max_dpp<0x140>(max_dpp<0x141>(max_dpp<0x4E>(max_dpp<0xB1>(v))));
+  const auto t = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v),
+                                                  __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned a = t[0], b = t[1];
+  v = fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+  const auto u = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v),
+                                                  __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned c = u[0], d = u[1];
+  return fmaxf(__builtin_bit_cast(float, c), __builtin_bit_cast(float, d));
+}
+
 // Sum over the 8 lanes of each aligned lane octet (quad swaps, then the
 // half-row mirror); every lane of the octet receives the sum.
 __device__ __forceinline__ float octet_sum(float v) {
