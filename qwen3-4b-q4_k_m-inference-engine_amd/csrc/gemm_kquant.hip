@@ -914,34 +914,46 @@ KQPlan rule_plan(int type, int64_t M, int64_t N, int64_t K) {
 // another (a CU with several resident takes as long as with one at a time:
 // 2.2-2.5 us per superblock of a 64-row Q4_K tile whether 1, 2 or 3 are
 // resident, a lone unit up to a third more), then the reduce of the splits (a
-// launch, and the partial products once through memory).
+// launch, and the partial products once through memory). At M <= 32, where a
+// unit has a few superblocks, its start counts too, and a lone unit hides
+// none of it.
 double plan_cost(int type, bool wide, int64_t tiles, int64_t splits, int64_t M, int64_t N, int64_t S) {
-  const bool q6 = type == QK_TYPE_Q6_K;
+  const bool q6 = type == QK_TYPE_Q6_K, short_m = M <= 32;
   const double superblock_ns = q6 ? (wide ? 3400.0 : 2400.0) : wide ? 2350.0 : 1500.0;
   const int64_t units = (tiles * splits + kPlanCUs - 1) / kPlanCUs;  // of the busiest CU
-  const double gemm = superblock_ns * static_cast<double>(units) * static_cast<double>((S + splits - 1) / splits);
+  const double unit = superblock_ns * static_cast<double>((S + splits - 1) / splits) + (short_m ? 1500.0 : 0.0);
   const double reduce = 3500.0 + 1e-3 * static_cast<double>(splits) * static_cast<double>(M) * static_cast<double>(N);
-  return gemm * (units == 1 ? 1.3 : 1.0) + (splits > 1 ? reduce : 0.0);
+  return unit * static_cast<double>(units) * (units > 1 ? 1.0 : short_m ? 1.5 : 1.3) + (splits > 1 ? reduce : 0.0);
 }
 
-// The rules above hold for K < 4096 at M > 64 and for M <= 32. For deep K, and
-// for the few tiles of M = 33..64, they leave up to half of the time on CUs
-// that wait for the busiest one; there the plan is the tile height and split
-// of least estimated time. Measured against the rules (us, prep and reduce
-// included; 22 shapes timed under every plan, the chosen one 1.13 times as fast
-// as the rules' on average and never more than 1% behind it): 2560 x 9728 Q6_K at M = 48 / 100 / 200 /
-// 350 / 800 37.4 / 63.3 / 78.8 / 112.6 / 256 -> 33.6 / 41.4 / 62.7 / 88.6 /
+// The rules above hold for K < 4096 at M > 64. For deep K, and for the few
+// tiles of M <= 64, they leave up to half of the time on CUs that wait for the
+// busiest one; there the plan is the tile height and split of least estimated
+// time. Measured against the rules (us, prep and reduce included; 22 shapes
+// timed under every plan, the chosen one 1.13 times as fast as the rules' on
+// average and never more than 1% behind it): 2560 x 9728 Q6_K at M = 48 / 100 /
+// 200 / 350 / 800 37.4 / 63.3 / 78.8 / 112.6 / 256 -> 33.6 / 41.4 / 62.7 / 88.6 /
 // 219, Q4_K at M = 100 / 512 38.9 / 97.9 -> 31.7 / 78.7, 1024 x 2560 Q6_K at
 // M = 48 21.0 -> 14.6. (At smaller K and larger M finer splits gain less, and
-// a row's sums are the same there at every M.)
+// a row's sums are the same there at every M.) At M <= 32 the rule's split is
+// the most: its units are one to three a CU, and a few over two a CU cost a
+// round (2560 x 9728 at M = 23, 26 -> 19 splits: Q6_K 27.1 -> 23.7, Q4_K 19.9 ->
+// 18.2; 9728 x 2560, 7 -> 5: Q4_K 18.2 -> 16.5, Q6_K 22.7 -> 20.8).
 constexpr int64_t kPlanSplits = 6;
 
 KQPlan plan(int type, int64_t M, int64_t N, int64_t K) {
   const KQPlan rule = rule_plan(type, M, N, K);
   const int64_t S = K / 256;
-  if (M <= 32 || M > 65535 || (M > 64 && S < 16)) return rule;
+  if (M > 65535 || (M > 64 && S < 16)) return rule;
   const int64_t n_tiles = (N + 127) / 128;
   const int64_t tiles32 = ((M + 31) / 32) * n_tiles, tiles64 = ((M + 63) / 64) * n_tiles;
+  if (M <= 32) {
+    KQPlan best = rule;
+    for (int64_t splits = rule.splits - 1; splits >= 1; --splits)
+      if (plan_cost(type, false, tiles32, splits, M, N, S) < plan_cost(type, false, tiles32, best.splits, M, N, S))
+        best.splits = static_cast<int>(splits);
+    return best;
+  }
   // Splits of at least 4 superblocks (2 at M <= 64), no fewer than the rule's
   // (longer fp32 sums), that keep the workspace within the scratch of
   // qk_matmul_noalloc where the rule's plan is within it.
