@@ -99,7 +99,7 @@ int matvec_rows_per_launch(int64_t K) {
 
 hipError_t launch_matvec(MatvecParams p, int mode, hipStream_t stream) {
   // M = 2..8: the whole-share batched mat-vec on the matrix cores
-  // (bmv_ws.hip), else (gate/up) the batched mat-vec (bmv.hip).
+  // (bmv_ws.hip), else (gate/up, q/k/v, ffn_down) the batched mat-vec (bmv.hip).
   bool launched = false;
   hipError_t e = launch_bmv_ws(p, mode, stream, launched);
   if (e != hipSuccess || launched) return e;
