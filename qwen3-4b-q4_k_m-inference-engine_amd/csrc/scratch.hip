@@ -92,8 +92,8 @@ hipError_t Scratch::get(size_t bytes, void*& ptr) {
         return hipSuccess;
       }
     }
-    if (i >= 0) errors.drop();
   }
+  errors.drop();
   const hipError_t error = hipMallocAsync(&ptr_, bytes, stream_);
   if (error != hipSuccess) ptr_ = nullptr;
   ptr = ptr_;
@@ -108,7 +108,9 @@ Scratch::~Scratch() {
   }
   std::lock_guard<std::mutex> lock(g_mutex);
   Block& b = g_blocks[device_][block_];
+  const OwnErrors errors;
   if (hipEventRecord(b.event, stream_) != hipSuccess) {  // not orderable: give it back instead
+    errors.drop();
     (void)hipFreeAsync(b.ptr, stream_);
     b.ptr = nullptr;
     b.bytes = 0;
