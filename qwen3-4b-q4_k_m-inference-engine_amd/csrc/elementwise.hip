@@ -29,9 +29,12 @@ __global__ __launch_bounds__(256) void silu_multiply_kernel(const float* __restr
   }
 }
 
-// The sum of the workgroup's four waves' `sum`, in every thread.
+// The sum of the workgroup's four waves' `sum`, in every thread. Lane bits
+// 5, 4, .. 0 in turn (row rotations stand for the exchanges of bits 3 to 0:
+// lanes that differ only in bits already added hold the same sum).
 __device__ __forceinline__ float workgroup_sum(float sum, float (&partial)[4]) {
-  sum = row_lanes_sum<64>(sum);
+  sum = swap16_sum(swap32_sum(sum));
+  sum = add_dpp<0x121>(add_dpp<0x122>(add_dpp<0x124>(add_dpp<0x128>(sum))));
   if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = sum;
   __syncthreads();
   return (partial[0] + partial[1]) + (partial[2] + partial[3]);
@@ -39,12 +42,14 @@ __device__ __forceinline__ float workgroup_sum(float sum, float (&partial)[4]) {
 
 // out = x * rsqrt(mean(x^2) + eps) * scale for one row per workgroup (the
 // mat-vec's RMSNorm fold does the same inside its prologue at M = 1). A few
-// rows are bound by latency alone, so a row of at most 1024 Q values stays in
-// registers: its Q 16-byte loads per thread and those of the scale are all
-// issued at entry, and the row is read once: 8 rows of 2560 in 4.8 us against
-// 7.3 with one value per lane and load, the row read twice (rocprof, in a
-// graph; a launch's own cost there is about 2).
-template <int Q>
+// rows are bound by latency alone, so a row of at most 256 R values stays in
+// registers: its loads and those of the scale are all issued at entry, and
+// the row is read once: 8 / 2047 rows of 2560 in 2.30 / 6.64 us against 3.98 /
+// 10.09 with the row read twice (a launch of 40 in a graph). Thread t adds
+// values t, t + 256, .. in order, as the form below does: the sum's last bit
+// reaches Q8 codes near a tie, so every width keeps one order of its sums
+// (four neighbours a thread and load: 2.15 / 6.63 us, and other codes).
+template <int R>
 __global__ __launch_bounds__(256) void rms_norm_row_kernel(const float* __restrict__ x,
                                                            const float* __restrict__ scale,
                                                            float* __restrict__ out, int width,
@@ -52,29 +57,26 @@ __global__ __launch_bounds__(256) void rms_norm_row_kernel(const float* __restri
   __shared__ float partial[4];
   const int64_t row = static_cast<int64_t>(blockIdx.x) * width;
   const int tid = static_cast<int>(threadIdx.x);
-  const int quads = width / 4;
-  f32x4 v[Q], s[Q];
+  float v[R], s[R];
 #pragma unroll
-  for (int i = 0; i < Q; ++i) {  // loads past the row re-read its last quad
-    const int at = 4 * min(tid + 256 * i, quads - 1);
-    v[i] = *reinterpret_cast<const f32x4_a4*>(x + row + at);
-    s[i] = *reinterpret_cast<const f32x4_a4*>(scale + at);
+  for (int i = 0; i < R; ++i) {  // loads past the row re-read its last value
+    const int at = min(tid + 256 * i, width - 1);
+    v[i] = x[row + at];
+    s[i] = scale[at];
   }
   float sum = 0.0f;
 #pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    const float t = (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
-    sum += tid + 256 * i < quads ? t : 0.0f;
+  for (int i = 0; i < R; ++i) {
+    const float t = tid + 256 * i < width ? v[i] : 0.0f;
+    sum = __builtin_fmaf(t, t, sum);
   }
   const float inv = rsqrtf(workgroup_sum(sum, partial) / static_cast<float>(width) + eps);
 #pragma unroll
-  for (int i = 0; i < Q; ++i)
-    if (tid + 256 * i < quads)
-      *reinterpret_cast<f32x4_a4*>(out + row + 4 * (tid + 256 * i)) =
-          f32x4{(v[i].x * inv) * s[i].x, (v[i].y * inv) * s[i].y, (v[i].z * inv) * s[i].z, (v[i].w * inv) * s[i].w};
+  for (int i = 0; i < R; ++i)
+    if (tid + 256 * i < width) out[row + tid + 256 * i] = (v[i] * inv) * s[i];
 }
 
-// Any other width: two passes over the row.
+// Wider rows: two passes over the row.
 __global__ __launch_bounds__(256) void rms_norm_kernel(const float* __restrict__ x,
                                                        const float* __restrict__ scale,
                                                        float* __restrict__ out, int width,
@@ -84,7 +86,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const float* __restrict__
   float* o = out + static_cast<int64_t>(blockIdx.x) * width;
   const int tid = static_cast<int>(threadIdx.x);
   float sum = 0.0f;
-  for (int i = tid; i < width; i += 256) sum += xr[i] * xr[i];
+  for (int i = tid; i < width; i += 256) sum = __builtin_fmaf(xr[i], xr[i], sum);
   const float inv = rsqrtf(workgroup_sum(sum, partial) / static_cast<float>(width) + eps);
   for (int i = tid; i < width; i += 256) o[i] = (xr[i] * inv) * scale[i];
 }
@@ -120,19 +122,19 @@ hipError_t launch_rms_norm(const float* x, const float* scale, float* out, int64
                            int64_t width, float eps, hipStream_t stream) {
   const dim3 grid(static_cast<uint32_t>(rows));
   const int w = static_cast<int>(width);
-  // Whole quads up to 8192 values take the one-pass form (Q rounds of 1024).
-  if (w % 4 != 0 || w > 8192)
-    rms_norm_kernel<<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
-  else if (w <= 1024)
-    rms_norm_row_kernel<1><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
-  else if (w <= 2048)
-    rms_norm_row_kernel<2><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
-  else if (w <= 3072)
-    rms_norm_row_kernel<3><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
-  else if (w <= 4096)
+  // Up to 8192 values the one-pass form, in the least of these rounds.
+  if (w <= 1024)
     rms_norm_row_kernel<4><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
-  else
+  else if (w <= 2048)
     rms_norm_row_kernel<8><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
+  else if (w <= 2560)
+    rms_norm_row_kernel<10><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
+  else if (w <= 4096)
+    rms_norm_row_kernel<16><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
+  else if (w <= 8192)
+    rms_norm_row_kernel<32><<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
+  else
+    rms_norm_kernel<<<grid, 256, 0, stream>>>(x, scale, out, w, eps);
   return hipGetLastError();
 }
 

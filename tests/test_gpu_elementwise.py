@@ -1,7 +1,7 @@
 """RMSNorm, residual_add and silu_multiply on the device against float64, at
 the widths and counts where the 16-byte forms change (one value short of, at
 and past whole quads, register rounds and workgroups), from pointers that are
-only float-aligned, and in place."""
+only float-aligned, and in place; RMSNorm's sums in one order at every width."""
 from __future__ import annotations
 
 import numpy as np
@@ -44,6 +44,31 @@ def test_rms_norm(gpu, width, rows):
     assert np.all(np.abs(got - want) <= bound * np.abs(want))
     gpu.rms_norm(px, ps, px, rows, width, 1e-6)  # in place
     assert np.array_equal(_get(gpu, bx, x.size).reshape(rows, width), got)
+
+
+@pytest.mark.parametrize("width", [1, 255, 1000, 1024, 2048, 2560, 2562, 4096, 8192])
+def test_rms_norm_sums_in_one_order_at_every_width(gpu, width):
+    """A row and the same row padded with zeros to 4^k times its width, past
+    the one-pass form: the sum is the same if its order is, the mean, eps and
+    1 / root scale by powers of two, so the outputs differ by 2^k exactly."""
+    rng = np.random.default_rng(width)
+    rows, eps = 64, 2.0 ** -20
+    k = 1
+    while width * 4 ** k <= 8192:
+        k += 1
+    wide = width * 4 ** k
+    x = rng.standard_normal((rows, width)).astype(np.float32)
+    scale = rng.standard_normal(width).astype(np.float32)
+    xw, sw = np.zeros((rows, wide), np.float32), np.zeros(wide, np.float32)
+    xw[:, :width], sw[:width] = x, scale
+    got = []
+    for xi, si, w, e in ((x, scale, width, eps), (xw, sw, wide, eps / 4 ** k)):
+        bx, px = _put(gpu, xi)
+        bs, ps = _put(gpu, si)
+        bo, po = _put(gpu, np.zeros_like(xi))
+        gpu.rms_norm(px, ps, po, rows, w, e)
+        got.append(_get(gpu, bo, xi.size).reshape(rows, w)[:, :width])
+    assert np.array_equal(got[0] * 2 ** k, got[1])
 
 
 @pytest.mark.parametrize("count", [1, 3, 4, 1023, 1024, 1027, 20480, 1024 * 16384 + 5])
