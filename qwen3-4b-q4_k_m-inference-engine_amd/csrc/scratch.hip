@@ -33,6 +33,17 @@ struct OwnErrors {
   }
 };
 
+// hipEventQuery, allowed while another stream is being captured: in any
+// capture mode but the relaxed one a query ends that capture with an error,
+// whichever event it asks about.
+hipError_t query(hipEvent_t event) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  const hipError_t status = hipEventQuery(event);
+  if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return status;
+}
+
 // An idle block for `stream`: its own of the right size or any of its own,
 // an unused one, one whose work is done; else -1. Called with the lock held.
 int choose(Block (&blocks)[kScratchBlocks], hipStream_t stream, size_t bytes) {
@@ -51,7 +62,7 @@ int choose(Block (&blocks)[kScratchBlocks], hipStream_t stream, size_t bytes) {
   if (unused >= 0) return unused;
   const OwnErrors errors;
   for (int i = 0; i < kScratchBlocks; ++i)
-    if (!blocks[i].busy && hipEventQuery(blocks[i].event) == hipSuccess) return i;
+    if (!blocks[i].busy && query(blocks[i].event) == hipSuccess) return i;
   errors.drop();  // "not ready"
   return -1;
 }

@@ -103,3 +103,46 @@ def test_capture_between_cached_calls(gpu, oracle):
         b.check()
     graph.destroy()
     stream.destroy()
+
+
+@pytest.mark.parametrize("others", [0, 8])
+def test_calls_while_another_stream_is_captured(gpu, oracle, others):
+    """Calls on other streams, from this thread and another, neither end nor
+    enter a capture, with no block allocated yet and with every block last
+    used by a further stream."""
+    gpu.release_scratch()
+    cases = [Case(gpu, oracle, Q4, 2560, 256, 33 + i, 20261501 + i) for i in range(3)]
+    used = [gpu.Stream() for _ in range(others)]
+    for s in used:
+        cases[0].run(s.ptr)
+    gpu.synchronize()
+    streams = [gpu.Stream() for _ in cases]
+    errors = []
+
+    def eager(i):
+        try:
+            cases[i].run(streams[i].ptr)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    def record():
+        cases[0].run(streams[0].ptr)
+        thread = threading.Thread(target=eager, args=(1,))
+        thread.start()
+        thread.join()
+        eager(2)
+
+    graph = gpu.Graph.capture(streams[0], record)
+    gpu.synchronize()
+    assert not errors
+    cases[1].check()
+    cases[2].check()
+    cases[0].y.fill(0)
+    for _ in range(3):
+        graph.launch(streams[0].ptr)
+        gpu.synchronize()
+        cases[0].check()
+        assert not cases[1].y.download(np.uint32).any() and not cases[2].y.download(np.uint32).any()
+    graph.destroy()
+    for s in used + streams:
+        s.destroy()
