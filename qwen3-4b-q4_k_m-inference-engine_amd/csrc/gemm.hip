@@ -135,11 +135,6 @@ size_t xsum_offset(int64_t M, int64_t K) {
   return (bytes + 15) & ~size_t{15};
 }
 
-size_t partial_offset(int64_t M, int64_t K) {
-  const size_t bytes = xsum_offset(M, K) + static_cast<size_t>(M) * static_cast<size_t>(K / 256) * 32;
-  return (bytes + 255) & ~size_t{255};
-}
-
 WorkspaceLayout layout(void* workspace, int64_t M, int64_t K) {
   auto* base = static_cast<_Float16*>(workspace);
   return {base, base + M * K, reinterpret_cast<float*>(base + 2 * M * K),
@@ -148,8 +143,8 @@ WorkspaceLayout layout(void* workspace, int64_t M, int64_t K) {
 
 }  // namespace
 
-size_t gemm_workspace_bytes(int64_t M, int64_t K, int type, int64_t N) {
-  const size_t bytes = partial_offset(M, K) + gemm_kq_partial_bytes(type, M, K, N);
+size_t gemm_planes_bytes(int64_t M, int64_t K) {
+  const size_t bytes = xsum_offset(M, K) + static_cast<size_t>(M) * static_cast<size_t>(K / 256) * 32;
   return (bytes + 255) & ~size_t{255};
 }
 
@@ -173,7 +168,7 @@ hipError_t launch_gemm_core(const float* x, const void* workspace, const void* w
   const WorkspaceLayout ws = layout(const_cast<void*>(workspace), M, K);
   if (!gemm_kq_fits(M, K, N)) return hipErrorInvalidValue;
   float* partials = reinterpret_cast<float*>(static_cast<char*>(const_cast<void*>(workspace)) +
-                                             partial_offset(M, K));
+                                             gemm_planes_bytes(M, K));
   return launch_gemm_kq(type, x, ws.hi, ws.row_scale, ws.xs, w, K, N, y, M, partials, stream);
 }
 

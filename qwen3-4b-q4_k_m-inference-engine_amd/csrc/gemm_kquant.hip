@@ -941,6 +941,12 @@ double plan_cost(int type, bool wide, int64_t tiles, int64_t splits, int64_t M, 
 // 18.2; 9728 x 2560, 7 -> 5: Q4_K 18.2 -> 16.5, Q6_K 22.7 -> 20.8).
 constexpr int64_t kPlanSplits = 6;
 
+// Bytes of the workspace of a product that runs in `splits` splits.
+size_t plan_bytes(int64_t M, int64_t N, int64_t K, int64_t splits) {
+  const size_t partials = splits > 1 ? static_cast<size_t>(splits) * M * N * sizeof(float) : 0;
+  return (gemm_planes_bytes(M, K) + partials + 255) & ~size_t{255};
+}
+
 KQPlan plan(int type, int64_t M, int64_t N, int64_t K) {
   const KQPlan rule = rule_plan(type, M, N, K);
   const int64_t S = K / 256;
@@ -958,15 +964,12 @@ KQPlan plan(int type, int64_t M, int64_t N, int64_t K) {
   // (longer fp32 sums), that keep the workspace within the scratch of
   // qk_matmul_noalloc where the rule's plan is within it.
   const int64_t most = std::max<int64_t>(rule.splits, std::clamp<int64_t>(S / (M <= 64 ? 2 : 4), 1, kPlanSplits));
-  const int64_t planes = M * K * 4 + M * S * 32 + M * 4 + 512;
-  const bool within = planes + (rule.splits > 1 ? rule.splits * M * N * 4 : 0) <= static_cast<int64_t>(QK_NOALLOC_SCRATCH_BYTES);
+  const bool within = plan_bytes(M, N, K, rule.splits) <= QK_NOALLOC_SCRATCH_BYTES;
   KQPlan best = rule;
   double least = plan_cost(type, rule.wide, rule.wide ? tiles64 : tiles32, rule.splits, M, N, S);
   for (const bool wide : {false, true})
     for (int64_t splits = rule.splits; splits <= most; ++splits) {
-      if (splits > rule.splits && within &&
-          planes + splits * M * N * 4 > static_cast<int64_t>(QK_NOALLOC_SCRATCH_BYTES))
-        break;
+      if (splits > rule.splits && within && plan_bytes(M, N, K, splits) > QK_NOALLOC_SCRATCH_BYTES) break;
       const double cost = plan_cost(type, wide, wide ? tiles64 : tiles32, splits, M, N, S);
       if (cost < least) {
         least = cost;
@@ -983,9 +986,8 @@ bool gemm_kq_fits(int64_t M, int64_t K, int64_t N) {
          M * N <= (int64_t{1} << 40);
 }
 
-size_t gemm_kq_partial_bytes(int type, int64_t M, int64_t K, int64_t N) {
-  const KQPlan p = plan(type, M, N, K);
-  return p.splits > 1 ? static_cast<size_t>(p.splits) * M * N * sizeof(float) : 0;
+size_t gemm_workspace_bytes(int64_t M, int64_t K, int type, int64_t N) {
+  return plan_bytes(M, N, K, plan(type, M, N, K).splits);
 }
 
 hipError_t launch_gemm_kq(int type, const float* x, const _Float16* hi, const float* row_scale,

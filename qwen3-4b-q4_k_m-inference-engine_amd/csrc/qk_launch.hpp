@@ -135,6 +135,8 @@ constexpr int64_t kGemvMaxRows = 8;
 // fp16 Q8 round trip, row scales, block sums) and, when the launch splits K,
 // the partial products of an N-column product of this type; rounded up to 256.
 size_t gemm_workspace_bytes(int64_t M, int64_t K, int type, int64_t N);
+// The part of it before the partial products, a multiple of 256.
+size_t gemm_planes_bytes(int64_t M, int64_t K);
 
 // A short prompt (at most kGemmShortRows rows) times matrices of at most
 // kGemmShortTiles 128-column tiles each: the GEMM forms its activation planes
@@ -160,10 +162,9 @@ hipError_t launch_gemm_core(const float* x, const void* workspace, const void* w
 
 // The Q4_K / Q6_K GEMM (gemm_kquant.hip) over the prepared planes: hi (lo
 // follows it), row scales and (Q4_K) sub-block sums of the workspace, partial
-// products in `partials` (gemm_kq_partial_bytes of them; unused when 0).
+// products in `partials` (unused without splits).
 // gemm_kq_fits: the shape is within its 32-bit tile and row indices.
 bool gemm_kq_fits(int64_t M, int64_t K, int64_t N);
-size_t gemm_kq_partial_bytes(int type, int64_t M, int64_t K, int64_t N);
 hipError_t launch_gemm_kq(int type, const float* x, const _Float16* hi, const float* row_scale,
                           const void* xsums, const void* w, int64_t K, int64_t N, float* y, int64_t M,
                           float* partials, hipStream_t stream);

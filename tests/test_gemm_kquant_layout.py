@@ -283,3 +283,49 @@ def test_weight_operand_fma_is_exact():
         assert np.array_equal(v.astype(np.float16).astype(np.float64), q * sc)
     assert np.all(np.float16(sc / 16.0).astype(np.float64) == sc / 16.0)
     assert np.all(np.float16(-1024.0 * sc).astype(np.float64) == -1024.0 * sc)
+
+
+def rule_splits(qtype, M, N, K):
+    """Splits of K the grid rule asks for (rule_plan)."""
+    n_tiles = -(-N // 128)
+    tiles64, tiles32 = -(-M // 64) * n_tiles, -(-M // 32) * n_tiles
+    wide = M > 32 and 2 * tiles64 >= (256 if qtype == 14 else 3 * 256)
+    tiles = tiles64 if wide else tiles32
+    if M > 65535:
+        return 1
+    if M <= 32:
+        return min(max(1, min(-(-512 // tiles), K // 256)), K // 256)
+    return min(max(1, min(512 // tiles, 4)), max(K // 256 // 4, 1))
+
+
+def planes_bytes(M, K):
+    return (((M * K * 4 + M * 4 + 15) & ~15) + M * (K // 256) * 32 + 255) & ~255
+
+
+def test_no_shape_leaves_the_fixed_scratch_that_the_grid_rule_keeps_in_it(qk):
+    """qk_matmul_noalloc takes a shape when its workspace fits 48 MiB. The plan
+    may ask for more splits than the grid rule, never for so many that a shape
+    whose rule fits no longer does, to the byte: rows up to the last that fits
+    at every depth, and columns up to the last that fits where K splits."""
+    limit = 48 << 20
+    shapes = {(12, 7168, 519, 1702), (14, 7168, 1185, 1702)}
+    for S in range(16, 120):
+        K = 256 * S
+        M = limit // (4 * K + 4 + 32 * S)
+        while planes_bytes(M, K) > limit:
+            M -= 1
+        for qtype in (12, 14):
+            for m in (M, M - 1):
+                shapes |= {(qtype, K, N, m) for N in (1, 519, 1024, 1185, 2560)}
+            for m in (33, 64, 65, 200, M // 2):
+                for splits in (2, 3, 4):
+                    N = max((limit - planes_bytes(m, K)) // (4 * m * splits), 1)
+                    shapes |= {(qtype, K, n, m) for n in (N, N - 1, N // 2) if n > 0}
+    kept = 0
+    for qtype, K, N, M in sorted(shapes):
+        splits = rule_splits(qtype, M, N, K)
+        rule = (planes_bytes(M, K) + (4 * splits * M * N if splits > 1 else 0) + 255) & ~255
+        if rule <= limit:
+            kept += 1
+            assert qk.matmul_workspace_size(qtype, K, N, M) <= limit, (qtype, K, N, M)
+    assert kept > 2000
