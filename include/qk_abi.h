@@ -97,13 +97,18 @@ int qk_matmul(const float *x, const void *w, int type, int64_t K, int64_t N, flo
  * (M*K*4 + M*4 bytes, rounded up to 16), their block sums (M*(K/256)*32) and,
  * when the launch plan splits K (few output tiles, deep K), the partial
  * products (splits*M*N*4); the total is rounded up to 256. The split plan is
- * internal: size workspaces with this function, not from the formula. */
+ * internal: size workspaces with this function, not from the formula. It does
+ * not grow with M everywhere: a product of 33..64 rows, or of 65 and more with
+ * K >= 4096, splits K for speed and can need more than a larger one. */
 size_t qk_matmul_workspace_size(int type, int64_t K, int64_t N, int64_t M);
 
 /* qk_matmul with a caller-owned device workspace (16-byte aligned) of at least
  * qk_matmul_workspace_size() bytes (may be NULL when that is 0); allocates
  * nothing, so it can be captured into a graph at any M. Same results as
- * qk_matmul. */
+ * qk_matmul. A smaller workspace that still holds the splits that the plan
+ * cannot do without (one sized for another M, say) is taken too: the product
+ * then runs in fewer splits, which is slower and adds in another order; below
+ * that QK_ERR_INVALID_ARGUMENT. The _ws forms below do the same. */
 int qk_matmul_ws(const float *x, const void *w, int type, int64_t K, int64_t N, float *y,
                  int64_t M, void *workspace, size_t workspace_bytes, qk_stream_t stream);
 

@@ -131,6 +131,15 @@ int run_single(const float* x, const qk_q8_block* q8, const void* w, int type, i
   return run_matvec(p, M, K, 0, stream);
 }
 
+// The largest of the segments' workspaces (they run one after another on one
+// prep); bytes: gemm_workspace_bytes or gemm_workspace_least.
+size_t segments_gemm_bytes(size_t (*bytes)(int64_t, int64_t, int, int64_t), int64_t M, int64_t K,
+                           const qk_segment* segments, int count) {
+  size_t need = 0;
+  for (int j = 0; j < count; ++j) need = std::max(need, bytes(M, K, segments[j].type, segments[j].N));
+  return need;
+}
+
 // Prefill path (M > 8 rows): activation prep once, then one MFMA GEMM per
 // weight matrix. Without a caller workspace the fp16 activation scratch is
 // taken for the call (scratch.hpp), where the reference allocates its Q8
@@ -144,17 +153,15 @@ int run_gemm(const float* x, int64_t M, int64_t K, const qk_segment* segments, i
     if (M > (int64_t{1} << 31) - 128 || m_tiles * n_tiles > (int64_t{1} << 31) - 1)
       return fail(QK_ERR_INVALID_ARGUMENT, "matmul rows x columns exceed the launch grid");
   }
-  size_t need = 0;  // the largest of the segments' needs (they run one after another)
-  for (int j = 0; j < count; ++j)
-    need = std::max(need, qk::gemm_workspace_bytes(M, K, segments[j].type, segments[j].N));
   void* scratch = workspace;
   qk::Scratch own(stream);
   if (scratch) {
-    if (workspace_bytes < need) return fail(QK_ERR_INVALID_ARGUMENT, "matmul workspace too small");
+    if (workspace_bytes < segments_gemm_bytes(qk::gemm_workspace_least, M, K, segments, count)) return fail(QK_ERR_INVALID_ARGUMENT, "matmul workspace too small");
     if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0)
       return fail(QK_ERR_INVALID_ARGUMENT, "matmul workspace must be 16-byte aligned");
   } else {
-    const hipError_t error = own.get(need, scratch);
+    workspace_bytes = segments_gemm_bytes(qk::gemm_workspace_bytes, M, K, segments, count);
+    const hipError_t error = own.get(workspace_bytes, scratch);
     if (error != hipSuccess) return hip_fail(error, "matmul workspace allocation failed");
   }
   // short prompt against narrow matrices: the GEMM forms its planes from x
@@ -178,8 +185,8 @@ int run_gemm(const float* x, int64_t M, int64_t K, const qk_segment* segments, i
         continue;
       }
     }
-    error = qk::launch_gemm_core(x_short, scratch, segments[j].w, segments[j].type, K, segments[j].N,
-                                 segments[j].y, M, stream);
+    error = qk::launch_gemm_core(x_short, scratch, workspace_bytes, segments[j].w, segments[j].type, K,
+                                 segments[j].N, segments[j].y, M, stream);
   }
   return error == hipSuccess ? QK_OK : hip_fail(error, "matmul launch failed");
 }
@@ -283,29 +290,32 @@ namespace {
 // where no split K is needed) into scratch, then SiLU(gate) * up into h. The
 // scratch (gate and up outputs, then the GEMM workspace) is the caller's
 // workspace when given, else taken for the call (scratch.hpp).
+size_t ffn_gemm_outputs(int64_t N, int64_t M) {
+  return (2 * static_cast<size_t>(M) * static_cast<size_t>(N) * sizeof(float) + 255) & ~size_t{255};
+}
 size_t ffn_gemm_bytes(int type, int64_t K, int64_t N, int64_t M) {
-  const size_t gu = (2 * static_cast<size_t>(M) * static_cast<size_t>(N) * sizeof(float) + 255) & ~size_t{255};
-  return gu + qk::gemm_workspace_bytes(M, K, type, N);
+  return ffn_gemm_outputs(N, M) + qk::gemm_workspace_bytes(M, K, type, N);
 }
 
 int run_ffn_gemm(const float* x, const void* gate, const void* up, int type, int64_t K, int64_t N,
                  float* h, int64_t M, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-  const size_t need = ffn_gemm_bytes(type, K, N, M);
+  const size_t gu_bytes = ffn_gemm_outputs(N, M);
   void* scratch = workspace;
   qk::Scratch own(stream);
   if (scratch) {
-    if (workspace_bytes < need) return fail(QK_ERR_INVALID_ARGUMENT, "ffn workspace too small");
+    if (workspace_bytes < gu_bytes + qk::gemm_workspace_least(M, K, type, N))
+      return fail(QK_ERR_INVALID_ARGUMENT, "ffn workspace too small");
     if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0)
       return fail(QK_ERR_INVALID_ARGUMENT, "ffn workspace must be 16-byte aligned");
   } else {
-    const hipError_t error = own.get(need, scratch);
+    workspace_bytes = ffn_gemm_bytes(type, K, N, M);
+    const hipError_t error = own.get(workspace_bytes, scratch);
     if (error != hipSuccess) return hip_fail(error, "ffn scratch allocation failed");
   }
   float* gu = static_cast<float*>(scratch);
-  const size_t gu_bytes = need - qk::gemm_workspace_bytes(M, K, type, N);
   const qk_segment segments[2] = {{gate, type, N, gu}, {up, type, N, gu + M * N}};
-  int status = run_gemm(x, M, K, segments, 2, static_cast<char*>(scratch) + gu_bytes, need - gu_bytes,
-                        stream);
+  int status = run_gemm(x, M, K, segments, 2, static_cast<char*>(scratch) + gu_bytes,
+                        workspace_bytes - gu_bytes, stream);
   if (status == QK_OK) {
     const hipError_t error = qk::launch_silu_multiply(gu, gu + M * N, h, M * N, stream);
     if (error != hipSuccess) status = hip_fail(error, "silu_multiply launch failed");
@@ -331,14 +341,6 @@ int ffn_gate_up(const float* x, const void* gate, const void* up, int type, int6
   p.seg[0] = {static_cast<const uint8_t*>(gate), nullptr, static_cast<int32_t>(N), type, 0, 0};
   p.seg[1] = {static_cast<const uint8_t*>(up), nullptr, static_cast<int32_t>(N), type, 0, 0};
   return run_matvec(p, M, K, 1, stream);
-}
-
-// Largest workspace of the segments (they run one after another on one prep).
-size_t segments_gemm_bytes(int64_t M, int64_t K, const qk_segment* segments, int count) {
-  size_t need = 0;
-  for (int j = 0; j < count; ++j)
-    need = std::max(need, qk::gemm_workspace_bytes(M, K, segments[j].type, segments[j].N));
-  return need;
 }
 
 int matmul_segments(const float* x, int64_t M, int64_t K, const qk_segment* segments, int count,
@@ -382,7 +384,7 @@ size_t qk_matmul_segments_workspace_size(int64_t M, int64_t K, const qk_segment*
     return 0;
   for (int j = 0; j < count; ++j)
     if (!supported_type(segments[j].type) || segments[j].N <= 0) return 0;
-  return segments_gemm_bytes(M, K, segments, count);
+  return segments_gemm_bytes(qk::gemm_workspace_bytes, M, K, segments, count);
 }
 
 int qk_matmul_segments_ws(const float* x, int64_t M, int64_t K, const qk_segment* segments, int count,

@@ -163,13 +163,13 @@ hipError_t launch_gemm_prep(const float* x, int64_t M, int64_t K, void* workspac
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_core(const float* x, const void* workspace, const void* w, int type, int64_t K,
-                            int64_t N, float* y, int64_t M, hipStream_t stream) {
+hipError_t launch_gemm_core(const float* x, const void* workspace, size_t workspace_bytes, const void* w,
+                            int type, int64_t K, int64_t N, float* y, int64_t M, hipStream_t stream) {
   const WorkspaceLayout ws = layout(const_cast<void*>(workspace), M, K);
   if (!gemm_kq_fits(M, K, N)) return hipErrorInvalidValue;
   float* partials = reinterpret_cast<float*>(static_cast<char*>(const_cast<void*>(workspace)) +
                                              gemm_planes_bytes(M, K));
-  return launch_gemm_kq(type, x, ws.hi, ws.row_scale, ws.xs, w, K, N, y, M, partials, stream);
+  return launch_gemm_kq(type, x, ws.hi, ws.row_scale, ws.xs, w, K, N, y, M, partials, workspace_bytes, stream);
 }
 
 hipError_t launch_gemm_core_multi(const float* x, const void* workspace, const qk_segment* segments, int count,

@@ -947,7 +947,9 @@ size_t plan_bytes(int64_t M, int64_t N, int64_t K, int64_t splits) {
   return (gemm_planes_bytes(M, K) + partials + 255) & ~size_t{255};
 }
 
-KQPlan plan(int type, int64_t M, int64_t N, int64_t K) {
+// The plan of a product whose workspace has `room` bytes: no more splits than
+// it holds, except the rule's.
+KQPlan plan(int type, int64_t M, int64_t N, int64_t K, size_t room = SIZE_MAX) {
   const KQPlan rule = rule_plan(type, M, N, K);
   const int64_t S = K / 256;
   if (M > 65535 || (M > 64 && S < 16)) return rule;
@@ -964,12 +966,13 @@ KQPlan plan(int type, int64_t M, int64_t N, int64_t K) {
   // (longer fp32 sums), that keep the workspace within the scratch of
   // qk_matmul_noalloc where the rule's plan is within it.
   const int64_t most = std::max<int64_t>(rule.splits, std::clamp<int64_t>(S / (M <= 64 ? 2 : 4), 1, kPlanSplits));
-  const bool within = plan_bytes(M, N, K, rule.splits) <= QK_NOALLOC_SCRATCH_BYTES;
+  if (plan_bytes(M, N, K, rule.splits) <= QK_NOALLOC_SCRATCH_BYTES)
+    room = std::min<size_t>(room, QK_NOALLOC_SCRATCH_BYTES);
   KQPlan best = rule;
   double least = plan_cost(type, rule.wide, rule.wide ? tiles64 : tiles32, rule.splits, M, N, S);
   for (const bool wide : {false, true})
     for (int64_t splits = rule.splits; splits <= most; ++splits) {
-      if (splits > rule.splits && within && plan_bytes(M, N, K, splits) > QK_NOALLOC_SCRATCH_BYTES) break;
+      if (splits > rule.splits && plan_bytes(M, N, K, splits) > room) break;
       const double cost = plan_cost(type, wide, wide ? tiles64 : tiles32, splits, M, N, S);
       if (cost < least) {
         least = cost;
@@ -990,10 +993,14 @@ size_t gemm_workspace_bytes(int64_t M, int64_t K, int type, int64_t N) {
   return plan_bytes(M, N, K, plan(type, M, N, K).splits);
 }
 
+size_t gemm_workspace_least(int64_t M, int64_t K, int type, int64_t N) {
+  return plan_bytes(M, N, K, std::min(rule_plan(type, M, N, K).splits, plan(type, M, N, K).splits));
+}
+
 hipError_t launch_gemm_kq(int type, const float* x, const _Float16* hi, const float* row_scale,
                           const void* xsums, const void* w, int64_t K, int64_t N, float* y, int64_t M,
-                          float* partials, hipStream_t stream) {
-  const KQPlan p = plan(type, M, N, K);
+                          float* partials, size_t room, hipStream_t stream) {
+  const KQPlan p = plan(type, M, N, K, room);
   const bool short_m = x != nullptr;  // the short form: planes formed from x in the GEMM
   if (short_m && M > kShortM) return hipErrorInvalidValue;
   KQGemmArgs a{};

@@ -134,7 +134,11 @@ constexpr int64_t kGemvMaxRows = 8;
 // Bytes of device scratch the prefill GEMM needs for M x K activations (their
 // fp16 Q8 round trip, row scales, block sums) and, when the launch splits K,
 // the partial products of an N-column product of this type; rounded up to 256.
+// gemm_workspace_least: what a call runs in with no more splits of K than the
+// grid rule asks for (a caller that sized its workspace for another M may
+// bring less than gemm_workspace_bytes).
 size_t gemm_workspace_bytes(int64_t M, int64_t K, int type, int64_t N);
+size_t gemm_workspace_least(int64_t M, int64_t K, int type, int64_t N);
 // The part of it before the partial products, a multiple of 256.
 size_t gemm_planes_bytes(int64_t M, int64_t K);
 
@@ -149,25 +153,26 @@ inline bool gemm_short_plan(int64_t M, int64_t N) {
   return M <= kGemmShortRows && (N + 127) / 128 <= kGemmShortTiles;
 }
 
-// workspace (>= gemm_workspace_bytes(M, K, ...), 16-byte aligned) = fp16 of
+// workspace (>= gemm_workspace_least(M, K, ...), 16-byte aligned) = fp16 of
 // the Q8 round trip of x[M x K], row scales, block sums (not needed when every
 // product of the call takes the short form: `skip`).
 hipError_t launch_gemm_prep(const float* x, int64_t M, int64_t K, void* workspace,
                             hipStream_t stream, bool skip = false);
 
 // y[M x N] = x . dequant(W)^T on MFMA, fp32 accumulation, over the prepared
-// workspace (M <= kGemmShortRows: over x itself).
-hipError_t launch_gemm_core(const float* x, const void* workspace, const void* w, int type, int64_t K,
-                            int64_t N, float* y, int64_t M, hipStream_t stream);
+// workspace of workspace_bytes (M <= kGemmShortRows: over x itself).
+hipError_t launch_gemm_core(const float* x, const void* workspace, size_t workspace_bytes, const void* w,
+                            int type, int64_t K, int64_t N, float* y, int64_t M, hipStream_t stream);
 
 // The Q4_K / Q6_K GEMM (gemm_kquant.hip) over the prepared planes: hi (lo
 // follows it), row scales and (Q4_K) sub-block sums of the workspace, partial
-// products in `partials` (unused without splits).
+// products in `partials` (unused without splits), all in a workspace of `room`
+// bytes, which bounds the splits.
 // gemm_kq_fits: the shape is within its 32-bit tile and row indices.
 bool gemm_kq_fits(int64_t M, int64_t K, int64_t N);
 hipError_t launch_gemm_kq(int type, const float* x, const _Float16* hi, const float* row_scale,
                           const void* xsums, const void* w, int64_t K, int64_t N, float* y, int64_t M,
-                          float* partials, hipStream_t stream);
+                          float* partials, size_t room, hipStream_t stream);
 
 // 2..4 weight matrices of width K (either type) on the same prepared
 // activations in one launch (attn q, k and v; gate and up): launched (and

@@ -399,8 +399,8 @@ def test_split_k_workspace_from_garbage_and_across_plans(gpu, oracle):
 def test_ffn_gate_up_workspace_variant_and_deep_k(gpu, oracle, qtype, K, N, M):
     """qk_ffn_gate_up_ws equals qk_ffn_gate_up bit for bit; the deep-K shape
     (K = 9728, N = 2560) takes the split-K GEMM for gate and up in separate
-    launches, checked against the oracle; a workspace short of
-    qk_ffn_gate_up_workspace_size is rejected."""
+    launches, checked against the oracle; a workspace that does not hold the
+    launches' outputs and planes is rejected."""
     gate = make_weight(gpu, qtype, N, K, SEED + 60)
     up = make_weight(gpu, qtype, N, K, SEED + 61)
     x = oracle.synth_normal(M * K, SEED + 62)
@@ -421,8 +421,11 @@ def test_ffn_gate_up_workspace_variant_and_deep_k(gpu, oracle, qtype, K, N, M):
     err = oracle.row_norm_error(a.reshape(M, N), ref)
     print(f"[case] ffn prefill type={qtype} K={K} N={N} M={M} error {err:.3e}", flush=True)
     assert err <= 1e-5
+    # (without its extra splits of K the call also runs in less: see the
+    # workspace sized for another row count below)
+    least = 2 * M * N * 4 + M * (4 * K + 4 + K // 8)  # outputs of gate and up, planes, one K range
     assert gpu.load().qk_ffn_gate_up_ws(xd.ptr, gate.ptr, up.ptr, qtype, K, N, h2.ptr, M, ws.ptr,
-                                        need - 256, None) == 1
+                                        least - 256, None) == 1
 
 
 def test_segments_workspace_variant(gpu, oracle):
@@ -498,3 +501,40 @@ def test_prefill_planned_splits_against_oracle(gpu, oracle, qtype, K, N, M):
     xr = np.concatenate([x.reshape(M, K)[r] for r in rows])
     ref = float64_reference(oracle, xr, w.download(np.uint8), qtype, K, N, len(rows))
     check(oracle, got, ref, f"planned {qtype} {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("qtype,K,N,M_sized,M", [
+    (Q4, 2560, 9728, 512, 56), (Q4, 2560, 9728, 512, 33), (Q6, 2560, 1024, 65, 48), (Q4, 4096, 9728, 400, 100),
+])
+def test_workspace_sized_for_more_rows_serves_fewer(gpu, oracle, qtype, K, N, M_sized, M):
+    """A workspace of qk_matmul_workspace_size at a larger M runs a smaller one
+    whose own size is larger (it would split K finer), alone, as a segment and
+    as gate and up: the results of the full workspace but for the order of
+    fp32 sums, and nothing written past the workspace."""
+    need = gpu.matmul_workspace_size(qtype, K, N, M)
+    has = gpu.matmul_workspace_size(qtype, K, N, M_sized)
+    assert has < need
+    w, up = make_weight(gpu, qtype, N, K, SEED + 95), make_weight(gpu, qtype, N, K, SEED + 96)
+    x = oracle.synth_normal(M * K, SEED + 97)
+    xd = gpu.DeviceBuffer.from_array(x)
+    y, h = gpu.DeviceBuffer(4 * M * N), gpu.DeviceBuffer(4 * M * N)
+    gpu.matmul(xd, w, qtype, K, N, y, M)
+    gpu.ffn_gate_up(xd, w, up, qtype, K, N, h, M)
+    gpu.synchronize()
+    want, want_h = (b.download(np.float32).reshape(M, N).astype(np.float64) for b in (y, h))
+    ws = gpu.DeviceBuffer.from_array(np.full(has + 256, 0xFF, np.uint8))
+    for call in (lambda: gpu.matmul_ws(xd, w, qtype, K, N, y, M, ws, has),
+                 lambda: gpu.matmul_segments_ws(xd, M, K, [(w, qtype, N, y)], ws, has)):
+        y.fill(0xFF)
+        call()
+        gpu.synchronize()
+        print(f"[case] {qtype} M={M} in the workspace of M={M_sized}: {gpu.last_launch()}", flush=True)
+        assert oracle.row_norm_error(y.download(np.float32).reshape(M, N), want) <= 1e-6
+        assert np.all(ws.download(np.uint8)[has:] == 0xFF)
+    has = gpu.ffn_gate_up_workspace_size(qtype, K, N, M) - 256  # a split less
+    ws = gpu.DeviceBuffer.from_array(np.full(has + 256, 0xFF, np.uint8))
+    h.fill(0xFF)
+    gpu.ffn_gate_up_ws(xd, w, up, qtype, K, N, h, M, ws, has)
+    gpu.synchronize()
+    assert oracle.row_norm_error(h.download(np.float32).reshape(M, N), want_h) <= 1e-6
+    assert np.all(ws.download(np.uint8)[has:] == 0xFF)
