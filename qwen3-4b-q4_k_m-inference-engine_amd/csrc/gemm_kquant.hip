@@ -1038,12 +1038,19 @@ hipError_t launch_gemm_kq_multi(const float* x, const _Float16* hi, const float*
                                 hipStream_t stream, bool& launched) {
   launched = false;
   if (count < 2 || count > kKQMaxSegments) return hipSuccess;
-  // One launch when the combined grid needs no split of K: each tile then
-  // does exactly the work of an unsplit launch of its matrix (outputs bit for
-  // bit those of the single launch when that does not split; within the
-  // splits' rounding of it otherwise: a split changes the order of the sums),
-  // in one grid that fills the CUs. Q6_K matrices first: their tiles take
-  // longer, so they start first.
+  // One launch when the combined grid needs no split of K by the grid rule:
+  // each tile then does exactly the work of an unsplit launch of its matrix
+  // (outputs bit for bit those of the single launch when that does not split;
+  // within the splits' rounding of it otherwise: a split changes the order of
+  // the sums), in one grid that fills the CUs. The rule decides, not the
+  // estimated time: that takes a split for a few per cent, while a launch of
+  // several matrices that would gain them runs as a GEMM and a reduce per
+  // matrix instead (us, workspaces, one launch against that: q/k/v 1024 ->
+  // 2048 + 1024 + 1024 at M = 33..48 13.4 against 28.9, gate/up 1024 -> 3072 in
+  // Q6_K at M = 33..64 19 against 27, 2560 -> 9728 in Q4_K at M = 33 / 64 41 /
+  // 47 against 44 / 48, q/k/v 4096 -> 4096 + 1024 + 1024 at M = 200 / 512 47 /
+  // 79 against 67 / 104). Q6_K matrices first: their tiles take longer, so
+  // they start first.
   int order[kKQMaxSegments], n = 0;
   bool q4 = false, q6 = false;
   int64_t total = 0;
@@ -1057,7 +1064,8 @@ hipError_t launch_gemm_kq_multi(const float* x, const _Float16* hi, const float*
   }
   if (!gemm_kq_fits(M, K, total)) return hipSuccess;
   const int type = q4 && q6 ? 0 : q4 ? QK_TYPE_Q4_K : QK_TYPE_Q6_K;
-  if (plan(type == 0 ? QK_TYPE_Q4_K : type, M, total, K).splits > 1) return hipSuccess;
+  const KQPlan rule = rule_plan(type == 0 ? QK_TYPE_Q4_K : type, M, total, K);
+  if (rule.splits > 1) return hipSuccess;
   // The tile shape of the combined grid. The mixed-type kernel exists for
   // 32 x 128 tiles only: it is taken while the grid has fewer than two
   // 64 x 128 tiles per CU (q + k + v at M = 512: 384), else same-type pairs run.
@@ -1067,7 +1075,7 @@ hipError_t launch_gemm_kq_multi(const float* x, const _Float16* hi, const float*
   if (type == 0 && !short_m) {
     if (((M + 63) / 64) * ((total + 127) / 128) >= 2 * kPlanCUs) return hipSuccess;
   } else if (type != 0) {
-    wide = plan(type, M, total, K).wide;
+    wide = rule.wide;
   }
   KQGemmArgs a{};
   a.x = x;

@@ -176,9 +176,9 @@ hipError_t launch_gemm_kq(int type, const float* x, const _Float16* hi, const fl
 
 // 2..4 weight matrices of width K (either type) on the same prepared
 // activations in one launch (attn q, k and v; gate and up): launched (and
-// `launched` set) when none needs a split K and all take the combined grid's
-// tile shape, else nothing is enqueued. Each output equals its single launch's
-// bit for bit.
+// `launched` set) when the combined grid needs no split K and all take its tile
+// shape, else nothing is enqueued. Each output equals its single launch's bit
+// for bit where that does not split K (else within the order of fp32 sums).
 hipError_t launch_gemm_kq_multi(const float* x, const _Float16* hi, const float* row_scale, const void* xsums,
                                 const qk_segment* segments, int count, int64_t K, int64_t M,
                                 hipStream_t stream, bool& launched);

@@ -538,3 +538,40 @@ def test_workspace_sized_for_more_rows_serves_fewer(gpu, oracle, qtype, K, N, M_
     gpu.synchronize()
     assert oracle.row_norm_error(h.download(np.float32).reshape(M, N), want_h) <= 1e-6
     assert np.all(ws.download(np.uint8)[has:] == 0xFF)
+
+
+@pytest.mark.parametrize("M,K,shapes", [
+    (33, 1024, [(Q4, 2048), (Q4, 1024), (Q4, 1024)]), (48, 1024, [(Q4, 2048), (Q4, 1024), (Q6, 1024)]),
+    (49, 1024, [(Q4, 2048), (Q4, 1024), (Q4, 1024)]), (64, 1024, [(Q4, 2048), (Q4, 1024), (Q6, 1024)]),
+    (200, 4096, [(Q4, 4096), (Q4, 1024), (Q6, 1024)]), (512, 4096, [(Q4, 4096), (Q4, 1024), (Q4, 1024)]),
+    (33, 1024, [(Q6, 3072), (Q6, 3072)]), (64, 1024, [(Q6, 3072), (Q6, 3072)]),
+    (33, 2560, [(Q4, 9728), (Q4, 9728)]), (64, 2560, [(Q4, 9728), (Q4, 9728)]), (65, 4096, [(Q4, 8192), (Q4, 8192)]),
+])
+def test_matrices_whose_grid_fills_the_cus_share_one_launch(gpu, oracle, M, K, shapes):
+    """q/k/v, and gate and up, whose grids together need no split of K run as
+    one unsplit launch, also where each alone would be split for speed; every
+    output within fp32 sums of its single product, and the first rows of the
+    last matrix against float64."""
+    ws = [make_weight(gpu, q, N, K, SEED + 110 + i) for i, (q, N) in enumerate(shapes)]
+    x = oracle.synth_normal(M * K, SEED + 111)
+    xd = gpu.DeviceBuffer.from_array(x)
+    ys = [gpu.DeviceBuffer(4 * M * N) for _, N in shapes]
+    gpu.matmul_segments(xd, M, K, [(w, q, N, y) for w, (q, N), y in zip(ws, shapes, ys)])
+    launch = gpu.last_launch()
+    print(f"[case] M={M} K={K} {shapes} launch {launch}", flush=True)
+    kind = shapes[0][0] if len({q for q, _ in shapes}) == 1 else 0
+    name, values = launch.split(">")[0].split("<")
+    values = [int(v) for v in values.split(",")]
+    assert name == "gemm_kq_kernel" and values[0] == kind and values[-1] == 1
+    grid, tiles = int(launch.split("grid=")[1]), -(-M // (32 * values[1])) * sum(-(-N // 128) for _, N in shapes)
+    assert grid == (tiles + 7) // 8 * 8  # the tiles of every matrix
+    gpu.synchronize()
+    for (q, N), w, y in zip(shapes, ws, ys):
+        one = gpu.DeviceBuffer(4 * M * N)
+        gpu.matmul(xd, w, q, K, N, one, M)
+        gpu.synchronize()
+        got = y.download(np.float32).reshape(M, N)
+        assert oracle.row_norm_error(got, one.download(np.float32).reshape(M, N).astype(np.float64)) <= 1e-6
+    q, N = shapes[-1]
+    ref = float64_reference(oracle, x[:3 * K], ws[-1].download(np.uint8), q, K, N, 3)
+    check(oracle, got[:3], ref, f"one launch M={M} K={K}")
