@@ -937,7 +937,9 @@ double plan_cost(int type, bool wide, int64_t tiles, int64_t splits, int64_t M, 
 // M = 48 21.0 -> 14.6. (At smaller K and larger M finer splits gain less, and
 // a row's sums are the same there at every M.) At M <= 32 the rule's split is
 // the most: its units are one to three a CU, and a few over two a CU cost a
-// round (2560 x 9728 at M = 23, 26 -> 19 splits: Q6_K 27.1 -> 23.7, Q4_K 19.9 ->
+// round; fewer splits only while no split takes more superblocks (no longer
+// fp32 sums: two a split of 8, where the rule has one, would be 7% faster at
+// 2048 -> 6144, M = 32, and is not taken) (2560 x 9728 at M = 23, 26 -> 19 splits: Q6_K 27.1 -> 23.7, Q4_K 19.9 ->
 // 18.2; 9728 x 2560, 7 -> 5: Q4_K 18.2 -> 16.5, Q6_K 22.7 -> 20.8).
 constexpr int64_t kPlanSplits = 6;
 
@@ -957,7 +959,8 @@ KQPlan plan(int type, int64_t M, int64_t N, int64_t K, size_t room = SIZE_MAX) {
   const int64_t tiles32 = ((M + 31) / 32) * n_tiles, tiles64 = ((M + 63) / 64) * n_tiles;
   if (M <= 32) {
     KQPlan best = rule;
-    for (int64_t splits = rule.splits - 1; splits >= 1; --splits)
+    const int64_t deepest = (S + rule.splits - 1) / rule.splits;
+    for (int64_t splits = rule.splits - 1; splits * deepest >= S; --splits)
       if (plan_cost(type, false, tiles32, splits, M, N, S) < plan_cost(type, false, tiles32, best.splits, M, N, S))
         best.splits = static_cast<int>(splits);
     return best;

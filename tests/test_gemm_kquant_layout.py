@@ -329,3 +329,20 @@ def test_no_shape_leaves_the_fixed_scratch_that_the_grid_rule_keeps_in_it(qk):
             kept += 1
             assert qk.matmul_workspace_size(qtype, K, N, M) <= limit, (qtype, K, N, M)
     assert kept > 2000
+
+
+def test_short_prompts_sum_no_more_superblocks_in_a_row_than_the_grid_rule(qk):
+    """At M <= 32 the plan may drop splits that only add a round of work units,
+    never so that a split adds more superblocks than the grid rule's largest,
+    which would lengthen the fp32 sums."""
+    fewer = 0
+    for M in (9, 17, 23, 32):
+        for S in (1, 2, 4, 8, 9, 10, 12, 16, 36, 38, 43):
+            for N in (64, 1024, 2560, 3001, 6144, 9728, 20000, 27038):
+                for qtype in (12, 14):
+                    K = 256 * S
+                    partials = qk.matmul_workspace_size(qtype, K, N, M) - planes_bytes(M, K)
+                    splits, rule = max(partials // (4 * M * N), 1), rule_splits(qtype, M, N, K)
+                    fewer += splits < rule
+                    assert splits <= rule and -(-S // splits) <= -(-S // rule), (qtype, K, N, M)
+    assert fewer > 0
