@@ -372,7 +372,7 @@ bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int (&count
     int64_t tiles = 0, units = 0;
     for (int j = 0; j < nseg; ++j) {
       const int per = p.seg[j].rows / count[j];
-      for (int n : {per, per + 1}) {
+      for (int n : {per, per + (p.seg[j].rows % count[j] != 0)}) {
         tiles = std::max(tiles, bmv_wave_tiles(n, parts, p.S, r));
         units = std::max<int64_t>(units, (parts * ((n + 15) / 16) * r + kBmvWaves - 1) / kBmvWaves);
       }

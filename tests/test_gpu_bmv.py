@@ -75,3 +75,20 @@ def test_several_matrices(gpu, oracle, K, shapes, M, takes):
         assert out[-1] == 123.0
         ref = oracle.reference_product(x, h, q, K, N).reshape(M, N)
         assert oracle.row_norm_error(out[:-1].reshape(M, N), ref) <= 1e-5
+
+
+@pytest.mark.parametrize("K,N,M,ranges", [(8192, 4096, 8, 16), (8192, 4095, 8, 16), (9728, 4096, 3, 13)])
+def test_runs_of_a_share_of_sixteen_rows(gpu, oracle, K, N, M, ranges):
+    """256 CUs of exactly 16 rows are one row group each, planned like those of
+    15 and 16: as many runs as the waves need."""
+    w_host = oracle.synth_superblocks(Q4, N, K, SEED + 80, 0.01, 0.01)
+    w = gpu.DeviceBuffer.from_array(w_host)
+    x = oracle.synth_normal(M * K, SEED + 81)
+    xd = gpu.DeviceBuffer.from_array(x)
+    y = gpu.DeviceBuffer(4 * M * N)
+    gpu.matmul(xd, w, Q4, K, N, y, M)
+    gpu.synchronize()
+    print(f"[case] K={K} N={N} M={M} launch {gpu.last_launch()}", flush=True)
+    assert gpu.last_launch() == f"bmv_kernel<12,0,{ranges},1,0> grid=256"
+    ref = oracle.reference_product(x, w_host, Q4, K, N).reshape(M, N)
+    assert oracle.row_norm_error(y.download(np.float32).reshape(M, N), ref) <= 1e-5
