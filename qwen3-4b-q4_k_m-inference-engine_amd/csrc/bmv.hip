@@ -316,14 +316,22 @@ int64_t bmv_wave_tiles(int64_t rows, int parts, int S, int ranges) {
   return per_wave * ((S + ranges - 1) / ranges);
 }
 
+struct BmvPlan {
+  int count[kMaxSegments] = {0};
+  int ranges = 0, groups_max = 0, lds = 0;
+  int rows_max = 0;       // of the largest share (with slots: of the largest that goes through them)
+  int64_t tiles = 0;      // on the busiest wave
+  int64_t all_tiles = 0;  // the same if LDS held the sums of any number of runs
+};
+
 // The workgroups of each matrix and the run split of a launch (the CPU index
 // model of the tests restates these rules). One matrix, or gate and up, over
 // every CU; several matrices: at most kBmvMaxGroups row groups of 16 a
 // workgroup (Q6_K: one of at most kBmvSlotRows rows, through the slots), the
 // fewest that fit the CUs, what is left in proportion to the bytes. Returns
 // false when the shape does not fit.
-bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int (&count)[kMaxSegments], int& ranges,
-              int& groups_max, int& rows_max, int& lds) {
+bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, BmvPlan& plan) {
+  int(&count)[kMaxSegments] = plan.count;
   const int parts = mode == 1 ? 2 : 1, nseg = mode == 1 ? 1 : p.nseg;
   bool slots = false;
   if (nseg == 1) {
@@ -350,8 +358,7 @@ bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int (&count
     for (int j = 0; j < nseg; ++j)
       count[j] = std::min(p.seg[j].rows, count[j] + static_cast<int>(left * bytes[j] / total));
   }
-  rows_max = 0;
-  int slot_rows = 0;
+  int rows_max = 0, slot_rows = 0;
   for (int j = 0; j < nseg; ++j) {
     const int rows = p.seg[j].rows / count[j] + (p.seg[j].rows % count[j] != 0);
     rows_max = std::max(rows_max, rows);
@@ -360,59 +367,94 @@ bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, int (&count
       if (rows > kBmvSlotRows || static_cast<int64_t>(p.seg[j].rows) * p.S * kQ6KBytes + 16 > INT32_MAX) return false;
     }
   }
-  groups_max = (rows_max + 15) / 16;
-  if (slots) rows_max = slot_rows;  // (what the slots are sized by)
+  plan.groups_max = (rows_max + 15) / 16;
+  plan.rows_max = slots ? slot_rows : rows_max;
   const int stride = p.K + 16, slot_bytes = slots ? kBmvWaves * bmv_slot_bytes(slot_rows) : 0;
   // runs per group: the fewest tiles on the busiest wave of any workgroup,
   // then the fewest units (each unit ends with a lane reduction)
-  ranges = 0;
   int64_t best = INT64_MAX;
+  plan.all_tiles = INT64_MAX;
   for (int r = 1; r <= p.S; ++r) {
-    if (bmv_lds_bytes(p.K, stride, parts, groups_max, r) + slot_bytes > max_lds) break;
+    const int lds = bmv_lds_bytes(p.K, stride, parts, plan.groups_max, r) + slot_bytes;
+    const bool fits = lds <= max_lds;
+    if (!fits && plan.ranges == 0) return false;
     int64_t tiles = 0, units = 0;
     for (int j = 0; j < nseg; ++j) {
-      const int per = p.seg[j].rows / count[j];
-      for (int n : {per, per + (p.seg[j].rows % count[j] != 0)}) {
-        tiles = std::max(tiles, bmv_wave_tiles(n, parts, p.S, r));
-        units = std::max<int64_t>(units, (parts * ((n + 15) / 16) * r + kBmvWaves - 1) / kBmvWaves);
-      }
+      const int rows = p.seg[j].rows / count[j] + (p.seg[j].rows % count[j] != 0);
+      tiles = std::max(tiles, bmv_wave_tiles(rows, parts, p.S, r));
+      units = std::max<int64_t>(units, (parts * ((rows + 15) / 16) * r + kBmvWaves - 1) / kBmvWaves);
     }
+    plan.all_tiles = std::min(plan.all_tiles, tiles);
     const int64_t cost = 8 * tiles + units;
-    if (cost < best) {
+    if (fits && cost < best) {
       best = cost;
-      ranges = r;
+      plan.ranges = r;
+      plan.tiles = tiles;
+      plan.lds = lds;
     }
   }
-  if (ranges == 0) return false;
-  lds = bmv_lds_bytes(p.K, stride, parts, groups_max, ranges) + slot_bytes;
   return true;
+}
+
+// Where a launch of mode 0 pays: measured on MI355X against the streaming and
+// per-row kernels, graphs over weights out of cache, 3,400 launches of M = 2..8,
+// 256 to 16384 columns, 16 to 8192 rows, one to three matrices; none that is
+// taken is more than 3% slower. us, the other kernel -> this one:
+//  - one Q4_K matrix from M = 3 (9728 -> 2560 at M = 3 / 8 13.2 / 22.2 -> 9.5 /
+//    14.6; at M = 2 9.2 -> 9.5).
+//  - one Q6_K matrix from M = 5 (9728 -> 2560 at M = 8 22.4 -> 17.9), at M = 8, and
+//    at M = 7 up to K = 8192, above 3 rows a CU (5120 -> 256 10.5 -> 11.2). At M = 3 and 4 while K <=
+//    8192, where the streaming kernel would run (6400 -> 256 9.7 -> 7.9), or
+//    above 8 rows a CU (9728 -> 2560 at M = 3 13.1 -> 12.2): with fewer a tile is
+//    mostly empty (9728 -> 256 9.6 -> 10.2).
+//  - several matrices from 9 superblocks a row: below, the waves have a tile
+//    each or none (2048 -> 4096 + 1024 + 1024 at M = 3 6.9 -> 8.0). From M = 5 all
+//    of these (2560 -> 4096 + 1024 + 1024 at M = 8 11.8 -> 8.4). At M = 2..4 not
+//    both types, nor over 20 rows a CU (24 at K = 4096), where 8 divides the
+//    superblocks and the others idle no lanes (6144 -> 4096 + 4064 at M = 3 12.9
+//    -> 14.3; 6400 0.88 times the time); all Q4_K from M = 3, at M = 2 up to K =
+//    6400, 8192 with at most 16 rows a CU (8192 -> 4096 + 1024 + 1024 10.6 ->
+//    13.1, 2048 + 512 + 512 10.6 -> 9.0); with Q6_K from M = 3 as one matrix of
+//    it, with both types only above 8 rows a CU (4352 -> 4096 + 1024 + 1024 0.89
+//    times the time, 1024 + 256 + 256 1.04).
+bool bmv_pays(const MatvecParams& p, int cus) {
+  int64_t rows = 0;
+  bool q4 = false, q6 = false;
+  for (int j = 0; j < p.nseg; ++j) {
+    rows += p.seg[j].rows;
+    (p.seg[j].type == QK_TYPE_Q4_K ? q4 : q6) = true;
+  }
+  const bool full = rows > 8 * cus;
+  if (p.nseg == 1) {
+    if (q4 || p.M < 3) return p.M >= 3;
+    if (p.M <= 4) return p.K <= 8192 || full;
+    return p.M <= 6 || rows > 3 * cus || (p.M == 7 && p.K > 8192);
+  }
+  if (p.S < 9 || p.M >= 5) return p.S >= 9;
+  if (p.S % 8 == 0 && ((q4 && q6) || rows > (p.K <= 4096 ? 24 : 20) * cus)) return false;
+  if (!q6) return p.M >= 3 || p.K <= (rows > 16 * cus ? 6400 : 8192);
+  return p.M >= 3 && (full || (!q4 && p.K <= 8192));
 }
 
 hipError_t launch_bmv(const MatvecParams& p, int mode, hipStream_t stream, bool& launched) {
   launched = false;
-  // Gate/up (mode 1), and at M >= 3 one matrix (mode 0) of at most 16 rows a
-  // workgroup (Q6_K: 13) that the whole-share kernel does not take (its weights
-  // and activations exceed LDS: ffn_down, K = 9728). Measured on MI355X, us, the
-  // streaming kernel before: ffn_down in fp32 Q4_K at M = 3 / 8 13.2 / 22.2 ->
-  // 9.5 / 14.6, Q6_K 13.1 / 22.4 -> 12.2 / 17.9; at M = 2 it is the faster one
-  // (9.2 against 9.5, 10.3 against 11.4).
-  // Several matrices (q/k/v): all-Q4_K at M = 3 / 5 / 8 8.3 / 11.5 / 11.8 -> 6.7 /
-  // 7.1 / 8.0, with a Q6_K v 7.4 / 10.9 / 11.3 -> 7.3 / 7.9 / 8.7 (at M = 2 the
-  // streaming kernel's 6.4 us are the faster ones there).
-  bool all_q4 = true;
-  for (int j = 0; j < p.nseg; ++j) all_q4 = all_q4 && p.seg[j].type == QK_TYPE_Q4_K;
-  const int least = mode == 1 || (p.nseg > 1 && all_q4) ? 2 : 3;
-  if (p.M < least || p.M > 8 || (mode != 0 && mode != 1)) return hipSuccess;
+  if (p.M < 2 || p.M > 8 || (mode != 0 && mode != 1)) return hipSuccess;
   if (mode == 1 ? p.x == nullptr || p.nseg != 2 : p.nseg > 1 && p.x == nullptr) return hipSuccess;
-  if (p.K > (INT32_MAX - 64) / 8) return hipSuccess;
+  if (p.K > INT32_MAX / 16) return hipSuccess;  // (the LDS plan counts in 32 bits)
   int cus = 0, max_lds = 0;
   hipError_t e = device_limits(cus, max_lds);
   if (e != hipSuccess) return e;
-  int count[kMaxSegments] = {0}, ranges = 0, groups_max = 0, rows_max = 0, lds = 0;
-  if (!bmv_plan(p, mode, cus, max_lds, count, ranges, groups_max, rows_max, lds)) return hipSuccess;
-  if (mode == 0 && p.nseg == 1 && groups_max > 1) return hipSuccess;
+  if (mode == 0 && !bmv_pays(p, cus)) return hipSuccess;
+  BmvPlan plan;
+  if (!bmv_plan(p, mode, cus, max_lds, plan)) return hipSuccess;
+  if (mode == 0 && p.nseg == 1 && plan.groups_max > 1) return hipSuccess;
+  // Runs that LDS has no room for leave waves idle: at M <= 4 the other kernels
+  // win as soon as the busiest wave has a tile more (Q6_K 10240 -> 2560, 5 tiles
+  // for 3, M = 4 1.12 times the time), at M >= 5 past twice its tiles (5 for 3
+  // 0.90 times at M = 8; 12288 -> 1024, 16 for 3, 20.7 -> 34.0 us).
+  if (mode == 0 && plan.tiles > (p.M <= 4 ? 1 : 2) * plan.all_tiles) return hipSuccess;
   if (p.hq != nullptr) {  // Q8(h) in the launch: a quad per (block, activation row) of a share
-    const int64_t rows_max = (p.seg[0].rows + count[0] - 1) / count[0];
+    const int64_t rows_max = (p.seg[0].rows + plan.count[0] - 1) / plan.count[0];
     const int64_t blocks = (rows_max + 30) / 32 + 1;  // blocks a run of rows_max rows can touch
     if (p.seg[0].rows % 32 != 0 || blocks > kBmvMaxCloseBlocks || 4 * blocks * p.M > 64 * kBmvWaves ||
         p.arrive == nullptr)
@@ -429,24 +471,24 @@ hipError_t launch_bmv(const MatvecParams& p, int mode, hipStream_t stream, bool&
   bp.K = p.K;
   bp.S = p.S;
   bp.stride = p.K + 16;
-  bp.ranges = ranges;
-  bp.groups_max = groups_max;
-  bp.rows_max = rows_max;
+  bp.ranges = plan.ranges;
+  bp.groups_max = plan.groups_max;
+  bp.rows_max = plan.rows_max;
   bp.nseg = p.nseg;
   int begin = 0;
   for (int j = 0; j < p.nseg; ++j) {
-    const int c = mode == 1 ? count[0] : count[j];
+    const int c = mode == 1 ? plan.count[0] : plan.count[j];
     bp.seg[j] = {p.seg[j].w, p.seg[j].y, p.seg[j].rows, p.seg[j].type, begin, p.seg[j].rows / c, p.seg[j].rows % c, 0};
     if (mode == 0 || j == 0) begin += c;
   }
   const int type = mode == 0 && p.nseg > 1 ? 0 : p.seg[0].type;
   const BmvKernel fn = bmv_kernel_for(type, mode, p.x == nullptr);
   if (!fn) return hipSuccess;
-  e = allow_lds(reinterpret_cast<const void*>(fn), lds);
+  e = allow_lds(reinterpret_cast<const void*>(fn), plan.lds);
   if (e != hipSuccess) return e;
-  note("bmv_kernel", begin, type, mode, ranges, groups_max, p.hq != nullptr);
+  note("bmv_kernel", begin, type, mode, plan.ranges, plan.groups_max, p.hq != nullptr);
   hipLaunchKernelGGL(fn, dim3(static_cast<uint32_t>(begin)), dim3(64 * kBmvWaves),
-                     static_cast<size_t>(lds), stream, bp);
+                     static_cast<size_t>(plan.lds), stream, bp);
   launched = true;
   return hipGetLastError();
 }

@@ -19,6 +19,12 @@ SEED = 20261501
     (Q4, 12288, 700, 8, True), (Q4, 9728, 2560, 2, False),
     (Q6, 9728, 2560, 3, True), (Q6, 9728, 2561, 4, True), (Q6, 9728, 2560, 5, True), (Q6, 9728, 2816, 8, True),
     (Q6, 9984, 257, 7, True), (Q6, 9728, 3329, 8, False), (Q6, 9728, 2560, 2, False),
+    # M = 3, 4: to K = 8192, or above 8 rows a CU; M = 8, and 7 to K = 8192: above 3 rows a CU
+    (Q6, 8192, 257, 4, True), (Q6, 8448, 2048, 3, False), (Q6, 8448, 2049, 4, True), (Q6, 5120, 768, 8, False),
+    (Q6, 5120, 769, 8, True), (Q6, 5888, 257, 7, False), (Q6, 8448, 257, 7, True), (Q6, 5888, 257, 6, True),
+    # LDS without room for the runs: 5 tiles on a wave for 3, 16 for 3, 53 for 4
+    (Q6, 10240, 2560, 4, False), (Q6, 10240, 2560, 5, True), (Q6, 12288, 1024, 3, False), (Q6, 12288, 1024, 8, False),
+    (Q4, 13568, 300, 3, False), (Q4, 13056, 300, 3, True),
 ])
 def test_one_wide_matrix(gpu, oracle, qtype, K, N, M, takes):
     w_host = oracle.synth_superblocks(qtype, N, K, SEED + N, 0.01, 0.01)
@@ -54,8 +60,27 @@ def test_one_wide_matrix(gpu, oracle, qtype, K, N, M, takes):
     (2560, [(Q4, 4096), (Q4, 1024), (Q6, 1024)], 2, False),
     (2560, [(Q6, 1700), (Q4, 33), (Q6, 1560), (Q4, 17)], 5, True),   # 13 rows of Q6_K a workgroup
     (2560, [(Q6, 1700), (Q4, 33), (Q6, 1700), (Q4, 17)], 5, False),  # past the CUs
-    (1024, [(Q4, 8160), (Q4, 32)], 4, True),                 # 256 workgroups of 32 rows
-    (1024, [(Q4, 8160), (Q4, 33)], 4, False),
+    (1280, [(Q4, 8160), (Q4, 32)], 5, False),                # under 9 superblocks a row
+    (2560, [(Q4, 8160), (Q4, 32)], 4, True),                 # 256 workgroups of 32 rows
+    (2560, [(Q4, 8160), (Q4, 33)], 4, False),
+    (2048, [(Q4, 4096), (Q4, 1024), (Q4, 1024)], 8, False),  # 8 superblocks a row, and 9
+    (2304, [(Q4, 4096), (Q4, 1024), (Q4, 1024)], 2, True),
+    (4096, [(Q4, 4096), (Q4, 1024), (Q4, 1024)], 2, True),   # 8 divides the superblocks: 24 rows a CU
+    (4096, [(Q4, 4096), (Q4, 2048), (Q4, 33)], 4, False),
+    (4096, [(Q4, 4096), (Q4, 2048), (Q4, 33)], 5, True),
+    (6144, [(Q4, 4096), (Q4, 1024)], 3, True),               # past K = 4096: 20
+    (6144, [(Q4, 4096), (Q4, 1024), (Q4, 33)], 3, False),
+    (4096, [(Q4, 2048), (Q4, 512), (Q6, 512)], 3, False),    # and not both types
+    (4352, [(Q4, 2048), (Q4, 512), (Q6, 512)], 3, True),
+    (4352, [(Q4, 1024), (Q4, 512), (Q6, 512)], 3, False),    # both types: above 8 rows a CU
+    (4352, [(Q4, 1024), (Q4, 513), (Q6, 512)], 4, True),
+    (4352, [(Q4, 1024), (Q4, 512), (Q6, 512)], 5, True),
+    (4352, [(Q6, 700), (Q6, 700)], 3, True),                 # one type
+    (8448, [(Q6, 700), (Q6, 700)], 4, False),
+    (6400, [(Q4, 4096), (Q4, 1024)], 2, True),               # M = 2: the last K
+    (6656, [(Q4, 4096), (Q4, 1024)], 2, False),
+    (8192, [(Q4, 2048), (Q4, 2048)], 2, True),
+    (8448, [(Q4, 2048), (Q4, 2048)], 2, False),
 ])
 def test_several_matrices(gpu, oracle, K, shapes, M, takes):
     """One launch of 2..4 matrices on fp32 activations against the oracle's
