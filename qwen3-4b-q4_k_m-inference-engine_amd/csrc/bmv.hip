@@ -416,7 +416,8 @@ bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, BmvPlan& pl
 //    6400, 8192 with at most 16 rows a CU (8192 -> 4096 + 1024 + 1024 10.6 ->
 //    13.1, 2048 + 512 + 512 10.6 -> 9.0); with Q6_K from M = 3 as one matrix of
 //    it, with both types only above 8 rows a CU (4352 -> 4096 + 1024 + 1024 0.89
-//    times the time, 1024 + 256 + 256 1.04).
+//    times the time, 1024 + 256 + 256 1.04), 16 below K = 3328 (2560 -> 2048 + 1024
+//    + 1024 1.04).
 bool bmv_pays(const MatvecParams& p, int cus) {
   int64_t rows = 0;
   bool q4 = false, q6 = false;
@@ -433,7 +434,8 @@ bool bmv_pays(const MatvecParams& p, int cus) {
   if (p.S < 9 || p.M >= 5) return p.S >= 9;
   if (p.S % 8 == 0 && ((q4 && q6) || rows > (p.K <= 4096 ? 24 : 20) * cus)) return false;
   if (!q6) return p.M >= 3 || p.K <= (rows > 16 * cus ? 6400 : 8192);
-  return p.M >= 3 && (full || (!q4 && p.K <= 8192));
+  if (q4) return p.M >= 3 && rows > (p.K < 3328 ? 16 : 8) * cus;
+  return p.M >= 3 && (full || p.K <= 8192);
 }
 
 hipError_t launch_bmv(const MatvecParams& p, int mode, hipStream_t stream, bool& launched) {

@@ -75,6 +75,9 @@ def test_one_wide_matrix(gpu, oracle, qtype, K, N, M, takes):
     (4352, [(Q4, 1024), (Q4, 512), (Q6, 512)], 3, False),    # both types: above 8 rows a CU
     (4352, [(Q4, 1024), (Q4, 513), (Q6, 512)], 4, True),
     (4352, [(Q4, 1024), (Q4, 512), (Q6, 512)], 5, True),
+    (2560, [(Q4, 2048), (Q4, 1024), (Q6, 1024)], 3, False),  # below K = 3328: 16
+    (2560, [(Q4, 2048), (Q4, 1025), (Q6, 1024)], 4, True),
+    (3328, [(Q4, 2048), (Q4, 1024), (Q6, 1024)], 3, True),
     (4352, [(Q6, 700), (Q6, 700)], 3, True),                 # one type
     (8448, [(Q6, 700), (Q6, 700)], 4, False),
     (6400, [(Q4, 4096), (Q4, 1024)], 2, True),               # M = 2: the last K
