@@ -14,21 +14,21 @@ int superblock_bytes(int type) { return type == QK_TYPE_Q4_K ? kQ4KBytes : kQ6KB
 
 }  // namespace
 
-BmvWsKernel bmv_ws_kernel_for(int type, int mode, bool q8in) {
+BmvWsKernel bmv_ws_kernel_for(int type, int mode, bool q8in, bool several) {
+  const bool q4 = type == QK_TYPE_Q4_K, q6 = type == QK_TYPE_Q6_K;
+  if (several) {
+    if (q8in || mode == 1) return nullptr;
+    return q4   ? &bmv_ws_kernel<QK_TYPE_Q4_K, 0, false, true>
+           : q6 ? &bmv_ws_kernel<QK_TYPE_Q6_K, 0, false, true>
+                : &bmv_ws_kernel<0, 0, false, true>;
+  }
+  if (!q4 && !q6) return nullptr;
   if (mode == 1) {
     if (q8in) return nullptr;
-    if (type == QK_TYPE_Q4_K) return &bmv_ws_kernel<QK_TYPE_Q4_K, 1, false>;
-    if (type == QK_TYPE_Q6_K) return &bmv_ws_kernel<QK_TYPE_Q6_K, 1, false>;
-    return nullptr;
+    return q4 ? &bmv_ws_kernel<QK_TYPE_Q4_K, 1, false, false> : &bmv_ws_kernel<QK_TYPE_Q6_K, 1, false, false>;
   }
-  if (q8in) {
-    if (type == QK_TYPE_Q4_K) return &bmv_ws_kernel<QK_TYPE_Q4_K, 0, true>;
-    if (type == QK_TYPE_Q6_K) return &bmv_ws_kernel<QK_TYPE_Q6_K, 0, true>;
-    return &bmv_ws_kernel<0, 0, true>;
-  }
-  if (type == QK_TYPE_Q4_K) return &bmv_ws_kernel<QK_TYPE_Q4_K, 0, false>;
-  if (type == QK_TYPE_Q6_K) return &bmv_ws_kernel<QK_TYPE_Q6_K, 0, false>;
-  return &bmv_ws_kernel<0, 0, false>;
+  if (q8in) return q4 ? &bmv_ws_kernel<QK_TYPE_Q4_K, 0, true, false> : &bmv_ws_kernel<QK_TYPE_Q6_K, 0, true, false>;
+  return q4 ? &bmv_ws_kernel<QK_TYPE_Q4_K, 0, false, false> : &bmv_ws_kernel<QK_TYPE_Q6_K, 0, false, false>;
 }
 
 // The plan of a launch (the CPU index model of the tests restates these
@@ -97,15 +97,17 @@ hipError_t launch_bmv_ws(const MatvecParams& p, int mode, hipStream_t stream, bo
   bp.stride = p.K + 16;
   bp.reg = plan.reg;
   bp.act = bmv_ws_act_bytes(p.K);
+  bool q4 = false, q6 = false;
   int begin = 0;
   for (int j = 0; j < nseg; ++j) {
+    (p.seg[j].type == QK_TYPE_Q4_K ? q4 : q6) = true;
     bp.seg[j] = {p.seg[j].w, p.seg[j].y, p.seg[j].rows, p.seg[j].type, begin,
                  p.seg[j].rows / plan.count[j], p.seg[j].rows % plan.count[j], 0};
     begin += plan.count[j];
   }
   if (mode == 1) bp.seg[1] = {p.seg[1].w, nullptr, p.seg[1].rows, p.seg[1].type, 0, 0, 0, 0};
-  const int type = nseg > 1 ? 0 : p.seg[0].type;
-  const BmvWsKernel fn = bmv_ws_kernel_for(type, mode, q8in);
+  const int type = q4 && q6 ? 0 : p.seg[0].type;
+  const BmvWsKernel fn = bmv_ws_kernel_for(type, mode, q8in, nseg > 1);
   if (!fn) return hipSuccess;
   e = allow_lds(reinterpret_cast<const void*>(fn), plan.lds);
   if (e != hipSuccess) return e;

@@ -268,25 +268,25 @@ __device__ __forceinline__ void bmv_ws_body(const BmvWsParams& p, const uint8_t*
   }
 }
 
-// TYPE: QK_TYPE_Q4_K or QK_TYPE_Q6_K, or 0 for a launch of several matrices
-// (each workgroup takes its matrix's type; the others read the arguments of
-// their own matrices only, since no load goes out before the last argument is
-// in: attn_output at M = 2 / 8 6.25 / 8.65 -> 5.80 / 8.29 us).
-template <int TYPE, int MODE, bool Q8IN>
+// TYPE: QK_TYPE_Q4_K or QK_TYPE_Q6_K, or 0 for a launch of both types (each
+// workgroup takes its matrix's). SEVERAL: a launch of several matrices; the
+// others read the arguments of their own only, since no load goes out before
+// the last argument is in (attn_output at M = 2 / 8 6.25 / 8.65 -> 5.80 / 8.29 us).
+template <int TYPE, int MODE, bool Q8IN, bool SEVERAL>
 __global__ __launch_bounds__(64 * kWsWaves) void bmv_ws_kernel(const BmvWsParams p) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
 #pragma unroll
-  for (int j = 0; j < (TYPE == 0 ? kMaxSegments : MODE + 1); ++j)
+  for (int j = 0; j < (SEVERAL ? kMaxSegments : MODE + 1); ++j)
     asm volatile("" ::"s"(p.seg[j].w), "s"(p.seg[j].y), "s"(p.seg[j].rows), "s"(p.seg[j].type),
                  "s"(p.seg[j].wg_begin), "s"(p.seg[j].per), "s"(p.seg[j].rem), "s"(p.seg[j].pad));
   asm volatile("" ::"s"(p.x), "s"(p.q8), "s"(p.h), "s"(p.M), "s"(p.K), "s"(p.S), "s"(p.nseg), "s"(p.stride),
                "s"(p.reg), "s"(p.act), "s"(p.pad));
   __builtin_amdgcn_sched_barrier(0);
-  const int wg = static_cast<int>(blockIdx.x), nseg = TYPE == 0 ? p.nseg : 1;
+  const int wg = static_cast<int>(blockIdx.x), nseg = SEVERAL ? p.nseg : 1;
   const int j = (nseg > 1 && wg >= p.seg[1].wg_begin) + (nseg > 2 && wg >= p.seg[2].wg_begin) +
                 (nseg > 3 && wg >= p.seg[3].wg_begin);
   auto pick = [j](auto f0, auto f1, auto f2, auto f3) {
-    if constexpr (TYPE != 0) return f0;
+    if constexpr (!SEVERAL) return f0;
     return j == 0 ? f0 : j == 1 ? f1 : j == 2 ? f2 : f3;
   };
   const int type = pick(p.seg[0].type, p.seg[1].type, p.seg[2].type, p.seg[3].type);
@@ -311,8 +311,8 @@ __global__ __launch_bounds__(64 * kWsWaves) void bmv_ws_kernel(const BmvWsParams
 
 using BmvWsKernel = void (*)(BmvWsParams);
 
-// The instantiations (bmv_ws.hip); type 0 is a launch of several matrices. Null when
-// there is no such kernel.
-BmvWsKernel bmv_ws_kernel_for(int type, int mode, bool q8in);
+// The instantiations (bmv_ws.hip); type 0 is a launch of both types. Null when
+// there is no such kernel (several matrices come from fp32 rows only).
+BmvWsKernel bmv_ws_kernel_for(int type, int mode, bool q8in, bool several);
 
 }  // namespace qk
