@@ -138,9 +138,13 @@ hipError_t release_scratch() {
   for (Block& b : g_blocks[device]) {
     if (error != hipSuccess || b.busy || !b.ptr) continue;
     error = hipFreeAsync(b.ptr, nullptr);
+    if (error != hipSuccess) break;
     b.ptr = nullptr;
     b.bytes = 0;
   }
+  // (a stream-ordered free returns the memory to the pool; the pool gives it
+  // back when its stream is next synchronised)
+  if (error == hipSuccess) error = hipStreamSynchronize(nullptr);
   return error;
 }
 

@@ -4,6 +4,7 @@ across block sizes, under capture and after a release, each result equal bit
 for bit to qk_matmul_ws on a workspace of its own."""
 from __future__ import annotations
 
+import ctypes
 import threading
 
 import numpy as np
@@ -145,4 +146,32 @@ def test_calls_while_another_stream_is_captured(gpu, oracle, others):
         assert not cases[1].y.download(np.uint32).any() and not cases[2].y.download(np.uint32).any()
     graph.destroy()
     for s in used + streams:
+        s.destroy()
+
+
+def _free_bytes(qk):
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert qk.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_release_gives_the_blocks_back(gpu, oracle):
+    """8 streams hold a block each; once qk_release_scratch has returned their
+    memory is free on the device, and later calls run as before."""
+    case = Case(gpu, oracle, Q4, 2560, 256, 33, 20261601)
+    streams = [gpu.Stream() for _ in range(8)]
+    gpu.release_scratch()
+    before = _free_bytes(gpu)
+    for s in streams:
+        case.run(s.ptr)
+    gpu.synchronize()
+    held = _free_bytes(gpu)
+    assert before - held >= 8 * (16 << 20)
+    case.check()
+    gpu.release_scratch()
+    assert _free_bytes(gpu) - held >= 8 * (16 << 20)
+    case.run(streams[0].ptr)
+    gpu.synchronize()
+    case.check()
+    for s in streams:
         s.destroy()
