@@ -401,7 +401,8 @@ bool bmv_plan(const MatvecParams& p, int mode, int cus, int max_lds, BmvPlan& pl
 // 256 to 16384 columns, 16 to 8192 rows, one to three matrices; none that is
 // taken is more than 3% slower. us, the other kernel -> this one:
 //  - one Q4_K matrix from M = 3 (9728 -> 2560 at M = 3 / 8 13.2 / 22.2 -> 9.5 /
-//    14.6; at M = 2 9.2 -> 9.5).
+//    14.6; at M = 2 9.2 -> 9.5), at M = 2 up to K = 8192 (the streaming kernel, which
+//    the quantiser's registers slowed there: 7936 -> 2560 10.65 -> 7.7).
 //  - one Q6_K matrix from M = 5 (9728 -> 2560 at M = 8 22.4 -> 17.9), at M = 8, and
 //    at M = 7 up to K = 8192, above 3 rows a CU (5120 -> 256 10.5 -> 11.2). At M = 3 and 4 while K <=
 //    8192, where the streaming kernel would run (6400 -> 256 9.7 -> 7.9), or
@@ -427,7 +428,8 @@ bool bmv_pays(const MatvecParams& p, int cus) {
   }
   const bool full = rows > 8 * cus;
   if (p.nseg == 1) {
-    if (q4 || p.M < 3) return p.M >= 3;
+    if (q4) return p.M >= 3 || p.K <= 8192;
+    if (p.M < 3) return false;
     if (p.M <= 4) return p.K <= 8192 || full;
     return p.M <= 6 || rows > 3 * cus || (p.M == 7 && p.K > 8192);
   }

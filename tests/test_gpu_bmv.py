@@ -16,7 +16,8 @@ SEED = 20261501
 
 @pytest.mark.parametrize("qtype,K,N,M,takes", [
     (Q4, 9728, 2560, 3, True), (Q4, 9728, 2561, 8, True), (Q4, 9728, 4096, 4, True), (Q4, 9728, 4097, 5, False),
-    (Q4, 12288, 700, 8, True), (Q4, 9728, 2560, 2, False),
+    (Q4, 12288, 700, 8, True), (Q4, 9728, 2560, 2, False), (Q4, 8192, 4096, 2, True), (Q4, 5888, 17, 2, True),
+    (Q4, 8448, 300, 2, False), (Q6, 5888, 300, 2, False),
     (Q6, 9728, 2560, 3, True), (Q6, 9728, 2561, 4, True), (Q6, 9728, 2560, 5, True), (Q6, 9728, 2816, 8, True),
     (Q6, 9984, 257, 7, True), (Q6, 9728, 3329, 8, False), (Q6, 9728, 2560, 2, False),
     # M = 3, 4: to K = 8192, or above 8 rows a CU; M = 8, and 7 to K = 8192: above 3 rows a CU
