@@ -2,12 +2,13 @@
 (qwen3-4b-q4_k_m-inference-engine_amd/csrc/bmv.hip, bmv.hpp), M = 2..8.
 
 For each shape the model restates the launcher's plan (workgroups per
-segment, superblock runs per row group, LDS size) and the kernel's cursors,
-then checks every global load of every lane of every wave of every workgroup
-(inside its superblock and its matrix, including the ring's refills past a
-wave's last tile), every LDS read and write against its region, and that each
-(part, row, superblock) is computed by exactly one tile and each unit's sums
-slot written once. A lane-level emulation of the arithmetic (the block-
+matrix, superblock runs per row group, LDS size with the slots, which launches
+are made at all) and the kernel's cursors, then checks every global load of
+every lane of every wave of every workgroup (inside its superblock and its
+matrix, including the ring's refills past a wave's last tile; Q6_K in mode 0:
+the chunks of a tile's rows, up to the zeros past the descriptor's end), every
+LDS read and write against its region, and that each (part, row, superblock)
+is computed by exactly one tile and each unit's sums slot written once. A lane-level emulation of the arithmetic (the block-
 diagonal A tiles as the lanes read them from the LDS image, the B operands as
 the lanes build them, v_mfma_i32_16x16x64_i8 as an integer product with the
 probed lane layout: lane l holds A[l%16][16(l/16)+t], B[16(l/16)+t][l%16] and
@@ -18,14 +19,19 @@ must be mirrored here."""
 import numpy as np
 import pytest
 
-CUS, MAX_LDS, WAVES = 256, 160 * 1024, 8
+CUS, MAX_LDS, WAVES = 256, 160 * 1024, 16
 BYTES = {12: 144, 14: 210}
-P = {12: 6, 14: 4}
-P_MIXED6 = 3
+P = {12: 2, 14: 1}
+SLOT_CHUNKS, SLOT_LOADS = 14, 3
+SLOT_ROWS = 64 * SLOT_LOADS // SLOT_CHUNKS
 
 
-def lds_bytes(K, stride, parts, groups, ranges):
+def sums_end(K, stride, parts, groups, ranges):
     return 8 * stride + 16 + 4 * K + parts * groups * 16 * ranges * 32
+
+
+def slot_bytes(rows):
+    return 16 * SLOT_CHUNKS * rows
 
 
 def wave_tiles(rows, parts, S, ranges):
@@ -36,38 +42,80 @@ def wave_tiles(rows, parts, S, ranges):
     return -(-units // WAVES) * -(-S // ranges)
 
 
-def plan(rows, types, K, mode, M):
-    """(workgroups per segment, ranges, groups_max, lds) or None when the launcher declines."""
-    if not 2 <= M <= 8 or mode not in (0, 1):
-        return None
+def counts(rows, types, mode):
+    """Workgroups of each matrix, or None past the CUs."""
+    if mode == 1 or len(rows) == 1:
+        return [min(CUS, rows[0])]
+    for groups in (1, 2):
+        need = [-(-r // (SLOT_ROWS if t == 14 else 16 * groups)) for r, t in zip(rows, types)]
+        if sum(need) <= CUS:
+            byt = [r * BYTES[t] for r, t in zip(rows, types)]
+            left = CUS - sum(need)
+            return [min(r, c + int(left * x / sum(byt))) for r, c, x in zip(rows, need, byt)]
+    return None
+
+
+def fits(rows, types, K, mode):
+    """bmv_plan: (workgroups per matrix, ranges, groups_max, lds, rows of a
+    slot, tiles on the busiest wave, the same with any LDS), or None."""
     nseg = 1 if mode == 1 else len(rows)
     parts = 2 if mode == 1 else 1
-    S = K // 256
-    if nseg > CUS:
+    S, stride = K // 256, K + 16
+    count = counts(rows, types, mode)
+    if count is None:
         return None
-    byt = [rows[j] * S * BYTES[types[j]] * parts for j in range(nseg)]
-    total = float(sum(byt))
-    count = [min(max(int(CUS * b / total + 0.5), 1), rows[j]) for j, b in enumerate(byt)]
-    while sum(count) > CUS:
-        count[count.index(max(count))] -= 1
-    stride = K + 16
-    groups_max = max(-(-(-(-rows[j] // count[j])) // 16) for j in range(nseg))
-    ranges, best = 0, None
+    most = [-(-rows[j] // count[j]) for j in range(nseg)]
+    slot_rows = max([most[j] for j in range(nseg) if mode == 0 and types[j] == 14], default=0)
+    if slot_rows > SLOT_ROWS:
+        return None
+    groups_max = max(-(-m // 16) for m in most)
+    best, all_tiles = None, None
     for r in range(1, S + 1):
-        if lds_bytes(K, stride, parts, groups_max, r) > MAX_LDS:
-            break
-        tiles = units = 0
-        for j in range(nseg):
-            per = rows[j] // count[j]
-            for n in (per, per + 1):
-                tiles = max(tiles, wave_tiles(n, parts, S, r))
-                units = max(units, -(-(parts * -(-n // 16) * r) // WAVES))
-        cost = 8 * tiles + units
-        if best is None or cost < best:
-            best, ranges = cost, r
-    if ranges == 0:
+        lds = sums_end(K, stride, parts, groups_max, r) + WAVES * slot_bytes(slot_rows)
+        if lds > MAX_LDS and best is None:
+            return None
+        tiles = max(wave_tiles(m, parts, S, r) for m in most)
+        units = max(-(-(parts * -(-m // 16) * r) // WAVES) for m in most)
+        all_tiles = tiles if all_tiles is None else min(all_tiles, tiles)
+        if lds <= MAX_LDS and (best is None or 8 * tiles + units < best[0]):
+            best = (8 * tiles + units, r, lds, tiles)
+    return count, best[1], groups_max, best[2], slot_rows, best[3], all_tiles
+
+
+def pays(rows, types, K, M):
+    """bmv_pays: the lines of mode 0."""
+    total, S, q4, q6 = sum(rows), K // 256, 12 in types, 14 in types
+    if len(rows) == 1:
+        if q4:
+            return M >= 3 or K <= 8192
+        if M < 3:
+            return False
+        if M <= 4:
+            return K <= 8192 or total > 8 * CUS
+        return M <= 6 or total > 3 * CUS or (M == 7 and K > 8192)
+    if S < 9 or M >= 5:
+        return S >= 9
+    if S % 8 == 0 and ((q4 and q6) or total > (24 if K <= 4096 else 20) * CUS):
+        return False
+    if not q6:
+        return M >= 3 or K <= (6400 if total > 16 * CUS else 8192)
+    if q4:
+        return M >= 3 and total > (16 if K < 3328 else 8) * CUS
+    return M >= 3 and (K <= 8192 or total > 8 * CUS)
+
+
+def plan(rows, types, K, mode, M):
+    """The launch's plan, or None when the launcher declines."""
+    if not 2 <= M <= 8 or mode not in (0, 1):
         return None
-    return count, ranges, groups_max, lds_bytes(K, stride, parts, groups_max, ranges)
+    if mode == 0 and not pays(rows, types, K, M):
+        return None
+    cfg = fits(rows, types, K, mode)
+    if cfg is None or mode == 1:
+        return cfg
+    if (len(rows) == 1 and cfg[2] > 1) or cfg[5] > (1 if M <= 4 else 2) * cfg[6]:
+        return None
+    return cfg
 
 
 class Share:
@@ -147,7 +195,7 @@ def load_ranges(qtype, sb):
 
 
 def workgroups(rows, types, K, mode, cfg):
-    count, ranges, groups_max, lds = cfg
+    count, ranges = cfg[:2]
     nseg = 1 if mode == 1 else len(rows)
     parts = 2 if mode == 1 else 1
     for j in range(nseg):
@@ -163,19 +211,20 @@ def check_indices(rows, types, K, mode, M, bases):
     checked for all of them."""
     cfg = plan(rows, types, K, mode, M)
     assert cfg is not None
-    count, ranges, groups_max, lds = cfg
-    assert lds <= MAX_LDS
+    count, ranges, groups_max, lds, slot_rows = cfg[:5]
     S, stride = K // 256, K + 16
     Z = 8 * stride + 16
-    mixed = mode == 0 and len(set(types)) > 1
     parts = 2 if mode == 1 else 1
     nseg = 1 if mode == 1 else len(rows)
+    end = sums_end(K, stride, parts, groups_max, ranges)  # the slots of the waves follow
+    assert end + WAVES * slot_bytes(slot_rows) == lds <= MAX_LDS and sum(count[:nseg]) <= CUS
     chosen = set()
     for j in range(nseg):
         per, rem = rows[j] // count[j], rows[j] % count[j]
         shares = [(g * per + min(g, rem), per + (1 if g < rem else 0)) for g in range(count[j])]
         assert shares[0][0] == 0 and shares[-1][0] + shares[-1][1] == rows[j]
         assert all(a + n == b for (a, n), (b, _) in zip(shares, shares[1:])), "shares partition the rows"
+        assert all(1 <= n <= 16 * groups_max for _, n in shares)
         if count[j] <= 32:
             chosen |= {(j, r0) for r0, _ in shares}
         else:
@@ -187,11 +236,27 @@ def check_indices(rows, types, K, mode, M, bases):
             continue
         qtype = types[j]
         B = BYTES[qtype]
-        depth = P_MIXED6 if (mixed and qtype == 14) else P[qtype]
         rb = S * B
+        through_slots = qtype == 14 and mode == 0
         slots = {}
         for wave in range(WAVES):
-            comps, loads = wave_streams(sh, wave, depth)
+            comps, loads = wave_streams(sh, wave, P[qtype])
+            if through_slots:
+                assert sh.nrows <= slot_rows <= SLOT_ROWS and sh.groups == 1
+                chunks = SLOT_CHUNKS * sh.nrows
+                end4 = (rows[j] * rb + 3) & ~3
+                c = np.minimum(LANE[:, None] + 64 * np.arange(SLOT_LOADS), chunks - 1)
+                assert set(c.ravel()) == set(range(chunks))  # every chunk of the tile is loaded
+                at = end + wave * slot_bytes(slot_rows) + 16 * c
+                assert np.all(at % 16 == 0) and np.all(at + 16 <= end + (wave + 1) * slot_bytes(slot_rows))
+                for s in {load[3] for load in loads}:
+                    first = (sh.r0 + np.arange(sh.nrows)) * rb + s * B
+                    off = ((first & ~3)[:, None] + 16 * np.arange(SLOT_CHUNKS))[c // SLOT_CHUNKS, c % SLOT_CHUNKS]
+                    assert np.all(off >= 0) and np.all(off + 16 <= end4 + 16) and np.all(off % 4 == 0)
+                    # the superblock's bytes lie in its row's chunks, the 54 dwords read in its part of the slot
+                    assert np.all((first & 3) + B <= 16 * SLOT_CHUNKS) and 4 * 54 <= 16 * SLOT_CHUNKS
+                    assert np.all(first + B <= rows[j] * rb)
+                loads = []
             for part, g, rr, s in loads:
                 w = bases[1] if (mode == 1 and part) else bases[j]
                 n_mat = rows[1] if (mode == 1 and part) else rows[j]
@@ -222,32 +287,36 @@ def check_indices(rows, types, K, mode, M, bases):
                                 off = Z + reg + 4 * ((8 * s + jj) * 8 + 4 * klo)
                                 assert np.all(off >= Z + reg) and np.all(off + 16 <= Z + reg + K)
                 else:
-                    valid = (LN >> 2) == LKQ
-                    base = (LN & 3) * stride + 16 * LKQ
                     for h in range(2):
                         for nib in range(2):
-                            for mh in range(2 if M > 4 else 1):
-                                aoff = np.where(valid, base + 4 * mh * stride + 256 * s + 128 * h + 64 * nib, 8 * stride)
+                            blk = 4 * h + 2 * nib + khi
+                            for p in range(2 if M > 4 else 1):
+                                if M > 4:  # two products of the same Q8 block
+                                    valid = ((LN >> 3) == khi) & (klo == p)
+                                    base, m0, sb16 = (LN & 7) * stride + 16 * LKQ, 4 * klo, 2 * blk + p
+                                else:
+                                    valid = (LN >> 2) == LKQ
+                                    base, m0, sb16 = (LN & 3) * stride + 16 * LKQ, 0, 8 * h + 4 * nib + LKQ
+                                aoff = np.where(valid, base + 256 * s + 128 * h + 64 * nib, 8 * stride)
                                 assert np.all(aoff % 16 == 0) and np.all(aoff + 16 <= 8 * stride + 16)
-                                blk = 4 * h + 2 * nib + khi
-                                sb16 = 8 * h + 4 * nib + LKQ
-                                off = Z + 4 * ((8 * s + blk) * 8 + 4 * mh)
+                                assert np.all(np.where(valid, aoff + 16 <= 8 * stride, True))
+                                off = Z + 4 * ((8 * s + blk) * 8 + m0)
                                 assert np.all(off + 16 <= Z + K)
-                                off = Z + 2 * K + 4 * ((16 * s + sb16) * 8 + 4 * mh)
+                                off = Z + 2 * K + 4 * ((16 * s + sb16) * 8 + m0)
                                 assert np.all(off >= Z + 2 * K) and np.all(off + 16 <= Z + 4 * K)
                 if last:
                     assert (part, g, rr) not in slots, "unit flushed twice"
                     slots[(part, g, rr)] = True
                     slot = ((part * groups_max + g) * 16 + LN) * ranges + rr
                     off = Z + 4 * K + 4 * (slot * 8)
-                    assert np.all(off + 32 <= lds)
+                    assert np.all(off + 32 <= end)
         assert len(slots) == parts * sh.groups * ranges, "every unit flushed"
         # totals read every run of every valid row
         for part in range(parts):
             for rw in range(sh.nrows):
                 for rr in range(ranges):
                     off = Z + 4 * K + 4 * ((((part * groups_max) * 16 + rw) * ranges + rr) * 8 + 7)
-                    assert off + 4 <= lds
+                    assert off + 4 <= end
     for j, sh in workgroups(rows, types, K, mode, cfg):
         if (j, sh.r0) in chosen:
             for part in range(parts):
@@ -260,20 +329,27 @@ def check_indices(rows, types, K, mode, M, bases):
 SHAPES = [  # rows, types, K, mode, M
     ([4096, 1024, 1024], [12, 12, 14], 2560, 0, 8),   # attn q/k/v
     ([4096, 1024, 1024], [12, 12, 14], 2560, 0, 3),
-    ([2560], [12], 4096, 0, 8),                         # attn_output
+    ([4096, 1024, 1024], [12, 12, 12], 2560, 0, 2),
     ([9728, 9728], [12, 12], 2560, 1, 8),               # ffn gate/up
     ([9728, 9728], [12, 12], 2560, 1, 5),
+    ([9728, 9728], [14, 14], 2560, 1, 6),
+    ([9728, 9728], [14, 14], 2560, 1, 3),
+    ([300, 300], [12, 12], 512, 1, 2),
     ([2560], [14], 9728, 0, 8),                         # ffn_down
     ([2560], [14], 9728, 0, 4),
-    ([151936], [14], 2560, 0, 8),                       # lm_head
-    ([1024], [14], 2560, 0, 2),
-    ([9728, 9728], [14, 14], 2560, 1, 6),
-    ([19], [12], 2560, 0, 5),
+    ([2560], [12], 9728, 0, 8),
+    ([4096], [12], 11008, 0, 3),
+    ([4096], [12], 8192, 0, 2),                         # 16 rows on every CU
+    ([17], [12], 256, 0, 5),
+    ([3328], [14], 8192, 0, 8),                         # 13 rows of Q6_K on every CU
+    ([2560], [14], 10240, 0, 5),                        # LDS bounds the runs
     ([19], [14], 9728, 0, 7),
     ([45], [14], 768, 0, 3),
     ([101], [14], 1280, 0, 5),
-    ([3, 1, 2], [12, 12, 14], 256, 0, 7),
-    ([300, 17], [14, 12], 512, 0, 8),
+    ([300, 17], [14, 12], 2304, 0, 8),
+    ([1700, 33, 1560, 17], [14, 12, 14, 12], 2560, 0, 5),  # 256 workgroups
+    ([8160, 32], [12, 12], 2560, 0, 4),
+    ([700, 700], [14, 14], 4352, 0, 3),
 ]
 
 
@@ -285,11 +361,23 @@ def test_bmv_indices_in_bounds(rows, types, K, mode, M):
 
 def test_bmv_plan_for_qwen3_shapes():
     """LDS plans of the decode batch's launches (one workgroup per CU)."""
-    assert plan([2560], [14], 9728, 0, 8)[3] <= MAX_LDS           # ffn_down: 8 x 9728 codes + scales
-    assert plan([151936], [14], 2560, 0, 8)[2] == 38              # lm_head: 593-594 rows per CU
+    down = plan([2560], [14], 9728, 0, 8)                         # 8 x 9728 codes + scales + slots
+    assert down[:3] == ([256], 13, 1) and down[3:] == (159376, 10, 3, 3)
     assert plan([9728, 9728], [12, 12], 2560, 1, 8)[0] == [256]
+    qkv = plan([4096, 1024, 1024], [12, 12, 14], 2560, 0, 8)
+    assert sum(qkv[0]) <= 256 and qkv[2] == 2 and qkv[4] <= SLOT_ROWS
     assert plan([2560], [12], 4096, 0, 1) is None                 # M = 1: the whole-share kernels
     assert plan([2560], [12], 4096, 0, 9) is None                 # M > 8: the prefill GEMM
+
+
+@pytest.mark.parametrize("rows,types,K,M", [
+    ([151936], [14], 2560, 8), ([4097], [12], 9728, 5), ([3329], [14], 9728, 8),       # more rows than a group or slot
+    ([8160, 33], [12, 12], 2560, 4), ([1700, 33, 1700, 17], [14, 12, 14, 12], 2560, 5),  # past the CUs
+    ([1024], [14], 12288, 8), ([2560], [14], 10240, 4), ([300], [12], 13568, 3),         # LDS holds too few runs
+    ([2560], [14], 9728, 2), ([1024], [14], 9728, 4), ([4096, 1024, 1024], [12, 12, 12], 2048, 8),
+])
+def test_bmv_plan_declines(rows, types, K, M):
+    assert plan(rows, types, K, 0, M) is None
 
 
 # ---------------------------------------------------------------- arithmetic
@@ -304,8 +392,8 @@ def _f16(bits):
 
 def emulate(oracle, rows, types, K, mode, M, weights, x, rng):
     """The kernel's arithmetic at lane level; returns y per segment (mode 0) or h (mode 1)."""
-    cfg = plan(rows, types, K, mode, M)
-    count, ranges, groups_max, lds = cfg
+    cfg = fits(rows, types, K, mode)
+    ranges, groups_max = cfg[1:3]
     S, stride = K // 256, K + 16
     parts = 2 if mode == 1 else 1
     codes_q, scales_q = oracle.quantize_q8(x)
@@ -353,7 +441,7 @@ def emulate(oracle, rows, types, K, mode, M, weights, x, rng):
         sums = np.full((parts, groups_max, 16, ranges, 8), np.nan)
         for wave in range(WAVES):
             comps, _ = wave_streams(sh, wave, P[qtype])
-            acc = np.zeros((64, 8))
+            acc = np.zeros((64, 4))
             for part, g, rr, s, last in comps:
                 w = weights[1] if (mode == 1 and part) else weights[j]
                 row = np.minimum(16 * g + LN, sh.nrows - 1) + sh.r0
@@ -386,15 +474,13 @@ def emulate(oracle, rows, types, K, mode, M, weights, x, rng):
                             minv += mn[:, None] * y4
                     d = np.array([_f16(v & 0xFFFF) for v in head[:, 0]])
                     dmin = np.array([_f16(v >> 16) for v in head[:, 0]])
-                    acc[:, :4] += d[:, None] * mainv - dmin[:, None] * minv
+                    acc += d[:, None] * mainv - dmin[:, None] * minv
                 else:
                     ql = [np.stack([sbs[l, 64 * h + 16 * kq[l]:64 * h + 16 * kq[l] + 16] for l in range(64)]).astype(np.int64) for h in range(2)]
                     qh = [np.stack([sbs[l, 128 + 32 * h + 16 * klo[l]:128 + 32 * h + 16 * klo[l] + 16] for l in range(64)]).astype(np.int64) for h in range(2)]
                     scb = np.stack([sbs[l, 192:208] for l in range(64)]).view(np.int8).astype(np.int64)
                     d = np.array([_f16(int(sbs[l, 208]) | int(sbs[l, 209]) << 8) for l in range(64)])
-                    valid = (LN >> 2) == kq
-                    base = (LN & 3) * stride + 16 * kq
-                    accsb = np.zeros((64, 8))
+                    accsb = np.zeros((64, 4))
                     for h in range(2):
                         for nib in range(2):
                             # the kernel's dword ops: lo nibbles, qh rotated right by
@@ -410,26 +496,28 @@ def emulate(oracle, rows, types, K, mode, M, weights, x, rng):
                                 word = (hs & 0x30303030) | (lo & ~np.uint64(0x30303030) & 0xFFFFFFFF)
                                 codes16[l] = np.frombuffer(word.astype(np.uint32).tobytes(), dtype=np.uint8)
                             Bm = b_tile(codes16)
-                            sb16 = 8 * h + 4 * nib + kq
-                            scf = scb[LANE, 4 * (2 * h + nib) + kq]
                             blk = 4 * h + 2 * nib + khi
-                            for mh in range(2 if M > 4 else 1):
-                                A = a_tile(np.where(valid, base + 4 * mh * stride + 256 * s + 128 * h + 64 * nib, 8 * stride))
-                                n4 = np.stack([xf[16 * s + sb16[l], 4 * mh:4 * mh + 4] for l in range(64)])
+                            k0 = 256 * s + 128 * h + 64 * nib
+                            for p in range(2 if M > 4 else 1):
+                                if M > 4:  # products of the two sub-blocks of one Q8 block
+                                    valid = ((LN >> 3) == khi) & (klo == p)
+                                    base, m0, sb16 = (LN & 7) * stride + 16 * kq, 4 * klo, 2 * blk + p
+                                else:
+                                    valid = (LN >> 2) == kq
+                                    base, m0, sb16 = (LN & 3) * stride + 16 * kq, 0 * klo, 8 * h + 4 * nib + kq
+                                A = a_tile(np.where(valid, base + k0, 8 * stride))
+                                n4 = np.stack([xf[16 * s + sb16[l], m0[l]:m0[l] + 4] for l in range(64)])
                                 C = lane_c(A @ Bm) + n4  # D = A B + C, exact in int32
-                                x4 = np.stack([xs[8 * s + blk[l], 4 * mh:4 * mh + 4] for l in range(64)])
-                                accsb[:, 4 * mh:4 * mh + 4] += scf[:, None] * (x4 * C)
+                                x4 = np.stack([xs[8 * s + blk[l], m0[l]:m0[l] + 4] for l in range(64)])
+                                accsb += scb[LANE, sb16][:, None] * (x4 * C)
                     acc += d[:, None] * accsb
                 if last:
-                    if qtype == 12:
-                        v = acc[:, :4] + acc[LANE ^ 32, :4]
-                        for l in range(32):
-                            sums[part, g, l & 15, rr, 4 * (l >> 4):4 * (l >> 4) + 4] = v[l]
-                    else:
-                        v = acc + acc[LANE ^ 32]
-                        v = v + v[LANE ^ 16]
-                        for l in range(16):
-                            sums[part, g, l, rr, :] = v[l]
+                    v = acc + acc[LANE ^ 32]
+                    lanes = 32  # activation rows 4 (kq & 1).. in lanes of kq < 2
+                    if qtype == 14 and M <= 4:
+                        v, lanes = v + v[LANE ^ 16], 16
+                    for l in range(lanes):
+                        sums[part, g, l & 15, rr, 4 * (l >> 4):4 * (l >> 4) + 4] = v[l]
                     acc[:] = 0.0
         for m in range(M):
             for rw in range(sh.nrows):
@@ -468,7 +556,6 @@ def test_bmv_arithmetic_matches_oracle(oracle, rows, types, K, mode, M):
         u = oracle.reference_product(x, weights[1], types[1], K, rows[1])
         ref = g / (1.0 + np.exp(-g)) * u
         assert oracle.row_norm_error(got[0], ref) <= 1e-6
-
 
 
 def _owner(r, per, rem):
@@ -521,7 +608,7 @@ def test_bmv_q8h_blocks_close_once(N, M, count):
 
 @pytest.mark.parametrize("K", [256, 2560])
 def test_q6k_pair_tile_model(K):
-    """Q6_K at M = 5..8 (bmv_tile6_pair): product p's A rows 4g..4g+3 hold
+    """Q6_K at M = 5..8 (bmv_half6<2>): product p's A rows 4g..4g+3 hold
     activation rows 4(g & 1).. against k-quarter 2(g >> 1) + p, so that lane
     (n, kq) gets both sub-blocks of Q8 block 4h + 2nib + (kq >> 1) for activation
     rows 4(kq & 1)..; every read stays in its LDS array, the integer sums stay
@@ -572,31 +659,16 @@ def test_q6k_pair_tile_model(K):
         assert np.allclose(v[l], want[LN[l], 4 * LKQ[l]:4 * LKQ[l] + 4], rtol=1e-12)
 
 
-# The launch form of bmv.hpp: 16 waves, rings of 2 (Q4_K) and 1 (Q6_K) tiles;
-# one matrix (mode 0) in up to 16 rows a workgroup, Q6_K through LDS slots.
-@pytest.mark.parametrize("rows,types,K,mode,M", [
-    ([9728, 9728], [12, 12], 2560, 1, 8), ([9728, 9728], [14, 14], 2560, 1, 3), ([300, 300], [12, 12], 512, 1, 2),
-    ([2560], [12], 9728, 0, 8), ([4096], [12], 11008, 0, 3), ([17], [12], 256, 0, 5),
-])
-def test_bmv_sixteen_waves(monkeypatch, rows, types, K, mode, M):
-    import sys
-
-    module = sys.modules[__name__]
-    monkeypatch.setattr(module, "WAVES", 16)
-    monkeypatch.setattr(module, "P", {12: 2, 14: 1})
-    check_indices(rows, types, K, mode, M, [0] * len(rows))
-
-
 @pytest.mark.parametrize("N,S", [(2560, 38), (3328, 10), (2561, 7), (3, 1), (40, 41)])
 def test_bmv_q6k_slots(N, S):
     """Q6_K in mode 0: the tile's chunks (dword-aligned 16-byte loads, at most
     three a lane) put every superblock of the share's rows into the wave's slot
     whole, where ws_tile6 reads its 54 dwords; no load passes the matrix's last
     dword except into the descriptor's zeros, no write passes the slot."""
-    CH, LOADS = 14, 3
+    CH, LOADS = SLOT_CHUNKS, SLOT_LOADS
     count = min(CUS, N)
     rows_max = -(-N // count)
-    assert rows_max <= 64 * LOADS // CH
+    assert rows_max <= SLOT_ROWS
     rb, total = S * 210, N * S * 210
     end4 = (total + 3) & ~3
     per, rem = N // count, N % count
@@ -618,34 +690,3 @@ def test_bmv_q6k_slots(N, S):
                 o = 16 * CH * row + (first & 3)
                 assert (first & 3) in (0, 2) and 4 * 54 <= 16 * CH
                 assert np.array_equal(slot[o:o + 210], mat[first:first + 210])
-
-
-def multi_plan(rows, types, cus=CUS):
-    """bmv_plan's workgroups per matrix of a launch of several."""
-    total = cus + 1
-    for groups in (1, 2):
-        need = [-(-r // (13 if t == 14 else 16 * groups)) for r, t in zip(rows, types)]
-        total = sum(need)
-        if total <= cus:
-            break
-    if total > cus:
-        return None
-    byt = [r * BYTES[t] for r, t in zip(rows, types)]
-    return [min(r, c + int((cus - total) * b / sum(byt))) for r, c, b in zip(rows, need, byt)]
-
-
-@pytest.mark.parametrize("rows,types", [
-    ([4096, 1024, 1024], [12, 12, 14]), ([4096, 1024, 1024], [12, 12, 12]), ([2048, 1024, 1024], [12, 12, 14]),
-    ([1700, 33, 1560, 17], [14, 12, 14, 12]), ([8160, 32], [12, 12]), ([1, 1, 1], [14, 12, 14]),
-])
-def test_bmv_several_matrices_plan(rows, types):
-    """Every matrix's rows are cut among its workgroups without a gap, no
-    workgroup has more rows than its form takes, the grid fits the CUs."""
-    count = multi_plan(rows, types)
-    assert count is not None and sum(count) <= CUS
-    for r, t, c in zip(rows, types, count):
-        shares = [r // c + (1 if g < r % c else 0) for g in range(c)]
-        assert sum(shares) == r and min(shares) >= 1
-        assert max(shares) <= (13 if t == 14 else 32)
-    assert multi_plan([1700, 33, 1700, 17], [14, 12, 14, 12]) is None
-    assert multi_plan([8160, 33], [12, 12]) is None

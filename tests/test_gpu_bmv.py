@@ -8,10 +8,21 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+from test_bmv_layout import plan
+
 pytestmark = pytest.mark.gpu
 
 Q4, Q6 = 12, 14
 SEED = 20261501
+
+
+def check_plan(launch, rows, types, K, M, takes):
+    """The launch is the one the CPU model of the indices checks."""
+    cfg = plan(rows, types, K, 0, M)
+    assert (cfg is not None) == takes
+    if takes:
+        kind = types[0] if len(types) == 1 else 0
+        assert launch == f"bmv_kernel<{kind},0,{cfg[1]},{cfg[2]},0> grid={sum(cfg[0])}"
 
 
 @pytest.mark.parametrize("qtype,K,N,M,takes", [
@@ -38,6 +49,7 @@ def test_one_wide_matrix(gpu, oracle, qtype, K, N, M, takes):
     launch = gpu.last_launch()
     print(f"[case] type={qtype} K={K} N={N} M={M} launch {launch}", flush=True)
     assert launch.startswith("bmv_kernel") == takes
+    check_plan(launch, [N], [qtype], K, M, takes)
     out = y.download(np.float32)
     assert out[0] == 123.0 and out[-1] == 123.0
     got = out[1:-1].reshape(M, N)
@@ -99,6 +111,7 @@ def test_several_matrices(gpu, oracle, K, shapes, M, takes):
     launch = gpu.last_launch()
     print(f"[case] K={K} {shapes} M={M} launch {launch}", flush=True)
     assert launch.startswith("bmv_kernel") == takes
+    check_plan(launch, [N for _, N in shapes], [q for q, _ in shapes], K, M, takes)
     for h, (q, N), y in zip(hosts, shapes, ys):
         out = y.download(np.float32)
         assert out[-1] == 123.0

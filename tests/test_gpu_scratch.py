@@ -90,20 +90,26 @@ def test_threads_sharing_a_stream(gpu, oracle):
     stream.destroy()
 
 
-def test_capture_between_cached_calls(gpu, oracle):
-    a, b = (Case(gpu, oracle, Q4, 2560, 256, 33 + i, 20261401 + i) for i in range(2))
-    stream = gpu.Stream()
-    a.run(stream.ptr)
-    graph = gpu.Graph.capture(stream, lambda: a.run(stream.ptr))
-    for _ in range(3):
-        b.run(stream.ptr)
-        graph.launch(stream.ptr)
-        b.run(stream.ptr)
+def test_captured_calls_beside_eager_ones(gpu, oracle):
+    """A call recorded on a stream that already has a cached block, replayed
+    on a second stream while that first stream makes eager calls of the same
+    size, with nothing between them in a round: the graph shares no block."""
+    a, b, c = (Case(gpu, oracle, Q4, 2560, 1024, 500 + i, 20261401 + i) for i in range(3))
+    eager, replay = gpu.Stream(), gpu.Stream()
+    a.run(eager.ptr)  # leaves the stream a block
+    graph = gpu.Graph.capture(eager, lambda: a.run(eager.ptr))
+    gpu.synchronize()
+    for _ in range(6):
+        for _ in range(4):
+            graph.launch(replay.ptr)
+            b.run(eager.ptr)
+            c.run(eager.ptr)
         gpu.synchronize()
-        a.check()
-        b.check()
+        for case in (a, b, c):
+            case.check()
     graph.destroy()
-    stream.destroy()
+    for s in (eager, replay):
+        s.destroy()
 
 
 @pytest.mark.parametrize("others", [0, 8])
@@ -157,7 +163,9 @@ def _free_bytes(qk):
 
 def test_release_gives_the_blocks_back(gpu, oracle):
     """8 streams hold a block each; once qk_release_scratch has returned their
-    memory is free on the device, and later calls run as before."""
+    memory is free on the device, and later calls run as before. (The pool takes
+    and gives 2 MiB pieces, some of which it may have had: half a block of slack.)"""
+    most = 8 * (16 << 20) - (8 << 20)
     case = Case(gpu, oracle, Q4, 2560, 256, 33, 20261601)
     streams = [gpu.Stream() for _ in range(8)]
     gpu.release_scratch()
@@ -166,10 +174,10 @@ def test_release_gives_the_blocks_back(gpu, oracle):
         case.run(s.ptr)
     gpu.synchronize()
     held = _free_bytes(gpu)
-    assert before - held >= 8 * (16 << 20)
+    assert before - held >= most
     case.check()
     gpu.release_scratch()
-    assert _free_bytes(gpu) - held >= 8 * (16 << 20)
+    assert _free_bytes(gpu) - held >= most
     case.run(streams[0].ptr)
     gpu.synchronize()
     case.check()
