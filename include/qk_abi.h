@@ -158,8 +158,8 @@ int qk_matmul_segments_ws(const float *x, int64_t M, int64_t K, const qk_segment
 
 /* h[M x N] = SiLU(Q8(x) . gate^T) * (Q8(x) . up^T), gate and up both `type`
  * with K columns and N rows: one launch for M <= 8; for M > 8 the prefill
- * GEMM (gate and up in one launch) into stream-ordered scratch, then the
- * SiLU kernel. Replaces matmul(gate), matmul(up), silu_multiply
+ * GEMM (gate and up in one launch where their grid needs no split of K) into
+ * the call's scratch, then the SiLU kernel. Replaces matmul(gate), matmul(up), silu_multiply
  * (src/Engine.cpp:98-100, src/cuda/silu_multiply.cu:6-12). */
 int qk_ffn_gate_up(const float *x, const void *gate, const void *up, int type, int64_t K,
                    int64_t N, float *h, int64_t M, qk_stream_t stream);
@@ -181,7 +181,7 @@ int qk_ffn_gate_up_ws(const float *x, const void *gate, const void *up, int type
  * rms_norm(ffn_norm) before the FFN (src/Engine.cpp:97-99,
  * src/cuda/rms_norm.cu:6-24,28-36). M = 1: the norm is folded into the one
  * launch and the normalised row never goes to memory; other M: the norm runs
- * first into stream-ordered scratch. eps must be > 0 (QK_ERR_INVALID_ARGUMENT
+ * first into the call's scratch. eps must be > 0 (QK_ERR_INVALID_ARGUMENT
  * otherwise, as the reference throws); M = 0 does nothing. */
 int qk_ffn_gate_up_norm(const float *x, const float *norm, float eps, const void *gate,
                         const void *up, int type, int64_t K, int64_t N, float *h, int64_t M,

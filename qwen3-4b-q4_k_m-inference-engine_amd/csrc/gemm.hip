@@ -59,11 +59,12 @@ constexpr int kPrepGroups = 8;  // groups of 8 activations held per thread: K <=
 // One workgroup per activation row: the row's max |x| (for the power-of-two
 // scale), then the Q8 round trip of every 32-value block. Rows up to 16384
 // values stay in registers between the two steps (G groups of 8 per thread,
-// the least that holds the row: a launch over few rows is all latency, and
-// rounds that no thread takes part in still cost their branches: 1024 x 2560 at
-// M = 200 19.0 -> 18.5 us with its GEMM, 9728 x 2560 at M = 23 19.4 -> 18.4, the
-// quantiser's nearest-integer form included); wider rows (G = 0) are read twice. K % 32 == 0, so the 4 lanes of a quad are always in or
-// out together.
+// the least of 1, 2, 5 and 8 that holds the row: 2 for K = 2560 and 4096, 5 for
+// 9728): a launch over few rows is all latency, and rounds that no thread takes
+// part in still cost their branches (1024 x 2560 at M = 200 19.0 -> 18.5 us with
+// its GEMM, 9728 x 2560 at M = 23 19.4 -> 18.4, the quantiser's nearest-integer
+// form included). Wider rows (G = 0) are read twice. K % 32 == 0, so the 4 lanes
+// of a quad are always in or out together.
 template <int G>
 __global__ __launch_bounds__(256) void prep_rows_kernel(const float* __restrict__ x,
                                                         _Float16* __restrict__ hi,

@@ -929,18 +929,19 @@ double plan_cost(int type, bool wide, int64_t tiles, int64_t splits, int64_t M, 
 // The rules above hold for K < 4096 at M > 64. For deep K, and for the few
 // tiles of M <= 64, they leave up to half of the time on CUs that wait for the
 // busiest one; there the plan is the tile height and split of least estimated
-// time. Measured against the rules (us, prep and reduce included; 22 shapes
-// timed under every plan, the chosen one 1.13 times as fast as the rules' on
-// average and never more than 1% behind it): 2560 x 9728 Q6_K at M = 48 / 100 /
-// 200 / 350 / 800 37.4 / 63.3 / 78.8 / 112.6 / 256 -> 33.6 / 41.4 / 62.7 / 88.6 /
-// 219, Q4_K at M = 100 / 512 38.9 / 97.9 -> 31.7 / 78.7, 1024 x 2560 Q6_K at
-// M = 48 21.0 -> 14.6. (At smaller K and larger M finer splits gain less, and
-// a row's sums are the same there at every M.) At M <= 32 the rule's split is
-// the most: its units are one to three a CU, and a few over two a CU cost a
-// round; fewer splits only while no split takes more superblocks (no longer
-// fp32 sums: two a split of 8, where the rule has one, would be 7% faster at
-// 2048 -> 6144, M = 32, and is not taken) (2560 x 9728 at M = 23, 26 -> 19 splits: Q6_K 27.1 -> 23.7, Q4_K 19.9 ->
-// 18.2; 9728 x 2560, 7 -> 5: Q4_K 18.2 -> 16.5, Q6_K 22.7 -> 20.8).
+// time. Measured against the rules (us, prep and reduce included): 2560 x 9728
+// Q6_K at M = 48 / 100 / 200 / 350 / 800 37.4 / 63.3 / 78.8 / 112.6 / 256 -> 33.6 /
+// 41.4 / 62.7 / 88.6 / 219, Q4_K at M = 100 / 512 38.9 / 97.9 -> 31.7 / 78.7, 1024 x
+// 2560 Q6_K at M = 48 21.0 -> 14.6; over 155 random shapes that it plans
+// otherwise (M = 33..1500, K to 12800, N to 20000) 0.82 times the rules' time on
+// average, five slower, by 3 to 5%, all at M > 64 and N > 6100 (142 x 8947 x 5632
+// Q4_K 66.7 -> 69.8). (At smaller K and larger M finer splits gain less, and a
+// row's sums are the same there at every M.) At M <= 32 the rule's split is the
+// most: its units are one to three a CU, and a few over two a CU cost a round.
+// Fewer splits only while no split takes more superblocks, which would be
+// longer fp32 sums (6144 x 2048 at M = 32, 8 splits of one: 4 would be 7%
+// faster). 2560 x 9728 at M = 23, 26 -> 19 splits: Q6_K 27.1 -> 23.7, Q4_K 19.9 ->
+// 18.2; 9728 x 2560, 7 -> 5: Q4_K 18.2 -> 16.5, Q6_K 22.7 -> 20.8.
 constexpr int64_t kPlanSplits = 6;
 
 // Bytes of the workspace of a product that runs in `splits` splits.

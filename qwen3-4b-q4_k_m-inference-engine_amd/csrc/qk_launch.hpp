@@ -81,9 +81,9 @@ hipError_t launch_bmv_ws(const MatvecParams& p, int mode, hipStream_t stream, bo
 // The batched mat-vec on the int8 matrix cores (bmv.hip): M = 2..8 rows of
 // fp32 activations in the gate/up mode (1; with p.hq and p.arrive it also
 // writes Q8(h)), of several matrices, or of one wide matrix (that also from Q8
-// blocks). Launched (and `launched` set) when the shape fits its LDS
-// plan (and, with p.hq, its block-closing step); otherwise nothing is
-// enqueued.
+// blocks) where it is the faster kernel. Launched (and `launched` set) when the
+// shape fits its LDS plan (and, with p.hq, its block-closing step); otherwise
+// nothing is enqueued.
 hipError_t launch_bmv(const MatvecParams& p, int mode, hipStream_t stream, bool& launched);
 
 // The multi-pass batched mat-vec on the int8 matrix cores (bmv_pass.hip): M =
