@@ -291,8 +291,9 @@ int qk_check_launch(void);
 
 /* Entry points that need device scratch and are given none (M > 8) take it
  * from up to 8 blocks per device of 16 or 64 MiB that stay allocated between
- * calls (larger requests, requests while no block is idle, and calls under
- * stream capture allocate and free stream-ordered). Waits for the current
+ * calls (larger requests, requests while no block is idle, calls on the
+ * per-thread default stream and calls under stream capture allocate and free
+ * stream-ordered). Waits for the current
  * device and gives its idle blocks back; later calls allocate them anew. Not
  * for use while a stream is being captured. */
 int qk_release_scratch(void);

@@ -3,6 +3,8 @@
 // its event has completed, so calls on different streams never wait for each
 // other. The stream waits for the block's event even when the handle is the
 // one that recorded it: a destroyed stream's handle may name a new stream.
+// (hipStreamPerThread is one handle for a stream of each thread, which would
+// wait for each other so: its calls allocate stream-ordered.)
 // A block is held by one call at a time (busy), so threads that share a
 // stream, and calls that make another call, take different blocks.
 #include "scratch.hpp"
@@ -74,7 +76,7 @@ hipError_t Scratch::get(size_t bytes, void*& ptr) {
   hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
   int device = -1;
   const OwnErrors errors;
-  if (size != 0 && hipStreamIsCapturing(stream_, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone &&
+  if (size != 0 && stream_ != hipStreamPerThread && hipStreamIsCapturing(stream_, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone &&
       hipGetDevice(&device) == hipSuccess && device >= 0 && device < kMaxDevices) {
     std::lock_guard<std::mutex> lock(g_mutex);
     Block(&blocks)[kScratchBlocks] = g_blocks[device];

@@ -16,8 +16,9 @@
 namespace qk {
 
 // At most kScratchBlocks blocks per device, of 16 or 64 MiB; larger requests,
-// requests while a block cannot be had, and calls under stream capture (whose
-// graph may be replayed beside later calls) are stream-ordered allocations.
+// requests while a block cannot be had, calls on the per-thread default stream
+// and calls under stream capture (whose graph may be replayed beside later
+// calls) are stream-ordered allocations.
 constexpr int kScratchBlocks = 8;
 constexpr size_t kScratchSmall = size_t{16} << 20;
 constexpr size_t kScratchLarge = size_t{64} << 20;

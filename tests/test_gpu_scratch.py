@@ -183,3 +183,35 @@ def test_release_gives_the_blocks_back(gpu, oracle):
     case.check()
     for s in streams:
         s.destroy()
+
+
+def test_per_thread_stream_holds_no_block(gpu, oracle):
+    """The per-thread default stream's handle (2) names a stream of each
+    thread: a block kept under it would make one thread's call wait for
+    another's, so its calls keep none; two threads' results are right."""
+    per_thread = 2
+    cases = [Case(gpu, oracle, Q4, 2560, 256, 33 + i, 20261701 + i) for i in range(2)]
+    cases[0].run(per_thread)  # (what the runtime itself allocates at first use)
+    gpu.synchronize()
+    gpu.release_scratch()
+    gpu.synchronize()
+    before = _free_bytes(gpu)
+    errors = []
+
+    def work(c):
+        try:
+            for _ in range(8):
+                c.run(per_thread)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(c,)) for c in cases]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    gpu.synchronize()
+    assert not errors
+    assert before - _free_bytes(gpu) < 16 << 20
+    for c in cases:
+        c.check()
