@@ -1,6 +1,6 @@
 // Batched mat-vec kernel entry (bmv.hpp) and its host launcher: M = 2..8
-// activation rows in fp32 or Q8 blocks, one matrix or gate and up, one
-// workgroup per CU.
+// activation rows in fp32 or (one matrix) Q8 blocks, one matrix, several or
+// gate and up, one workgroup per CU.
 #include <algorithm>
 #include <climits>
 
